@@ -166,3 +166,20 @@ def test_query_metric_kernel_against_host_metric_and_restatement(q_dtype):
         assert np.abs(gm[b * HKV_:(b + 1) * HKV_] - refg).max() <= 1e-5 * np.abs(refg).max()
         o = O.query_metric(M_pre.double().numpy(), qrows[b].float().numpy(), T, inv.double().numpy(), sc)
         assert np.abs(got - o).max() <= 2e-5 * np.abs(o).max()
+
+
+@pytest.mark.parametrize("batch", [256, 257, 300])
+def test_sym_eig_top_layouts_agree(batch):
+    """Eight waves per matrix (up to 256 matrices) and four (beyond) form every sum in one order:
+    the same bits, whatever the size of the batch a matrix is solved in, also at k = 64 (two staged
+    blocks of output columns)."""
+    print(f"[case] sym_eig_top layouts batch={batch}", flush=True)
+    rng = np.random.default_rng(11)
+    few = np.stack([m.astype(np.float32) for m in _spectra(rng).values()])
+    for k in (32, 64):
+        ev, vec, sw = _solve(few, k)
+        many = few[np.arange(batch) % len(few)]
+        ev2, vec2, sw2 = _solve(many, k)
+        for i in range(batch):
+            assert np.array_equal(ev2[i], ev[i % len(few)]) and np.array_equal(vec2[i], vec[i % len(few)])
+            assert sw2[i] == sw[i % len(few)]
