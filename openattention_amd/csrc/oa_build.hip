@@ -29,6 +29,7 @@
 // hardware's, so the CPU restatement matches them up to an agreement rate (ties of the bf16
 // result), not bit for bit.
 #include <algorithm>
+#include <type_traits>
 
 #include "oa_common.h"
 
@@ -325,39 +326,57 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2v));
 }
 
-// One 256-thread workgroup per (kAsgTiles 64-token tiles, query row): the row's centroids (bf16,
-// B operands: centroid lane % 16 of a 16-centroid block, dims 4*(lane/16)..+3) and
-// bf16(|c|^2 / 2) are staged in LDS once and every wave then takes every fourth tile.
-// Per 16-token block and centroid block one v_mfma_f32_16x16x16bf16_1k gives 16 x 16 dots;
-// the distance bf16(bf16(dot) - half) is ranked through the key (bf16 key << 16 | 255 - c), so the
-// maximum over the 16 centroid lanes (a DPP row) and over the blocks is the argmax with ties to
-// the lower cluster.
+// bf16(b) above the high half of `tag`, which comes from a scalar register: left to the compiler, every
+// distinct tag took a vector register
+__device__ __forceinline__ uint32_t cvt_pk_bf16_tag(uint32_t tag, float b) {
+  uint32_t r;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "s"(tag), "v"(b));
+  return r;
+}
+
+// One 256-thread workgroup per (4 x tiles_per_wave 64-token tiles, query row).  The row's centroids
+// (bf16) are the A operand of v_mfma_f32_16x16x16bf16_1k and 16 tokens the B operand, so that a lane
+// holds distances of one token: centroids 16 cb + 4 (lane / 16) + i of token lane % 16 for the
+// centroid blocks cb, kept in registers with their bf16(|c|^2 / 2) for all of the wave's tiles.
+//
+// A distance bf16(bf16(dot) - half) is ranked as one integer: the conversion that rounds it to bf16
+// puts it above a 16-bit tag that is larger for a lower cluster (v_cvt_pk_bf16_f32 with a constant
+// for the low half).  As a signed integer that order is the distance's own wherever the best one is
+// positive, as it is for most tokens once the centroids are means; a block of 16 tokens with a best
+// distance that is not a positive finite number is ranked again with the negative distances' order
+// set right (two instructions more per distance), and so are the blocks after it until one would not
+// have needed it.  A row with a centroid of half = +0 (only there can bf16(x - half) be -0, which
+// ranks as +0) is ranked with a third order.
+//
+// Bound by vector issue: 3.5 instructions per distance and about 26 per 16 tokens; with tokens as
+// rows a distance took about 8 (keys and tags formed apart) and each block of 16 tokens a 16-lane
+// maximum of four registers.  32 sequences of 32767 tokens, 64 clusters: 725 -> 432 us per
+// assignment; two of 10007 tokens, 256 clusters: 109 -> 38 us.
 constexpr int kAsgThreads = 256;
-constexpr int kAsgTiles = 32;
-__global__ void __launch_bounds__(kAsgThreads) kmeans_assign_kernel(const uint16_t* zraw,
+constexpr int kAsgMaxTiles = 8;                // tiles per wave where the grid is full without
+constexpr uint32_t kTag = 0x3f00u;             // low half of a ranked distance: kTag | 63 - (4 cb + i)
+template <int CB>
+__global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : 4) kmeans_assign_kernel(const uint16_t* zraw,
                                                                     const float* colmean, long zps, int T,
                                                                     const float* cent, int C,
                                                                     int32_t* asg, long as,
-                                                                    uint8_t* asg8, long a8s) {
-  __shared__ uint16_t s_cb[kMaxC * kRC];
-  __shared__ uint16_t s_half[kMaxC];
-  const int lane = threadIdx.x & 63;
+                                                                    uint8_t* asg8, long a8s,
+                                                                    int tiles_per_wave) {
+  __shared__ __align__(16) uint16_t s_cb[CB * 16 * kRC];
+  __shared__ __align__(16) float s_half[CB * 16];
+  const int lane = threadIdx.x & 63, grp = lane >> 4;
   const int wave = threadIdx.x >> 6;
   const int row = blockIdx.y;
-  const int CB = (C + 15) / 16;
   const int ntiles = (T + 63) / 64;
   const float* cr = cent + (long)row * C * kRC;
   // four centroid values per thread and iteration (C * kRC is a multiple of 4)
   for (int i = 4 * threadIdx.x; i < CB * 16 * kRC; i += 4 * kAsgThreads) {
-    if (i < C * kRC) {
-      const float4 x = *reinterpret_cast<const float4*>(cr + i);
-      s_cb[i] = oa::f32_to_bf16(x.x);
-      s_cb[i + 1] = oa::f32_to_bf16(x.y);
-      s_cb[i + 2] = oa::f32_to_bf16(x.z);
-      s_cb[i + 3] = oa::f32_to_bf16(x.w);
-    } else {
-      s_cb[i] = s_cb[i + 1] = s_cb[i + 2] = s_cb[i + 3] = 0;
-    }
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < C * kRC) x = *reinterpret_cast<const float4*>(cr + i);
+    s_cb[i] = oa::f32_to_bf16(x.x);
+    s_cb[i + 1] = oa::f32_to_bf16(x.y);
+    s_cb[i + 2] = oa::f32_to_bf16(x.z);
+    s_cb[i + 3] = oa::f32_to_bf16(x.w);
   }
   int zero_half = 0;          // this thread staged a real centroid with bf16(|c|^2 / 2) = +0
   for (int c = threadIdx.x; c < CB * 16; c += kAsgThreads) {
@@ -372,82 +391,88 @@ __global__ void __launch_bounds__(kAsgThreads) kmeans_assign_kernel(const uint16
       hv = oa::f32_to_bf16(0.5f * s);
       zero_half |= hv == 0;
     }
-    s_half[c] = hv;
+    s_half[c] = oa::bf16_to_f32(hv);
   }
-  // bf16(x - half) is -0 only for half = +0 (x - x rounds to +0): without such a centroid the
-  // distances need no -0 -> +0 step, and their keys are formed two at a time from the packed pair
-  const bool fast = __syncthreads_or(zero_half) == 0;
+  const bool plain = __syncthreads_or(zero_half) == 0;
+  short4v ca[CB];
+  float4 hf[CB];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    ca[cb] = *reinterpret_cast<const short4v*>(s_cb + (cb * 16 + (lane & 15)) * kRC + 4 * grp);
+    hf[cb] = *reinterpret_cast<const float4*>(s_half + cb * 16 + 4 * grp);
+  }
   // zP = bf16(k W) - colmean, formed from the stored bf16 projection (the same fp32 values)
   float cm[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) cm[e] = colmean[row * kRC + 4 * (lane >> 4) + e];
-  const int tend = min(ntiles, (blockIdx.x + 1) * kAsgTiles);
-  for (int tile = blockIdx.x * kAsgTiles + wave; tile < tend; tile += kAsgThreads / 64) {
+  for (int e = 0; e < 4; ++e) cm[e] = colmean[row * kRC + 4 * grp + e];
+  const uint16_t* zr = zraw + (long)row * zps + 4 * grp;
+  auto load = [&](uint2 (&z)[4], int tile) {
 #pragma unroll
+    for (int blk = 0; blk < 4; ++blk)
+      z[blk] = *reinterpret_cast<const uint2*>(zr + (long)min(tile * 64 + blk * 16 + (lane & 15), T - 1) * kRC);
+  };
+  const int tile0 = (blockIdx.x * (kAsgThreads / 64) + wave) * tiles_per_wave;
+  const int tend = min(ntiles, tile0 + tiles_per_wave);
+  uint2 z[4];
+  if (tile0 < tend) load(z, tile0);
+  bool positive = plain;     // the last block's best distances were: try the cheap order on the next
+#pragma unroll 1
+  for (int tile = tile0; tile < tend; ++tile) {
+    uint2 zn[4];
+    load(zn, min(tile + 1, ntiles - 1));
+    int mine = 0;              // the ranked best of this lane's token of the tile (token lane)
+#pragma unroll 1
     for (int blk = 0; blk < 4; ++blk) {
-      const int t0 = tile * 64 + blk * 16;
-      const int ta = min(t0 + (lane & 15), T - 1);
-      const uint2 zr =
-          *reinterpret_cast<const uint2*>(zraw + (long)row * zps + (long)ta * kRC + 4 * (lane >> 4));
-      short4v a;
-      a[0] = (short)oa::f32_to_bf16_rn(__uint_as_float(zr.x << 16) - cm[0]);
-      a[1] = (short)oa::f32_to_bf16_rn(__uint_as_float(zr.x & 0xffff0000u) - cm[1]);
-      a[2] = (short)oa::f32_to_bf16_rn(__uint_as_float(zr.y << 16) - cm[2]);
-      a[3] = (short)oa::f32_to_bf16_rn(__uint_as_float(zr.y & 0xffff0000u) - cm[3]);
-      uint32_t best[4] = {0u, 0u, 0u, 0u};
-      for (int cb = 0; cb < CB; ++cb) {
-        const int c = cb * 16 + (lane & 15);
-        const uint16_t* bp = s_cb + c * kRC + 4 * (lane >> 4);
-        short4v b;
-        b[0] = (short)bp[0]; b[1] = (short)bp[1]; b[2] = (short)bp[2]; b[3] = (short)bp[3];
-        float4v acc = {0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-        const float hf = oa::bf16_to_f32(s_half[c]);
-        // bf16(bf16(dot) - half), two values per conversion; + 0 turns -0 into +0 (one score); the
-        // key is the distance's order-preserving key (its top 16 bits: the bf16 key) with the tag
-        // 255 - c below it
-        const uint32_t tag = (uint32_t)(255 - c);
-        const uint32_t p01 = cvt_pk_bf16(acc[0], acc[1]), p23 = cvt_pk_bf16(acc[2], acc[3]);
-        const uint32_t q01 = cvt_pk_bf16(__uint_as_float(p01 << 16) - hf, __uint_as_float(p01 & 0xffff0000u) - hf);
-        const uint32_t q23 = cvt_pk_bf16(__uint_as_float(p23 << 16) - hf, __uint_as_float(p23 & 0xffff0000u) - hf);
-        if (fast) {
-          // the order-preserving key of each bf16 half (negative: every bit flipped; otherwise
-          // the sign bit set), two halves per instruction, then key << 16 | tag per distance
-          const uint32_t k01 = q01 ^ (((q01 >> 15) & 0x00010001u) * 0x7fffu | 0x80008000u);
-          const uint32_t k23 = q23 ^ (((q23 >> 15) & 0x00010001u) * 0x7fffu | 0x80008000u);
-          best[0] = max(best[0], (k01 << 16) | tag);
-          best[1] = max(best[1], (k01 & 0xffff0000u) | tag);
-          best[2] = max(best[2], (k23 << 16) | tag);
-          best[3] = max(best[3], (k23 & 0xffff0000u) | tag);
-        } else {
-          const float e[4] = {__uint_as_float(q01 << 16) + 0.f, __uint_as_float(q01 & 0xffff0000u) + 0.f,
-                              __uint_as_float(q23 << 16) + 0.f, __uint_as_float(q23 & 0xffff0000u) + 0.f};
+      const uint2 w = make_uint2(
+          cvt_pk_bf16(__uint_as_float(z[0].x << 16) - cm[0], __uint_as_float(z[0].x & 0xffff0000u) - cm[1]),
+          cvt_pk_bf16(__uint_as_float(z[0].y << 16) - cm[2], __uint_as_float(z[0].y & 0xffff0000u) - cm[3]));
+      const short4v tok = __builtin_bit_cast(short4v, w);
+      z[0] = z[1]; z[1] = z[2]; z[2] = z[3];
+      // the token's best: 0 as the bits stand (right where it is positive), 1 in the distances' order,
+      // 2 the same with -0 as +0
+      auto rank = [&](auto mode_c) {
+        constexpr int MODE = decltype(mode_c)::value;
+        int best = (int)0x80000000u;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) best[i] = max(best[i], (oa::float_key(e[i]) & 0xffff0000u) | tag);
-        }
-      }
-      // maximum over the 16 lanes of each DPP row (the 16 centroids of one block column set)
+        for (int cb = 0; cb < CB; ++cb) {
+          float4v acc = {0.f, 0.f, 0.f, 0.f};
+          acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ca[cb], tok, acc, 0, 0, 0);
+          const float h[4] = {hf[cb].x, hf[cb].y, hf[cb].z, hf[cb].w};
+          int v[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        uint32_t v = best[i];
-        v = max(v, oa::dpp_u32<0xB1, 0xf>(v));
-        v = max(v, oa::dpp_u32<0x4E, 0xf>(v));
-        v = max(v, oa::dpp_u32<0x141, 0xf>(v));
-        v = max(v, oa::dpp_u32<0x140, 0xf>(v));
-        best[i] = v;
-      }
-      if ((lane & 15) < 4) {
-        const int i = lane & 15;
-        const int t = t0 + 4 * (lane >> 4) + i;
-        // lane (16g + i) holds token 4g + i of the block: best[i] of its row
-        uint32_t v = i == 0 ? best[0] : (i == 1 ? best[1] : (i == 2 ? best[2] : best[3]));
-        if (t < T) {
-          const int cid = 255 - (int)(v & 0xffu);   // (every real distance key exceeds 0)
-          asg[(long)row * as + t] = cid;
-          asg8[(long)row * a8s + t] = (uint8_t)cid;
+          for (int i = 0; i < 4; ++i) {
+            float d = __uint_as_float(cvt_pk_bf16(0.f, acc[i])) - h[i];
+            if (MODE == 2) d = __uint_as_float(cvt_pk_bf16(0.f, d)) + 0.f;
+            v[i] = (int)cvt_pk_bf16_tag((kTag | (63 - (4 * cb + i))) << 16, d);
+            if (MODE) v[i] ^= (v[i] >> 31) & 0x7fff0000;   // a negative distance's magnitude reversed
+          }
+          best = max(max(best, v[0]), v[1]);
+          best = max(max(best, v[2]), v[3]);
         }
+        // tag 63 - (4 cb + i) of lane group g -> 255 - (16 cb + 4 g + i), then the best of the groups
+        const uint32_t u = (uint32_t)best;
+        best = (int)((u & 0xffff0000u) | ((u & 0x3cu) << 2) | (u & 3u) | (uint32_t)(4 * (3 - grp)));
+        const auto r16 = __builtin_amdgcn_permlane16_swap((uint32_t)best, (uint32_t)best, false, false);
+        best = max((int)r16[0], (int)r16[1]);
+        const auto r32 = __builtin_amdgcn_permlane32_swap((uint32_t)best, (uint32_t)best, false, false);
+        return max((int)r32[0], (int)r32[1]);
+      };
+      int best = 0;
+      if (positive) best = rank(std::integral_constant<int, 0>());
+      if (!positive || __ballot(best <= 0 || best >= 0x7f800000) != 0ull) {
+        best = plain ? rank(std::integral_constant<int, 1>()) : rank(std::integral_constant<int, 2>());
+        positive = plain && __ballot(best <= 0 || best >= 0x7f800000) == 0ull;
       }
+      mine = grp == blk ? best : mine;
     }
+    const int t = tile * 64 + lane;
+    if (t < T) {
+      const int cid = 255 - (mine & 0xff);
+      asg[(long)row * as + t] = cid;
+      asg8[(long)row * a8s + t] = (uint8_t)cid;
+    }
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) z[blk] = zn[blk];
   }
 }
 
@@ -769,10 +794,23 @@ extern "C" int oa_kmeans_assign(const uint16_t* zraw, const float* colmean, long
       z_stride < (long)T * kRC || z_stride % 4 || asg_stride < T || asg8_stride < T ||
       (reinterpret_cast<uintptr_t>(zraw) & 7))
     return OA_EINVAL;
-  const int ntiles = (T + 63) / 64;
-  hipLaunchKernelGGL(kmeans_assign_kernel, dim3((ntiles + kAsgTiles - 1) / kAsgTiles, rows),
-                     dim3(kAsgThreads), 0, (hipStream_t)stream, zraw, colmean, z_stride, T, cent, C, asg,
-                     asg_stride, asg8, asg8_stride);
+  // eight tiles per wave spread the centroids' staging; fewer where the grid would not give every
+  // SIMD eight waves
+  const int ntiles = (T + 63) / 64, waves = kAsgThreads / 64;
+  const int tpw = (int)std::min<long>(kAsgMaxTiles, std::max<long>(1, (long)ntiles * rows / 8192));
+  const dim3 grid((ntiles + waves * tpw - 1) / (waves * tpw), rows), block(kAsgThreads);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, zraw, colmean, z_stride, T, cent, C, asg,
+                       asg_stride, asg8, asg8_stride, tpw);
+  };
+  // the centroid blocks a wave holds: the least of these that covers C (padding ranks below)
+  const int cb = (C + 15) / 16;
+  if (cb <= 1) launch(kmeans_assign_kernel<1>);
+  else if (cb <= 2) launch(kmeans_assign_kernel<2>);
+  else if (cb <= 4) launch(kmeans_assign_kernel<4>);
+  else if (cb <= 8) launch(kmeans_assign_kernel<8>);
+  else if (cb <= 12) launch(kmeans_assign_kernel<12>);
+  else launch(kmeans_assign_kernel<16>);
   return OA_LAUNCH_STATUS();
 }
 

@@ -1284,3 +1284,40 @@ def test_split_gate_equals_whole_gate(B, N, rho):
     assert np.array_equal(res["whole"]["TMn"], res["split"]["TMn"]), "split: tile minima differ"
     hits = (res["split"]["sel"] >= 0).sum()
     print(f"  bit-exact over {R} rows ({hits} selected tokens)", flush=True)
+
+
+@pytest.mark.parametrize("C", [1, 15, 16, 17, 33, 64, 65, 100, 128, 129, 192, 200, 256])
+@pytest.mark.parametrize("T", [1, 63, 65, 700])
+def test_kmeans_assign_edges_exact(C, T):
+    """Every centroid-block size and ragged tile of the assignment on small whole numbers, where each
+    dot product is exact in fp32 whatever the order of its sum: the ids equal the restatement's.  Row
+    0: centroids near the tokens (best distances positive); row 1: tokens far from all centroids on
+    the other side (every distance negative); row 2: many equal centroids (ties to the lower id); row
+    3: a zero centroid and tokens whose best distance is +0; row 4: a token with an infinity and one
+    with a NaN, which take cluster 0 (all distances NaN)."""
+    print(f"[case] k-means assignment edges C={C} T={T}", flush=True)
+    rng = np.random.default_rng(C * 1000 + T)
+    R = 5
+    zP = rng.integers(-3, 4, (R, T, 16)).astype(np.float32)
+    cent = rng.integers(-3, 4, (R, C, 16)).astype(np.float32)
+    cent[0] += 2 * (np.abs(cent[0]).sum(-1, keepdims=True) == 0)
+    zP[1], cent[1] = np.abs(zP[1]) + 1, -np.abs(cent[1]) - 1
+    cent[2] = cent[2][rng.integers(0, max(1, C // 8), C)]
+    cent[3, C // 2] = 0.0
+    zP[3] = 0.0
+    zP[4, 0, 3] = np.inf
+    zP[4, T - 1, 5] = np.nan
+    zraw = torch.from_numpy(zP).to(DEV).to(torch.bfloat16)
+    cm = torch.zeros(R, 16, device=DEV)
+    asg = torch.full((R, T + 3), -1, device=DEV, dtype=torch.int32)
+    asg8 = torch.full((R, T + 3), 255, device=DEV, dtype=torch.uint8)
+    ops.kmeans_assign(zraw, cm, T, torch.from_numpy(cent).to(DEV).contiguous(), asg, asg8)
+    torch.cuda.synchronize()
+    got = asg.cpu().numpy()
+    ref = O.kmeans_assign(zP, cent)
+    assert np.array_equal(got[:4, :T], ref[:4])
+    fin = np.isfinite(zP[4]).all(-1)
+    assert np.array_equal(got[4, :T][fin], ref[4][fin])
+    assert got[4, T - 1] == 0 and 0 <= got[4, 0] < C
+    assert (got[:, T:] == -1).all() and (asg8.cpu().numpy()[:, T:] == 255).all()
+    assert np.array_equal(asg8.cpu().numpy()[:, :T], got[:, :T].astype(np.uint8))
