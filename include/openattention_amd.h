@@ -465,6 +465,44 @@ int oa_query_metric(const void* q, int q_bf16, long q_stride_row, long q_stride_
 int oa_sym_eig_top(const float* M, long m_stride, int batch, int n, int k, float* evals,
                    float* evecs, int* sweeps, void* stream);
 
+/*
+ * One decode step, or one group of question rows, in one call: oa_index_prep (update = 1) or
+ * oa_qgs_prep (update = 0), then oa_qgs_scan_heads, oa_topk_gate_fill, oa_topq_heads and
+ * oa_residual_flash with these arguments, launched in order on the stream; the same outputs as those
+ * calls.  The first call to fail ends the step and its status is returned.
+ *
+ * Question rows (update = 0): 2^qshift query rows per sequence, laid out in every per-row array as
+ * row ((kv << qshift) + i) * 4 + head for KV row kv, question row i and head of the KV row's four;
+ * rows = (kv_rows << qshift) * 4.  Row i attends n + i keys (n from n_dev) of an index that already
+ * holds n + 2^qshift - 1 + later keys, and its cluster statistics are the index's with the keys from
+ * n + i on taken back in reverse position order (oa_index_downdate's arithmetic), formed in rnb
+ * (rows, C) and rSk, rSk2, rSv (rows, C, 128); the index is not changed.  With qshift = 0 and later =
+ * 0 they may be NULL.  sel has ns + nl + k_top columns; budget is oa_topk_gate_fill's, E the columns of
+ * exp_idx.
+ */
+typedef struct oa_step_args {
+  const void* q; long q_stride;
+  const void* K; const void* V; long kv_stride_b, kv_stride_s;
+  int rows, kv_rows, head_dim;
+  int update, qshift, later;
+  int8_t* codes; int Lmax;
+  const float* U; const float* scale; const void* W; const float* colmean; const float* cent; int C;
+  int32_t* asg; long asg_stride; uint8_t* asg8; long asg8_stride;
+  float* nb; float* Sk; float* Sk2; float* Sv;
+  int32_t* reclist; int32_t* reccnt; int rmax;
+  int8_t* limbs; int* fexp;
+  uint16_t* H; long h_stride; float* TM; long tm_stride; int ntiles; float* TMn;
+  float* S32; long s32_stride;
+  int32_t* sel; long sel_stride;
+  float* score; float* n_t; float* quota; float* qsk;
+  int32_t* exp_idx; int E; int budget;
+  void* out; long out_stride; int out_is_f32;
+  const int* n_dev; int ns, nl, k_top;
+  float sm_scale, sm_scale_sq;
+  float* rnb; float* rSk; float* rSk2; float* rSv;
+} oa_step_args;
+int oa_step(const oa_step_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -235,6 +235,15 @@ __device__ __forceinline__ int xcd_row(int b, int rows) {
   return (rows & 7) ? b : (b & 7) * (rows >> 3) + (b >> 3);
 }
 
+// Question rows.  A launch over several query rows per sequence (2^qsh of them) lays its rows out as
+// ((KV row << qsh) + question row) * 4 + head: unit u = row / 4 has its own query limbs, scores and
+// statistics; codes, keys, values and cluster ids are those of KV row u >> qsh, and question row i of
+// a unit sees n + i keys.  qsh = 0 is the decode step.  (A power of two, so that the map is a shift:
+// the per-row kernels are chains of dependent latencies, and a division would lengthen them.)
+__device__ __forceinline__ int row_kv(int row, int qsh) { return row >> (2 + qsh); }
+__device__ __forceinline__ int row_asg(int row, int qsh) { return ((row >> (2 + qsh)) << 2) | (row & 3); }
+__device__ __forceinline__ int row_extra(int row, int qsh) { return (row >> 2) & ((1 << qsh) - 1); }
+
 // order-preserving uint32 image of a float (larger float -> larger key, -inf lowest)
 __device__ __forceinline__ uint32_t float_key(float s) {
   const uint32_t b = __float_as_uint(s);

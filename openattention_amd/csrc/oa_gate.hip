@@ -17,6 +17,7 @@
 #include "oa_detmath.h"
 #include "oa_topk_row.h"
 #include "oa_gate_row.h"
+#include "oa_rows.h"
 
 namespace {
 
@@ -69,7 +70,7 @@ __device__ __forceinline__ void gate_row(const GateArgs& a, int row, float* s_sc
   const float q_lo = oa::bf16_to_f32(a.q[(long)row * a.q_stride + lane]);
   const float q_hi = oa::bf16_to_f32(a.q[(long)row * a.q_stride + lane + 64]);
   const float qq_lo = q_lo * q_lo, qq_hi = q_hi * q_hi;
-  const int cm = tokm >= 0 ? a.asg[(long)row * a.asg_stride + tokm] : -1;
+  const int cm = tokm >= 0 ? a.asg[(long)oa::row_asg(row, a.qsh) * a.asg_stride + tokm] : -1;
   uint4 kw0 = make_uint4(0u, 0u, 0u, 0u), kw1 = kw0;
   if (tok0 >= 0)
     kw0 = *reinterpret_cast<const uint4*>(a.K + (long)kvr * a.k_sb + (long)tok0 * a.k_ss + (e0 % kW) * 8);
@@ -595,7 +596,7 @@ __device__ __forceinline__ void fix_finish(const GateArgs& a, int row, FixLds& L
   // selected tokens: cluster ids (one per thread) and key words (16 bytes each, up to four per
   // thread), all requested together
   const int tokm = tid < n_sel ? L.sel[tid] : -1;
-  const int cm = tokm >= 0 ? a.asg[(long)row * a.asg_stride + tokm] : -1;
+  const int cm = tokm >= 0 ? a.asg[(long)oa::row_asg(row, a.qsh) * a.asg_stride + tokm] : -1;
   uint4 kw[4];
   int ke[4];
 #pragma unroll
@@ -759,7 +760,7 @@ __global__ void __launch_bounds__(64 * W) topk_gate2_fill_kernel(TopkArgs t, Gat
   const int tid = threadIdx.x;
   if (tid < 64)
     oa_sel::topk_reg_row<TPL, KR, true>(t.H, t.h_stride, t.TM, t.tm_stride, t.ntiles, sel,
-                                        a.sel_stride, *t.n_dev, t.ns, t.nl, t.k_top, t.rs, row, tid,
+                                        a.sel_stride, *t.n_dev + oa::row_extra(row, a.qsh), t.ns, t.nl, t.k_top, t.rs, row, tid,
                                         L.f.sel);
   else
     pooled_batches<W>(a, row, L);
@@ -825,17 +826,18 @@ extern "C" int oa_errorgate(const void* q, long q_stride, const void* K, long k_
   return OA_LAUNCH_STATUS();
 }
 
-extern "C" int oa_gate_fill(const void* q, long q_stride, const void* K, long k_stride_b,
+static int gate_fill(const void* q, long q_stride, const void* K, long k_stride_b,
                             long k_stride_s, int rows, int kv_rows, int head_dim,
                             const int32_t* asg, long asg_stride, const int32_t* sel, long sel_stride,
                             int n_sel, const float* Sk, const float* Sk2, const float* nb, int C,
                             float sm_scale, float sm_scale_sq, int budget, float* score, float* n_t,
-                            float* quota, float* qsk, void* stream) {
+                            float* quota, float* qsk, int qsh, void* stream) {
   if (head_dim != OA_D || kv_rows <= 0 || rows % kv_rows != 0 || n_sel < 0 || n_sel > kMaxSel ||
       C <= 0 || C > kMaxC || budget < 0 || k_stride_b % 8 || k_stride_s % 8 ||
       (reinterpret_cast<uintptr_t>(K) & 15))
     return OA_EINVAL;
-  GateArgs a;
+  GateArgs a{};
+  a.qsh = qsh;
   a.q = (const uint16_t*)q; a.q_stride = q_stride;
   a.K = (const uint16_t*)K; a.k_sb = k_stride_b; a.k_ss = k_stride_s; a.G = rows / kv_rows;
   a.asg = asg; a.asg_stride = asg_stride;
@@ -863,7 +865,18 @@ extern "C" int oa_gate_fill(const void* q, long q_stride, const void* K, long k_
   return launch_fill(score, n_t, rows, C, budget, quota, (hipStream_t)stream);
 }
 
-extern "C" int oa_topk_gate_fill(uint16_t* H, long h_stride, const float* TM, long tm_stride,
+extern "C" int oa_gate_fill(const void* q, long q_stride, const void* K, long k_stride_b,
+                            long k_stride_s, int rows, int kv_rows, int head_dim,
+                            const int32_t* asg, long asg_stride, const int32_t* sel, long sel_stride,
+                            int n_sel, const float* Sk, const float* Sk2, const float* nb, int C,
+                            float sm_scale, float sm_scale_sq, int budget, float* score, float* n_t,
+                            float* quota, float* qsk, void* stream) {
+  return gate_fill(q, q_stride, K, k_stride_b, k_stride_s, rows, kv_rows, head_dim, asg, asg_stride, sel,
+                   sel_stride, n_sel, Sk, Sk2, nb, C, sm_scale, sm_scale_sq, budget, score, n_t, quota, qsk, 0,
+                   stream);
+}
+
+int oa_rows::topk_gate_fill(uint16_t* H, long h_stride, const float* TM, long tm_stride,
                                  int ntiles, const int* n_dev, int ns, int nl, int k_top,
                                  const int8_t* codes, int Lmax, const int8_t* limbs,
                                  const int* fexp, const void* q, long q_stride, const void* K,
@@ -872,7 +885,7 @@ extern "C" int oa_topk_gate_fill(uint16_t* H, long h_stride, const float* TM, lo
                                  long sel_stride, const float* Sk, const float* Sk2,
                                  const float* nb, int C, float sm_scale, float sm_scale_sq,
                                  int budget, float* score, float* n_t, float* quota, float* qsk,
-                                 void* stream) {
+                                 int qsh, void* stream) {
   const int n_sel = ns + nl + k_top;
   const int tpl = (ntiles + 63) / 64;
   const int reg = (k_top <= 9 && tpl <= 9) ? 1 : (k_top <= 16 && tpl <= 16) ? 2 : (k_top <= 16 && tpl <= 32) ? 3 : 0;
@@ -881,16 +894,16 @@ extern "C" int oa_topk_gate_fill(uint16_t* H, long h_stride, const float* TM, lo
   // a B = 32 batch's rows waiting for a workgroup slot (measured slower than two launches)
   if (!reg || (rows >= kFuseRows && C > 64)) {
     // two launches: the top-k the row needs, then the gate and fill
-    int st = oa_topk_select_heads(H, h_stride, TM, tm_stride, rows, ntiles, sel, sel_stride, n_dev,
-                                  ns, nl, k_top, codes, kv_rows, Lmax, limbs, fexp, stream);
+    int st = oa_rows::topk_select_heads(H, h_stride, TM, tm_stride, rows, ntiles, sel, sel_stride, n_dev,
+                                  ns, nl, k_top, codes, kv_rows, Lmax, limbs, fexp, qsh, stream);
     if (st) return st;
-    return oa_gate_fill(q, q_stride, K, k_stride_b, k_stride_s, rows, kv_rows, head_dim, asg,
+    return gate_fill(q, q_stride, K, k_stride_b, k_stride_s, rows, kv_rows, head_dim, asg,
                         asg_stride, sel, sel_stride, n_sel, Sk, Sk2, nb, C, sm_scale, sm_scale_sq,
-                        budget, score, n_t, quota, qsk, stream);
+                        budget, score, n_t, quota, qsk, qsh, stream);
   }
   // the checks of both launches it replaces
   if (!H || !codes || !limbs || !fexp || !q || !K || !asg || (!sel && n_sel > 0) || !Sk || !Sk2 ||
-      !nb || !score || !n_t || !quota || kv_rows <= 0 || rows != kv_rows * oa_sel::GQ ||
+      !nb || !score || !n_t || !quota || kv_rows <= 0 || rows != (kv_rows << qsh) * oa_sel::GQ ||
       Lmax <= 0 || (reinterpret_cast<uintptr_t>(codes) & 15) ||
       (reinterpret_cast<uintptr_t>(limbs) & 3) || ntiles <= 0 || k_top < 0 || k_top > ntiles ||
       ns < 0 || nl < 0 || ns > 64 || nl > 64 || sel_stride < n_sel || head_dim != OA_D ||
@@ -900,8 +913,9 @@ extern "C" int oa_topk_gate_fill(uint16_t* H, long h_stride, const float* TM, lo
   TopkArgs t;
   t.H = H; t.h_stride = h_stride; t.TM = TM; t.tm_stride = tm_stride; t.ntiles = ntiles;
   t.n_dev = n_dev; t.ns = ns; t.nl = nl; t.k_top = k_top;
-  t.rs = oa_sel::Rescore{codes, (long)Lmax, limbs, fexp};
+  t.rs = oa_sel::Rescore{codes, (long)Lmax, limbs, fexp, qsh};
   GateArgs a{};
+  a.qsh = qsh;
   a.q = (const uint16_t*)q; a.q_stride = q_stride;
   a.K = (const uint16_t*)K; a.k_sb = k_stride_b; a.k_ss = k_stride_s; a.G = rows / kv_rows;
   a.asg = asg; a.asg_stride = asg_stride;
@@ -940,6 +954,22 @@ extern "C" int oa_topk_gate_fill(uint16_t* H, long h_stride, const float* TM, lo
 #undef OA_TG2_NS
 #undef OA_TG2
   return OA_LAUNCH_STATUS();
+}
+
+extern "C" int oa_topk_gate_fill(uint16_t* H, long h_stride, const float* TM, long tm_stride,
+                                 int ntiles, const int* n_dev, int ns, int nl, int k_top,
+                                 const int8_t* codes, int Lmax, const int8_t* limbs,
+                                 const int* fexp, const void* q, long q_stride, const void* K,
+                                 long k_stride_b, long k_stride_s, int rows, int kv_rows,
+                                 int head_dim, const int32_t* asg, long asg_stride, int32_t* sel,
+                                 long sel_stride, const float* Sk, const float* Sk2,
+                                 const float* nb, int C, float sm_scale, float sm_scale_sq,
+                                 int budget, float* score, float* n_t, float* quota, float* qsk,
+                                 void* stream) {
+  return oa_rows::topk_gate_fill(H, h_stride, TM, tm_stride, ntiles, n_dev, ns, nl, k_top, codes, Lmax, limbs,
+                                 fexp, q, q_stride, K, k_stride_b, k_stride_s, rows, kv_rows, head_dim, asg,
+                                 asg_stride, sel, sel_stride, Sk, Sk2, nb, C, sm_scale, sm_scale_sq, budget,
+                                 score, n_t, quota, qsk, 0, stream);
 }
 
 extern "C" int oa_waterfill(const float* score, const float* n_t, int rows, int C, int budget,

@@ -22,6 +22,7 @@ struct GateArgs {
   float* score; float* n_t; long out_stride;
   float* qsk;                                         // optional: q . Sk_c of every cluster
   int C; float sc; float sc2;
+  int qsh = 0;                                        // question rows per KV row (oa_common.h)
 };
 
 // x / den for den >= 1, given r = 1 / den correctly rounded: q = RN(x r) lies within one ulp of

@@ -17,13 +17,13 @@ __device__ __forceinline__ void qgs_prep_row(const uint16_t* __restrict__ q, lon
                                              const float* __restrict__ scale,  // (BH, RQ)
                                              int G, int8_t* __restrict__ limbs, // (BH, 16, RQ)
                                              int* __restrict__ fexp, float* __restrict__ zq_out,
-                                             int row, int lane) {
+                                             int row, int lane, int qsh = 0) {
   constexpr int RQ = kPrepRQ;
   const int kvr = row / G;
   const int g = row % G;
   const float q_lo = bf16_to_f32(q[(long)row * q_stride + lane]);
   const float q_hi = bf16_to_f32(q[(long)row * q_stride + lane + 64]);
-  const float* Ub = U + (long)kvr * OA_D * RQ;
+  const float* Ub = U + (long)(kvr >> qsh) * OA_D * RQ;
   // lane l holds rows l and l+64 of U (32 contiguous floats each)
   float ul[RQ], uh[RQ], sc[RQ];
 #pragma unroll
@@ -34,7 +34,7 @@ __device__ __forceinline__ void qgs_prep_row(const uint16_t* __restrict__ q, lon
     uh[j] = b.x; uh[j + 1] = b.y; uh[j + 2] = b.z; uh[j + 3] = b.w;
   }
 #pragma unroll
-  for (int j = 0; j < RQ; ++j) sc[j] = scale[(long)kvr * RQ + j];
+  for (int j = 0; j < RQ; ++j) sc[j] = scale[(long)(kvr >> qsh) * RQ + j];
   float myz = 0.f;
 #pragma unroll
   for (int j = 0; j < RQ; ++j) {

@@ -28,6 +28,7 @@
 // oa_residual writes kbar', vbar' (bf16) and ln n' instead of the softmax (the operator
 // surface of the reference's residual kernels), for use with oa_flash_decode.
 #include "oa_common.h"
+#include "oa_rows.h"
 
 namespace {
 
@@ -50,6 +51,7 @@ struct ResArgs {
   int C; float sm_scale;
   void* out; long out_stride; int out_f32;      // fused variant
   uint16_t* kbar_r; uint16_t* vbar_r; float* logn;  // residual-only variant
+  int qsh;                                      // question rows per KV row (oa_common.h)
 };
 
 struct Soft {
@@ -366,7 +368,7 @@ __global__ void __launch_bounds__(kRFThreads, 8) resflash_kernel(ResArgs a) {
   int scid = -1;
   const int stok = a.n_sel > 0 ? s_tok[min(tid, a.n_sel - 1)] : -1;
   if (a.n_sel > 0) {
-    const int c = a.asg[(long)row * a.asg_stride + max(stok, 0)];
+    const int c = a.asg[(long)oa::row_asg(row, a.qsh) * a.asg_stride + max(stok, 0)];
     scid = stok >= 0 ? c : -1;
   }
   for (int i = tid; i < NI; i += kRFThreads) {
@@ -497,7 +499,7 @@ int launch(bool fused, const void* q, long q_stride, const void* K, const void* 
            const int32_t* sel, long sel_stride, int n_sel, const int32_t* exp_idx, int E,
            const float* quota, const float* n_t, const float* Sk, const float* Sv, int C,
            float sm_scale, void* out, long out_stride, int out_f32, void* kbar_r, void* vbar_r,
-           float* logn, const float* qsk, void* stream) {
+           float* logn, const float* qsk, int qsh, void* stream) {
   if (head_dim != OA_D || kv_rows <= 0 || rows % kv_rows != 0 || C <= 0 || C > kMaxC ||
       n_sel < 0 || n_sel > kMaxSel || E < 0 || E > kMaxE || (kv_ss % 8) != 0 || (kv_sb % 8) != 0)
     return OA_EINVAL;
@@ -510,7 +512,7 @@ int launch(bool fused, const void* q, long q_stride, const void* K, const void* 
   a.exq = exp_idx; a.E = E; a.quota = quota; a.n_t = n_t; a.Sk = Sk; a.Sv = Sv; a.qsk = qsk;
   a.C = C; a.sm_scale = sm_scale;
   a.out = out; a.out_stride = out_stride; a.out_f32 = out_f32 ? 1 : 0;
-  a.kbar_r = (uint16_t*)kbar_r; a.vbar_r = (uint16_t*)vbar_r; a.logn = logn;
+  a.kbar_r = (uint16_t*)kbar_r; a.vbar_r = (uint16_t*)vbar_r; a.logn = logn; a.qsh = qsh;
   if (fused) {
     const size_t lds = sizeof(int) * 3 * (size_t)(n_sel + E);
     if (lds > 65536) {
@@ -526,6 +528,18 @@ int launch(bool fused, const void* q, long q_stride, const void* K, const void* 
 
 }  // namespace
 
+int oa_rows::residual_flash(const void* q, long q_stride, const void* K, const void* V, long kv_stride_b,
+                            long kv_stride_s, int rows, int kv_rows, const int32_t* asg, long asg_stride,
+                            const int32_t* sel, long sel_stride, int n_sel, const int32_t* exp_idx, int E,
+                            const float* quota, const float* n_t, const float* Sk, const float* Sv, int C,
+                            float sm_scale, void* out, long out_stride, int out_is_f32, const float* qsk,
+                            int qsh, void* stream) {
+  if (!out || (q_stride % 8) != 0 || rows != (kv_rows << qsh) * 4) return OA_EINVAL;
+  return launch(true, q, q_stride, K, V, kv_stride_b, kv_stride_s, rows, kv_rows, OA_D, asg, asg_stride, sel,
+                sel_stride, n_sel, exp_idx, E, quota, n_t, Sk, Sv, C, sm_scale, out, out_stride, out_is_f32,
+                nullptr, nullptr, nullptr, qsk, qsh, stream);
+}
+
 extern "C" int oa_residual_flash(const void* q, long q_stride, const void* K, const void* V,
                                  long kv_stride_b, long kv_stride_s, int rows, int kv_rows,
                                  int head_dim, const int32_t* asg, long asg_stride,
@@ -537,7 +551,7 @@ extern "C" int oa_residual_flash(const void* q, long q_stride, const void* K, co
   if (!out || (q_stride % 8) != 0) return OA_EINVAL;
   return launch(true, q, q_stride, K, V, kv_stride_b, kv_stride_s, rows, kv_rows, head_dim, asg,
                 asg_stride, sel, sel_stride, n_sel, exp_idx, E, quota, n_t, Sk, Sv, C, sm_scale,
-                out, out_stride, out_is_f32, nullptr, nullptr, nullptr, qsk, stream);
+                out, out_stride, out_is_f32, nullptr, nullptr, nullptr, qsk, 0, stream);
 }
 
 extern "C" int oa_residual(const void* K, const void* V, long kv_stride_b, long kv_stride_s,
@@ -550,5 +564,5 @@ extern "C" int oa_residual(const void* K, const void* V, long kv_stride_b, long 
   // the residual-only variant reads no query; K stands in so the pointer is valid
   return launch(false, K, 0, K, V, kv_stride_b, kv_stride_s, rows, kv_rows, head_dim, asg,
                 asg_stride, sel, sel_stride, n_sel, exp_idx, E, quota, n_t, Sk, Sv, C, 0.f,
-                nullptr, 0, 0, kbar_r, vbar_r, log_n, nullptr, stream);
+                nullptr, 0, 0, kbar_r, vbar_r, log_n, nullptr, 0, stream);
 }

@@ -21,6 +21,7 @@
 #include "oa_prep.h"
 #include "oa_topk_row.h"
 #include "oa_gate_row.h"
+#include "oa_rows.h"
 
 typedef int oa_v4i __attribute__((ext_vector_type(4)));
 
@@ -37,8 +38,8 @@ __global__ void __launch_bounds__(64) qgs_prep_kernel(const uint16_t* __restrict
                                                       const float* __restrict__ scale, int G,
                                                       int8_t* __restrict__ limbs,
                                                       int* __restrict__ fexp,
-                                                      float* __restrict__ zq_out) {
-  oa::qgs_prep_row(q, q_stride, U, scale, G, limbs, fexp, zq_out, blockIdx.x, threadIdx.x);
+                                                      float* __restrict__ zq_out, int qsh) {
+  oa::qgs_prep_row(q, q_stride, U, scale, G, limbs, fexp, zq_out, blockIdx.x, threadIdx.x, qsh);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -56,6 +57,7 @@ struct ScanArgs {
   void* Sv; long s_stride; float* TM; long tm_stride;
   const int* n_dev; int ns; int nl;
   float* TMn;      // optional: each tile's least finite score (+inf for a tile without one)
+  int qsh = 0;     // question rows per KV row: block row kvr is unit (KV row << qsh) + question row
 };
 
 // HEADS: the score rows hold 16-bit key heads (oa::score_head) instead of fp32 scores.
@@ -79,7 +81,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs& sa, int chunk, int kv
   const int nn = lane & 15;        // token inside a 16-token block; limb row for A
   const int tile_begin = chunk * (kTokWG / 64) + wave * kTilesPerWave;
   const int ntile_total = (Lmax + 63) / 64;
-  const int8_t* cb = codes + (long)kvr * Lmax * RQ;
+  const int8_t* cb = codes + (long)(kvr >> sa.qsh) * Lmax * RQ;
   // every code of the wave's tiles in flight at once (addresses clamped to the last token;
   // tokens past Lmax are zeroed below)
   long b_op[kTilesPerWave][4];
@@ -91,7 +93,7 @@ __device__ __forceinline__ void scan_block(const ScanArgs& sa, int chunk, int kv
       b_op[t][b] = __builtin_nontemporal_load(
           reinterpret_cast<const long*>(cb + (long)min(tok, Lmax - 1) * RQ + kg * 8));
     }
-  const int n = *sa.n_dev;
+  const int n = *sa.n_dev + (kvr & ((1 << sa.qsh) - 1));
   const int dead_hi = n - nl;      // positions >= dead_hi are local or not yet written
   const long a_op = *reinterpret_cast<const long*>(limbs + (long)kvr * 16 * RQ + nn * RQ + kg * 8);
   const int row = kvr * GQ + kg;
@@ -226,7 +228,7 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
   __shared__ unsigned long long s_win[kMaxTop];
   const int row = oa::xcd_row(blockIdx.x, gridDim.x);   // a KV row's query rows share one L2
   const int lane = threadIdx.x;
-  const int n = *n_dev;
+  const int n = *n_dev + oa::row_extra(row, rs.qsh);
   const int dead_hi = n - nl;
   if (k_top == 0) {                                     // uniform: sink and local only
     int32_t* sr = sel + (long)row * sel_stride;
@@ -298,7 +300,7 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
   if (HEADS) {
     // exact scores of the list, four candidates' codes in flight per lane (a dead candidate
     // scores -inf; its code address is clamped into the row's written positions)
-    const int kvr = row / GQ;
+    const int kvr = oa::row_kv(row, rs.qsh);
     for (int i0 = 0; i0 < nc; i0 += 256) {
       int pos[4];
       uint4 c0[4], c1[4];
@@ -363,8 +365,8 @@ __global__ void __launch_bounds__(64) topk_select_reg_kernel(void* __restrict__ 
                                                              const int* __restrict__ n_dev, int ns,
                                                              int nl, int k_top, Rescore rs) {
   const int row = oa::xcd_row(blockIdx.x, gridDim.x);   // a KV row's query rows share one L2
-  topk_reg_row<TPL, KR, HEADS>(Sv, s_stride, TM, tm_stride, ntiles, sel, sel_stride, *n_dev, ns,
-                               nl, k_top, rs, row, threadIdx.x);
+  topk_reg_row<TPL, KR, HEADS>(Sv, s_stride, TM, tm_stride, ntiles, sel, sel_stride,
+                               *n_dev + oa::row_extra(row, rs.qsh), ns, nl, k_top, rs, row, threadIdx.x);
 }
 
 }  // namespace
@@ -374,7 +376,7 @@ extern "C" int oa_qgs_prep(const void* q, long q_stride, const float* U, const f
                            float* zq_out, void* stream) {
   if (head_dim != OA_D || rank != RQ || kv_rows <= 0 || rows != kv_rows * GQ) return OA_EINVAL;
   hipLaunchKernelGGL(qgs_prep_kernel, dim3(rows), dim3(64), 0, (hipStream_t)stream,
-                     (const uint16_t*)q, q_stride, U, scale, GQ, limbs, fexp, zq_out);
+                     (const uint16_t*)q, q_stride, U, scale, GQ, limbs, fexp, zq_out, 0);
   return OA_LAUNCH_STATUS();
 }
 
@@ -382,12 +384,12 @@ namespace {
 template <bool HEADS>
 int launch_scan(const int8_t* codes, int kv_rows, int Lmax, int rank, const int8_t* limbs,
                 const int* fexp, void* S, long s_stride, float* TM, long tm_stride, float* TMn,
-                const int* n_dev, int ns, int nl, void* stream) {
+                const int* n_dev, int ns, int nl, void* stream, int qsh = 0) {
   if (rank != RQ || kv_rows <= 0 || Lmax <= 0) return OA_EINVAL;
   const int ntile = (Lmax + 63) / 64;
   if (s_stride < (long)ntile * 64 || tm_stride < ntile || ns < 0 || nl < 0) return OA_EINVAL;
-  dim3 grid((Lmax + kTokWG - 1) / kTokWG, kv_rows);
-  const ScanArgs sa{codes, Lmax, limbs, fexp, S, s_stride, TM, tm_stride, n_dev, ns, nl, TMn};
+  dim3 grid((Lmax + kTokWG - 1) / kTokWG, kv_rows << qsh);
+  const ScanArgs sa{codes, Lmax, limbs, fexp, S, s_stride, TM, tm_stride, n_dev, ns, nl, TMn, qsh};
   if (TMn)
     hipLaunchKernelGGL((qgs_scan_kernel<HEADS, true>), grid, dim3(kScanThreads), 0, (hipStream_t)stream, sa);
   else
@@ -442,6 +444,32 @@ extern "C" int oa_qgs_scan_heads(const int8_t* codes, int kv_rows, int Lmax, int
                            TMn, n_dev, ns, nl, stream);
 }
 
+namespace oa_rows {
+int qgs_prep(const void* q, long q_stride, const float* U, const float* scale, int kv_rows, int8_t* limbs,
+             int* fexp, int qsh, void* stream) {
+  hipLaunchKernelGGL(qgs_prep_kernel, dim3((kv_rows << qsh) * GQ), dim3(64), 0, (hipStream_t)stream,
+                     (const uint16_t*)q, q_stride, U, scale, GQ, limbs, fexp, (float*)nullptr, qsh);
+  return OA_LAUNCH_STATUS();
+}
+int scan_heads(const int8_t* codes, int kv_rows, int Lmax, const int8_t* limbs, const int* fexp, uint16_t* H,
+               long h_stride, float* TM, long tm_stride, float* TMn, const int* n_dev, int ns, int nl, int qsh,
+               void* stream) {
+  if (!H || (reinterpret_cast<uintptr_t>(H) & 7) || h_stride % 4) return OA_EINVAL;
+  return launch_scan<true>(codes, kv_rows, Lmax, RQ, limbs, fexp, H, h_stride, TM, tm_stride, TMn, n_dev, ns,
+                           nl, stream, qsh);
+}
+int topk_select_heads(uint16_t* H, long h_stride, const float* TM, long tm_stride, int rows, int ntiles,
+                      int32_t* sel, long sel_stride, const int* n_dev, int ns, int nl, int k_top,
+                      const int8_t* codes, int kv_rows, int Lmax, const int8_t* limbs, const int* fexp,
+                      int qsh, void* stream) {
+  if (!H || !codes || !limbs || !fexp || kv_rows <= 0 || rows != (kv_rows << qsh) * GQ || Lmax <= 0 ||
+      (reinterpret_cast<uintptr_t>(codes) & 15) || (reinterpret_cast<uintptr_t>(limbs) & 3))
+    return OA_EINVAL;
+  return launch_topk<true>(H, h_stride, TM, tm_stride, rows, ntiles, sel, sel_stride, n_dev, ns,
+                           nl, k_top, Rescore{codes, (long)Lmax, limbs, fexp, qsh}, stream);
+}
+}  // namespace oa_rows
+
 extern "C" int oa_topk_select(float* S, long s_stride, const float* TM, long tm_stride, int rows,
                               int ntiles, int32_t* sel, long sel_stride, const int* n_dev, int ns,
                               int nl, int k_top, void* stream) {
@@ -454,11 +482,8 @@ extern "C" int oa_topk_select_heads(uint16_t* H, long h_stride, const float* TM,
                                     const int* n_dev, int ns, int nl, int k_top,
                                     const int8_t* codes, int kv_rows, int Lmax,
                                     const int8_t* limbs, const int* fexp, void* stream) {
-  if (!H || !codes || !limbs || !fexp || kv_rows <= 0 || rows != kv_rows * GQ || Lmax <= 0 ||
-      (reinterpret_cast<uintptr_t>(codes) & 15) || (reinterpret_cast<uintptr_t>(limbs) & 3))
-    return OA_EINVAL;
-  return launch_topk<true>(H, h_stride, TM, tm_stride, rows, ntiles, sel, sel_stride, n_dev, ns,
-                           nl, k_top, Rescore{codes, (long)Lmax, limbs, fexp}, stream);
+  return oa_rows::topk_select_heads(H, h_stride, TM, tm_stride, rows, ntiles, sel, sel_stride, n_dev, ns, nl,
+                                    k_top, codes, kv_rows, Lmax, limbs, fexp, 0, stream);
 }
 
 extern "C" int oa_qgs_scan_gate(const int8_t* codes, int kv_rows, int Lmax, int rank,

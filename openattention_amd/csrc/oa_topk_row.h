@@ -24,6 +24,7 @@ struct Rescore {
   const int8_t* codes; long lmax;   // (BH, Lmax, 32)
   const int8_t* limbs;              // (BH, 16, 32)
   const int* fexp;                  // (R,)
+  int qsh = 0;                      // question rows per KV row (oa_common.h)
 };
 
 // candidate score of position pos of a query-head row (sink, local and unwritten: -inf)
@@ -33,7 +34,7 @@ __device__ __forceinline__ float cand_score(const void* Sv, long s_stride, int r
                                             double inv) {
   if (!HEADS) return static_cast<const float*>(Sv)[(long)row * s_stride + pos];
   if (pos < ns || pos >= dead_hi) return -INFINITY;
-  return oa::qgs_score(rs.codes, rs.lmax, row / GQ, pos, lw, inv);
+  return oa::qgs_score(rs.codes, rs.lmax, oa::row_kv(row, rs.qsh), pos, lw, inv);
 }
 template <bool HEADS>
 __device__ __forceinline__ void mark_selected(void* Sv, long s_stride, int row, int pos) {
@@ -98,7 +99,7 @@ __device__ __forceinline__ void topk_reg_row(void* __restrict__ Sv, long s_strid
     // others count as -inf
     // (the heads and every candidate's code are loaded in one round)
     const uint16_t* Hrow = static_cast<const uint16_t*>(Sv) + (long)row * s_stride;
-    const int kvr = row / GQ;
+    const int kvr = oa::row_kv(row, rs.qsh);
     const int dead_hi = n - nl;
     uint32_t hv[KR];
     uint4 cw[KR][2];

@@ -51,6 +51,7 @@
 
 #include "oa_common.h"
 #include "oa_score.h"
+#include "oa_rows.h"
 
 namespace {
 
@@ -96,6 +97,7 @@ struct TopqArgs {
   // least finite score (TMn) from the scan; then the row's range comes from them instead of a
   // pass over the row, and every group of positions is binned as soon as it arrives
   const float* TM; const float* TMn; long tm_stride;
+  int qsh;         // question rows per KV row (oa_common.h)
 };
 
 // the largest t = head - 0x7f of a finite float (head 0xff7f): the linear-bin kernel caps t here
@@ -475,9 +477,9 @@ __device__ __forceinline__ void topq_row_body(const TopqArgs& a, int row, unsign
   constexpr int sh1 = 32 - LB;
   constexpr int sh1p = sh1 + sb;          // shift giving a level-1 bin's pad-word count
   const int trash = C * HS + lane;        // per-lane histogram slot for non-members
-  const int n = *a.n_dev;
+  const int n = *a.n_dev + oa::row_extra(row, a.qsh);
   const float* srow = a.S + (long)row * a.s_stride;
-  const uint8_t* arow = a.asg8 + (long)row * a.a_stride;
+  const uint8_t* arow = a.asg8 + (long)oa::row_asg(row, a.qsh) * a.a_stride;
   int32_t* erow = a.exp_idx + (long)row * E;
 
   // register i of a thread holds position sg*SEG + (i/4)*4096 + 4*tid + i%4: each group of four
@@ -930,12 +932,12 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
   const int wave = tid >> 6;
   const int lane = tid & 63;
   const int C = a.C, E = a.E;
-  const int n = *a.n_dev;
+  const int n = *a.n_dev + oa::row_extra(row, a.qsh);
   const float* srow = a.S + (long)row * a.s_stride;
   const uint16_t* hrow = a.H + (long)row * a.h_stride;
-  const uint8_t* arow = a.asg8 + (long)row * a.a_stride;
+  const uint8_t* arow = a.asg8 + (long)oa::row_asg(row, a.qsh) * a.a_stride;
   int32_t* erow = a.exp_idx + (long)row * E;
-  const int kvr = row / 4;
+  const int kvr = oa::row_kv(row, a.qsh);
 
   constexpr int SEG = kThreads * PPT;
   constexpr int NG = PPT / 4;
@@ -1024,7 +1026,7 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
   float qv[4];
   if (wave == 0) quota_load(a.quota + (long)row * C, C, lane, qv);
   int lwv = 0;
-  if (HEADS && tid < 32) lwv = oa::limb_words(a.limbs, kvr, row % 4)[tid];
+  if (HEADS && tid < 32) lwv = oa::limb_words(a.limbs, row / 4, row % 4)[tid];
   const int ntu = (n + 63) / 64;
   constexpr int TL = kMulti ? kTileLd : 1;
   float tx[TL], tn[TL];
@@ -1446,15 +1448,15 @@ extern "C" int oa_topq(const float* S, long s_stride, const uint8_t* asg8, long 
 // over 16-bit key heads (oa_qgs_scan_heads + oa_topk_select_heads).  path 0: as oa_topq (rows
 // the linear-bin kernel leaves are recomputed into S32 and selected by the key-prefix kernel);
 // path 2: the linear-bin kernel alone; path 3: every row is left to the key-prefix kernel
-extern "C" int oa_topq_heads(const uint16_t* H, long h_stride, const uint8_t* asg8,
+int oa_rows::topq_heads(const uint16_t* H, long h_stride, const uint8_t* asg8,
                              long asg8_stride, const float* quota, int rows, int C, int Lmax,
                              int32_t* exp_idx, int E, const int* n_dev, const int8_t* codes,
                              int kv_rows, const int8_t* limbs, const int* fexp, float* S32,
                              long s32_stride, const float* TM, const float* TMn, long tm_stride,
-                             int path, void* stream) {
+                             int path, int qsh, void* stream) {
   const long lmax4 = ((long)Lmax + 3) & ~3L;
   if (!topq_sizes_ok(rows, C, E, Lmax) || !H || !asg8 || !quota || !n_dev || !codes || !limbs ||
-      !fexp || !S32 || (E > 0 && !exp_idx) || kv_rows <= 0 || rows != kv_rows * 4 ||
+      !fexp || !S32 || (E > 0 && !exp_idx) || kv_rows <= 0 || rows != (kv_rows << qsh) * 4 ||
       (!TM != !TMn) || (TM && tm_stride < ((long)Lmax + 63) / 64) ||
       h_stride % 4 || asg8_stride % 4 || s32_stride % 4 || h_stride < lmax4 ||
       asg8_stride < lmax4 || s32_stride < lmax4 || (reinterpret_cast<uintptr_t>(H) & 7) ||
@@ -1468,6 +1470,16 @@ extern "C" int oa_topq_heads(const uint16_t* H, long h_stride, const uint8_t* as
   a.C = C; a.E = E; a.n_dev = n_dev; a.exp_idx = exp_idx;
   a.H = H; a.h_stride = h_stride; a.codes = codes; a.lmax_codes = Lmax; a.limbs = limbs;
   a.fexp = fexp; a.S32 = S32; a.s32_stride = s32_stride; a.force_mark = path == 3;
-  a.TM = TM; a.TMn = TMn; a.tm_stride = tm_stride;
+  a.TM = TM; a.TMn = TMn; a.tm_stride = tm_stride; a.qsh = qsh;
   return topq_launch(a, rows, C, Lmax, E, true, true, path != 2, (hipStream_t)stream);
+}
+
+extern "C" int oa_topq_heads(const uint16_t* H, long h_stride, const uint8_t* asg8,
+                             long asg8_stride, const float* quota, int rows, int C, int Lmax,
+                             int32_t* exp_idx, int E, const int* n_dev, const int8_t* codes,
+                             int kv_rows, const int8_t* limbs, const int* fexp, float* S32,
+                             long s32_stride, const float* TM, const float* TMn, long tm_stride,
+                             int path, void* stream) {
+  return oa_rows::topq_heads(H, h_stride, asg8, asg8_stride, quota, rows, C, Lmax, exp_idx, E, n_dev, codes,
+                             kv_rows, limbs, fexp, S32, s32_stride, TM, TMn, tm_stride, path, 0, stream);
 }

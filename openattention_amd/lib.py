@@ -19,6 +19,20 @@ I = ct.c_int
 F = ct.c_float
 Dd = ct.c_double
 
+class StepArgs(ct.Structure):
+    """oa_step_args of the header, field for field."""
+    _fields_ = [("q", P), ("q_stride", L), ("K", P), ("V", P), ("kv_stride_b", L), ("kv_stride_s", L),
+                ("rows", I), ("kv_rows", I), ("head_dim", I), ("update", I), ("qshift", I), ("later", I),
+                ("codes", P), ("Lmax", I), ("U", P), ("scale", P), ("W", P), ("colmean", P), ("cent", P), ("C", I),
+                ("asg", P), ("asg_stride", L), ("asg8", P), ("asg8_stride", L),
+                ("nb", P), ("Sk", P), ("Sk2", P), ("Sv", P), ("reclist", P), ("reccnt", P), ("rmax", I),
+                ("limbs", P), ("fexp", P), ("H", P), ("h_stride", L), ("TM", P), ("tm_stride", L), ("ntiles", I),
+                ("TMn", P), ("S32", P), ("s32_stride", L), ("sel", P), ("sel_stride", L),
+                ("score", P), ("n_t", P), ("quota", P), ("qsk", P), ("exp_idx", P), ("E", I), ("budget", I),
+                ("out", P), ("out_stride", L), ("out_is_f32", I), ("n_dev", P), ("ns", I), ("nl", I), ("k_top", I),
+                ("sm_scale", F), ("sm_scale_sq", F), ("rnb", P), ("rSk", P), ("rSk2", P), ("rSv", P)]
+
+
 # name -> argtypes, in the order of include/openattention_amd.h
 SIGNATURES = {
     "oa_abi_version": [],
@@ -60,6 +74,7 @@ SIGNATURES = {
     "oa_cluster_sums": [P, P, L, L, I, I, I, I, P, P, P, P, P, L, P, P, P],
     "oa_query_metric": [P, I, L, L, I, I, P, I, P, P, Dd, P, I, P, P, P],
     "oa_sym_eig_top": [P, L, I, I, I, P, P, P, P],
+    "oa_step": [ct.POINTER(StepArgs), P],
 }
 
 # must equal oa_abi_version() of the loaded library (OA_ABI_VERSION in the header): a library

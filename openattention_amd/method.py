@@ -27,6 +27,7 @@ G = HQ // HKV
 SC = D ** -0.5
 RMAX = 256
 SCAN_TILE = 64
+ROWS_FULL = 1024           # query-head rows of a multi-row call's launch (4 per compute unit)
 TOPQ_SEGMENT = 36 * 1024   # positions the top-q kernel holds in registers at once (36 per thread)
 
 
@@ -251,13 +252,8 @@ class OursHIP(Method):
         return self.stages(self.st[l], C.K[l].view(-1, self.Lmax, D), C.V[l].view(-1, self.Lmax, D), q,
                            C.n_dev, n)[0]
 
-    def stages(self, st, K, V, q, n_dev, n, counts: tuple | None = None, update_index: bool = True):
-        """The decode stages over an explicit index state and K, V (B * HKV, >= n, D) bf16 rows
-        (any row stride), as (name, call) pairs in launch order, and the step's sel buffer.
-        n on the host fixes the sink / local / top-k counts unless `counts` = (ns, nl, k_top)
-        gives them; n_dev holds n on the device.  update_index: the first stage adds the token
-        at n - 1 to the index (the decode step); otherwise it only projects the queries (a row
-        of a multi-row call over an index that already holds its keys)."""
+    def _step_inputs(self, K, V, q, n, counts):
+        """The checked inputs of a step: its query rows, sel buffer and sink / local / top-k counts."""
         qr = q.reshape(self.R, D)
         if not qr.is_contiguous():
             qr = qr.contiguous()
@@ -268,8 +264,16 @@ class OursHIP(Method):
         ns, nl, k_top = self.bud.counts(n) if counts is None else counts
         if n - ns - nl < k_top:
             raise ValueError(f"n={n} too small for sink {ns} + local {nl} + top-k {k_top}")
-        NS = ns + nl + k_top
-        sel = self.sel_buffer(NS)
+        return qr, self.sel_buffer(ns + nl + k_top), ns, nl, k_top
+
+    def stages(self, st, K, V, q, n_dev, n, counts: tuple | None = None, update_index: bool = True):
+        """The decode stages over an explicit index state and K, V (B * HKV, >= n, D) bf16 rows
+        (any row stride), as (name, call) pairs in launch order, and the step's sel buffer.
+        n on the host fixes the sink / local / top-k counts unless `counts` = (ns, nl, k_top)
+        gives them; n_dev holds n on the device.  update_index: the first stage adds the token
+        at n - 1 to the index (the decode step); otherwise it only projects the queries (a row
+        of a multi-row call over an index that already holds its keys)."""
+        qr, sel, ns, nl, k_top = self._step_inputs(K, V, q, n, counts)
         sc = self.sm_scale
         out = []
         if update_index:
@@ -347,6 +351,13 @@ class OursHIP(Method):
                 main.wait_stream(s)
             self.last_sel = sel
             return self.out.view(self.B, HQ, 1, D)
+        if self.fused and self.gate_mode == "fused" and marks is None:
+            # the same launches from one call of the library
+            qr, sel, ns, nl, k_top = self._step_inputs(K, V, q, n, counts)
+            ops.step(K, V, st, n_dev, qr, self, sel, self.out, ns, nl, k_top, self.sm_scale, self.E, RMAX,
+                     update=update_index)
+            self.last_sel = sel
+            return self.out.view(self.B, HQ, 1, D)
         calls, sel = self.stages(st, K, V, q, n_dev, n, counts=counts, update_index=update_index)
         mark("start")
         for name, fn in calls:
@@ -375,6 +386,8 @@ class OursHIP(Method):
         if n_keys - Q + 1 - ns - nl < k_top:
             raise ValueError(f"{n_keys} keys leave the first of {Q} causal rows too few positions for "
                              f"sink {ns} + local {nl} + top-k {k_top}")
+        if self.fused and self.gate_mode == "fused" and self.groups == 1:
+            return self._rows_grouped(st, K, V, q, n_dev, n_keys, out, record, counts)
         snap = (st.nb.clone(), st.Sk.clone(), st.Sk2.clone(), st.Sv.clone())
         try:
             for i in range(Q - 1, -1, -1):
@@ -389,6 +402,59 @@ class OursHIP(Method):
         finally:
             for t, s in zip((st.nb, st.Sk, st.Sk2, st.Sv), snap):
                 t.copy_(s)
+            n_dev.fill_(n_keys)
+        return out
+
+    def _rows_grouped(self, st, K, V, q, n_dev, n_keys, out, record, counts):
+        """rows_step with the rows taken in groups of a power of two, each group one launch per stage
+        over every sequence's rows (ops.step's question rows; every row's statistics formed beside the
+        index, which is not changed).  The group is the largest whose rows fill the chip, ROWS_FULL
+        query-head rows: 64 rows of one 32K sequence took 64 chains of 5 launches at 32 of 256 compute
+        units, 5.0 ms of device time (8.9 ms with the host's 600 launches), and take 0.4 ms."""
+        B, _, Q, _ = q.shape
+        ns, nl, k_top = counts
+        NS, C = ns + nl + k_top, self.Cn
+        sh_max = max(0, (max(1, ROWS_FULL // self.R)).bit_length() - 1)
+        while sh_max and (1 << sh_max) > Q:
+            sh_max -= 1
+        # work buffers of the largest group, shared by all (a smaller group uses their first rows)
+        R = self.R << sh_max
+        f32 = dict(device=q.device, dtype=torch.float32)
+        i32 = dict(device=q.device, dtype=torch.int32)
+        one = lambda t, **kw: torch.empty((R,) + t.shape[1:], **kw)  # noqa: E731
+        w = dict(limbs=torch.empty(R // G, 16, 32, device=q.device, dtype=torch.int8), fexp=torch.empty(R, **i32),
+                 H=one(self.H, device=q.device, dtype=torch.int16), TM=one(self.TM, **f32),
+                 TMn=None if self.TMn is None else one(self.TMn, **f32), S=one(self.S, **f32),
+                 score=torch.empty(R, C, **f32), n_t=torch.empty(R, C, **f32), quota=torch.empty(R, C, **f32),
+                 qsk=torch.empty(R, C, **f32), exp_idx=one(self.exp_idx, **i32))
+        stats = (torch.empty(R, C, **f32),) + tuple(torch.empty(R, C, D, **f32) for _ in range(3))
+        sel = torch.empty(R, NS, **i32)
+        o = torch.empty(R, D, device=q.device, dtype=self.out.dtype)
+        # rows ((kv row, question row), head of the KV row's four)
+        qr = q.view(B, HKV, G, Q, D).permute(0, 1, 3, 2, 4)
+        outr = out.view(B, HKV, G, Q, D).permute(0, 1, 3, 2, 4)
+        i0 = Q
+        try:
+            while i0 > 0:
+                sh = min(sh_max, i0.bit_length() - 1)
+                nq = 1 << sh
+                i0 -= nq
+                Rg = self.R << sh
+                n_dev.fill_(n_keys - Q + i0 + 1)
+                wg = types.SimpleNamespace(**{k: None if t is None else t[:Rg if k != "limbs" else Rg // G]
+                                              for k, t in w.items()})
+                ops.step(K, V, st, n_dev, qr[:, :, i0:i0 + nq].reshape(Rg, D), wg, sel[:Rg], o[:Rg], ns, nl, k_top,
+                         self.sm_scale, self.E, RMAX, update=False, qshift=sh, later=Q - i0 - nq,
+                         stats=tuple(t[:Rg] for t in stats))
+                outr[:, :, i0:i0 + nq] = o[:Rg].view(B, HKV, nq, G, D)
+                row = lambda t, j: t[:Rg].view(B * HKV, nq, G, -1)[:, j].reshape(self.R, -1)  # noqa: E731
+                if record is not None:
+                    for j in range(nq - 1, -1, -1):
+                        record.append((i0 + j, row(sel, j).clone(), row(w["quota"], j).clone(),
+                                       row(w["exp_idx"], j).clone()))
+                if i0 == 0:
+                    self.last_sel = row(sel, 0)
+        finally:
             n_dev.fill_(n_keys)
         return out
 

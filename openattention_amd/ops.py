@@ -416,6 +416,67 @@ def topk_fix_fill(H, TM, n_dev, ns: int, nl: int, k_top: int, codes, limbs, fexp
              _ptr(quota), _stream(dev))
 
 
+_ROW_MAPS: tuple = (("score", torch.float32), ("n_t", torch.float32), ("quota", torch.float32),
+                    ("qsk", torch.float32))
+
+
+def step(K, V, st, n_dev, q, w, sel, out, ns: int, nl: int, k_top: int, sm_scale: float, E: int, rmax: int,
+         update: bool = True, qshift: int = 0, later: int = 0, stats=None) -> None:
+    """The decode stages in one call (oa_step): index_prep (update) or qgs_prep, qgs_scan_heads,
+    topk_gate_fill, topq_heads, residual_flash over the index st and the work buffers of w (limbs,
+    fexp, H, TM, TMn, S, score, n_t, quota, qsk, exp_idx); the same outputs.  qshift > 0 or later > 0
+    (update False): 2^qshift question rows per sequence, rows laid out ((kv << qshift) + i) * 4 + head
+    in q, sel, out and w; stats = (nb, Sk, Sk2, Sv) receives their statistics."""
+    dev = _dev(K, V, n_dev, q, w.limbs, w.fexp, w.H, w.TM, w.S, w.score, w.n_t, w.quota, w.exp_idx, sel, out)
+    BH, Lk, _ = K.shape
+    Lmax = st.codes.shape[1]
+    R, C = st.nb.shape
+    Rv = R << qshift
+    _chk(K, "K", torch.bfloat16, (BH, None, HEAD_DIM))
+    _need(V.shape == K.shape and V.stride() == K.stride() and V.dtype == K.dtype, "V must match K")
+    _need(R == GROUP * BH, "nb must have one row per query-head row")
+    _chk(st.codes, "codes", torch.int8, (BH, None, RANK_Q), contiguous=True)
+    _chk(st.asg, "asg", torch.int32, (R, -Lk))
+    _chk(st.asg8, "asg8", torch.uint8, (R, -max(Lk, Lmax)))
+    _chk(st.nb, "nb", torch.float32, (R, C), contiguous=True)
+    _stats(R, C, (st.Sk, "Sk"), (st.Sk2, "Sk2"), (st.Sv, "Sv"))
+    if update:
+        _need(Lmax >= Lk, "codes: fewer positions than K")
+    _chk(n_dev, "n_dev", torch.int32)
+    _chk(q, "q", torch.bfloat16, (Rv, HEAD_DIM))
+    _chk(w.limbs, "limbs", torch.int8, (BH << qshift, 16, RANK_Q), contiguous=True)
+    _chk(w.fexp, "fexp", torch.int32, (Rv,), contiguous=True)
+    _chk(w.H, "H", torch.int16, (Rv, -Lmax))
+    _chk(w.TM, "TM", torch.float32, (Rv, -((Lmax + 63) // 64)))
+    _tile_min(w.TM, w.TMn)
+    _chk(w.S, "S32", torch.float32, (Rv, -Lmax))
+    _chk(sel, "sel", torch.int32, (Rv, ns + nl + k_top), contiguous=True)
+    for name, dtype in _ROW_MAPS:
+        _chk(getattr(w, name), name, dtype, (Rv, C), contiguous=True)
+    _chk(w.exp_idx, "exp_idx", torch.int32, (Rv, None), contiguous=True)
+    Ex = w.exp_idx.shape[1]
+    _need(out.shape == (Rv, HEAD_DIM) and out.dtype in (torch.bfloat16, torch.float32) and out.stride(1) == 1,
+          "out must be (rows, 128) bf16 or fp32 with contiguous rows")
+    rs = (None,) * 4
+    if qshift or later:
+        _need(stats is not None, "question rows need their statistics' buffers")
+        _chk(stats[0], "row nb", torch.float32, (Rv, C), contiguous=True)
+        _stats(Rv, C, (stats[1], "row Sk"), (stats[2], "row Sk2"), (stats[3], "row Sv"))
+        rs = tuple(t.data_ptr() for t in stats)
+    a = lib.StepArgs(
+        q.data_ptr(), q.stride(0), K.data_ptr(), V.data_ptr(), K.stride(0), K.stride(1), Rv, BH, HEAD_DIM,
+        int(update), qshift, later, st.codes.data_ptr(), Lmax, st.U.data_ptr(), st.scale.data_ptr(),
+        st.W.data_ptr(), st.colmean.data_ptr(), st.cent.data_ptr(), C, st.asg.data_ptr(), st.asg.stride(0),
+        st.asg8.data_ptr(), st.asg8.stride(0), st.nb.data_ptr(), st.Sk.data_ptr(), st.Sk2.data_ptr(),
+        st.Sv.data_ptr(), st.reclist.data_ptr(), st.reccnt.data_ptr(), rmax, w.limbs.data_ptr(),
+        w.fexp.data_ptr(), w.H.data_ptr(), w.H.stride(0), w.TM.data_ptr(), w.TM.stride(0), w.TM.shape[1],
+        _ptr(w.TMn), w.S.data_ptr(), w.S.stride(0), sel.data_ptr(), sel.stride(0), w.score.data_ptr(),
+        w.n_t.data_ptr(), w.quota.data_ptr(), w.qsk.data_ptr(), w.exp_idx.data_ptr(), Ex, int(E), out.data_ptr(),
+        out.stride(0), int(out.dtype == torch.float32), n_dev.data_ptr(), ns, nl, k_top, sm_scale,
+        sm_scale * sm_scale, *rs)
+    lib.call("oa_step", a, _stream(dev))
+
+
 def waterfill(score, n_t, quota, E: int) -> None:
     dev = _dev(score, n_t, quota)
     R, C = score.shape

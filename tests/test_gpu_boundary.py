@@ -291,3 +291,40 @@ def test_custom_attention_full_mask_rows_are_dense():
 
 def att_state(meta):
     return meta["oa_hip"][0]["m"].st[0]
+
+
+@pytest.mark.parametrize("B,N,Q,rho", [(1, 700, 1, 0.01), (1, 4096, 2, 0.05), (2, 4101, 37, 0.01), (1, 2500, 64, 0.10),
+                                       (1, 40011, 5, 0.01), (3, 1999, 19, 0.03)])
+def test_question_rows_in_groups_equal_rows_one_by_one(B, N, Q, rho):
+    """rows_step with its rows in groups of a power of two (32 + 4 + 1 of 37, one launch per stage and
+    group, every row's statistics formed beside the index) against the rows run one after the other
+    with the keys taken back in place: selections, quotas, expanded sets and output bits, from a
+    transposed query view, with one and several groups, one and several top-q segments; the index is
+    left as it was."""
+    print(f"[case] grouped rows B={B} N={N} Q={Q} rho={rho}", flush=True)
+    from openattention_amd import synth
+    from openattention_amd.method import OursHIP
+    from openattention_amd.prefill import build_rows
+    K, V, _, qq, _ = synth.make_layer(7, B, N, N, 64, "cuda", n_question=max(Q, 8))
+    static = synth.static_metric(1)
+    got = {}
+    for mode in ("fused", "separate"):
+        m = OursHIP(types.SimpleNamespace(rho=rho), B, N, "cuda", n_layers=1, static=static, gate_mode=mode)
+        build_rows(m.st[0], K, V, qq, N, static["M"][0], static["inv_freq"], 1.0, 0)
+        q = qq[:, :, :Q].transpose(1, 2).contiguous().transpose(1, 2)
+        before = m.st[0].to_numpy()
+        n_dev = torch.zeros(1, device="cuda", dtype=torch.int32)
+        out = torch.empty(B, 32, Q, 128, device="cuda", dtype=torch.bfloat16)
+        rec = []
+        m.rows_step(m.st[0], K.view(-1, N, 128), V.view(-1, N, 128), q, n_dev, N, out, record=rec)
+        torch.cuda.synchronize()
+        after = m.st[0].to_numpy()
+        assert all(np.array_equal(before[f], after[f]) for f in before)
+        assert int(n_dev) == N
+        got[mode] = (out, sorted(rec, key=lambda t: t[0]))
+    (o1, r1), (o2, r2) = got["fused"], got["separate"]
+    assert [t[0] for t in r1] == [t[0] for t in r2] == list(range(Q))
+    for a, b in zip(r1, r2):
+        for x, y in zip(a[1:], b[1:]):
+            assert torch.equal(x, y), a[0]
+    assert torch.equal(o1, o2)
