@@ -183,3 +183,22 @@ def test_sym_eig_top_layouts_agree(batch):
         for i in range(batch):
             assert np.array_equal(ev2[i], ev[i % len(few)]) and np.array_equal(vec2[i], vec[i % len(few)])
             assert sw2[i] == sw[i % len(few)]
+
+
+@pytest.mark.parametrize("kv_rows,P_rows", [(64, 64), (65, 7), (129, 1), (257, 33)])
+def test_query_metric_slices_agree(kv_rows, P_rows):
+    """Eight, four, two and one workgroup per KV row form every sum in one order: a KV row's metrics
+    and group mean are the bits that a call with that KV row alone (eight slices) gives."""
+    print(f"[case] query metric slices kv_rows={kv_rows}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(kv_rows)
+    Qn = P_rows + 2
+    q = torch.randn(kv_rows * G, Qn, D, device=DEV, generator=g).to(torch.bfloat16)
+    pick = torch.arange(P_rows, device=DEV, dtype=torch.int32)
+    ang = torch.rand(P_rows, D, device=DEV, generator=g, dtype=torch.float64)
+    mst = torch.randn(32, D, D, device=DEV, generator=g)
+    gm, m = ops.query_metric(q, pick, ang.cos(), ang.sin(), 1.0, mst, G)
+    for kv in (0, 1, kv_rows // 2, kv_rows - 1):
+        first = kv * G % 32
+        heads = mst[torch.arange(first, first + G, device=DEV) % 32].contiguous()
+        g1, m1 = ops.query_metric(q[kv * G:(kv + 1) * G], pick, ang.cos(), ang.sin(), 1.0, heads, G)
+        assert torch.equal(gm[kv], g1[0]) and torch.equal(m[kv * G:(kv + 1) * G], m1)
