@@ -401,6 +401,17 @@ int oa_kmeans_assign(const uint16_t* zraw, const float* colmean, long z_stride, 
                      long asg8_stride, void* stream);
 
 /*
+ * A whole k-means iteration in two launches: oa_kmeans_assign's assignment, then oa_kmeans_update's
+ * centroids in cent (in place), with no member lists.  The fp64 sums are formed per workgroup (exact,
+ * so equal to the position-order sums, unless a column spans more than 2^14 times its mean).  asg and
+ * asg8 both NULL (not written) or both given.  ws: oa_kmeans_step_ws(rows, T, C) bytes, 8-byte aligned.
+ */
+long oa_kmeans_step_ws(int rows, int T, int C);
+int oa_kmeans_step(const uint16_t* zraw, const float* colmean, long z_stride, int rows, int T, float* cent,
+                   int C, const int32_t* init_idx, int32_t* asg, long asg_stride, uint8_t* asg8,
+                   long asg8_stride, void* ws, long ws_bytes, void* stream);
+
+/*
  * k-means update: centroid = mean of the members' zP rows (fp64 sum in position order, one
  * rounding), or zP[init_idx[c]] for an empty cluster; zP = zraw - colmean as in
  * oa_kmeans_assign; cnt_out (rows, C) member counts or NULL.  mem_ws (rows, mem_stride >= T),

@@ -355,15 +355,30 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16_tag(uint32_t tag, float b) {
 constexpr int kAsgThreads = 256;
 constexpr int kAsgMaxTiles = 8;                // tiles per wave where the grid is full without
 constexpr uint32_t kTag = 0x3f00u;             // low half of a ranked distance: kTag | 63 - (4 cb + i)
-template <int CB>
-__global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : 4) kmeans_assign_kernel(const uint16_t* zraw,
+//
+// ACC (a whole Lloyd iteration): each token's zP also joins its cluster's fp64 sum, in LDS per
+// workgroup, and the workgroup's sums and counts go to part / pcnt for kmeans_mean_kernel; asg and
+// asg8 may be null.  The fp64 sums of fp32 values within a factor 2^14 of colmean's magnitude are
+// exact (every zP is a whole multiple of colmean's last place, or half of it, and 2^15 of them fit 53
+// bits), so that no order shows in the centroids.  Before, the ids of every iteration were sorted into
+// member lists and each cluster's rows gathered again: 0.14 + 0.44 ms per iteration at 32 sequences.
+constexpr int kAccStride = kRC + 1;            // doubles per cluster in LDS (spread over the banks)
+template <int CB, bool ACC>
+__global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : CB <= 12 || !ACC ? 4 : 3) kmeans_assign_kernel(const uint16_t* zraw,
                                                                     const float* colmean, long zps, int T,
                                                                     const float* cent, int C,
                                                                     int32_t* asg, long as,
                                                                     uint8_t* asg8, long a8s,
-                                                                    int tiles_per_wave) {
+                                                                    int tiles_per_wave, double* part,
+                                                                    int32_t* pcnt) {
   __shared__ __align__(16) uint16_t s_cb[CB * 16 * kRC];
   __shared__ __align__(16) float s_half[CB * 16];
+  __shared__ double s_acc[ACC ? CB * 16 * kAccStride : 1];
+  __shared__ int s_cnt[ACC ? CB * 16 : 1];
+  if (ACC) {
+    for (int i = threadIdx.x; i < CB * 16 * kAccStride; i += kAsgThreads) s_acc[i] = 0.0;
+    for (int i = threadIdx.x; i < CB * 16; i += kAsgThreads) s_cnt[i] = 0;
+  }
   const int lane = threadIdx.x & 63, grp = lane >> 4;
   const int wave = threadIdx.x >> 6;
   const int row = blockIdx.y;
@@ -423,9 +438,9 @@ __global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : 4) kmeans_assign_ke
     int mine = 0;              // the ranked best of this lane's token of the tile (token lane)
 #pragma unroll 1
     for (int blk = 0; blk < 4; ++blk) {
-      const uint2 w = make_uint2(
-          cvt_pk_bf16(__uint_as_float(z[0].x << 16) - cm[0], __uint_as_float(z[0].x & 0xffff0000u) - cm[1]),
-          cvt_pk_bf16(__uint_as_float(z[0].y << 16) - cm[2], __uint_as_float(z[0].y & 0xffff0000u) - cm[3]));
+      const float zp[4] = {__uint_as_float(z[0].x << 16) - cm[0], __uint_as_float(z[0].x & 0xffff0000u) - cm[1],
+                           __uint_as_float(z[0].y << 16) - cm[2], __uint_as_float(z[0].y & 0xffff0000u) - cm[3]};
+      const uint2 w = make_uint2(cvt_pk_bf16(zp[0], zp[1]), cvt_pk_bf16(zp[2], zp[3]));
       const short4v tok = __builtin_bit_cast(short4v, w);
       z[0] = z[1]; z[1] = z[2]; z[2] = z[3];
       // the token's best: 0 as the bits stand (right where it is positive), 1 in the distances' order,
@@ -464,9 +479,17 @@ __global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : 4) kmeans_assign_ke
         positive = plain && __ballot(best <= 0 || best >= 0x7f800000) == 0ull;
       }
       mine = grp == blk ? best : mine;
+      if (ACC && tile * 64 + blk * 16 + (lane & 15) < T) {
+        const int cid = 255 - (best & 0xff);          // of token lane % 16, in every lane group
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          __hip_atomic_fetch_add(&s_acc[cid * kAccStride + 4 * grp + e], (double)zp[e], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (grp == 0) atomicAdd(&s_cnt[cid], 1);
+      }
     }
     const int t = tile * 64 + lane;
-    if (t < T) {
+    if (t < T && (!ACC || asg)) {
       const int cid = 255 - (mine & 0xff);
       asg[(long)row * as + t] = cid;
       asg8[(long)row * a8s + t] = (uint8_t)cid;
@@ -474,9 +497,49 @@ __global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : 4) kmeans_assign_ke
 #pragma unroll
     for (int blk = 0; blk < 4; ++blk) z[blk] = zn[blk];
   }
+  if (ACC) {
+    __syncthreads();
+    const long g = ((long)row * gridDim.x + blockIdx.x) * C;
+    for (int i = threadIdx.x; i < C * kRC; i += kAsgThreads)
+      part[g * kRC + i] = s_acc[(i / kRC) * kAccStride + i % kRC];
+    for (int i = threadIdx.x; i < C; i += kAsgThreads) pcnt[g + i] = s_cnt[i];
+  }
 }
 
-constexpr int kMemBuf = 2048;   // member positions staged in LDS at a time
+// The centroids from the workgroups' sums (added in workgroup order): one thread per value, its
+// partials 8 at a time in flight; an empty cluster keeps its initial point.
+__global__ void __launch_bounds__(256) kmeans_mean_kernel(const double* part, const int32_t* pcnt, int nwg, int C,
+                                                          const uint16_t* zraw, const float* colmean, long zps,
+                                                          const int32_t* init_idx, float* cent) {
+  const int row = blockIdx.y;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= C * kRC) return;
+  const int c = i / kRC, j = i % kRC;
+  const double* p = part + (long)row * nwg * C * kRC + i;
+  const int32_t* q = pcnt + (long)row * nwg * C + c;
+  double acc = 0.0;
+  int cnt = 0;
+  for (int g0 = 0; g0 < nwg; g0 += 8) {
+    double x[8];
+    int y[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int g = min(g0 + u, nwg - 1);
+      x[u] = p[(long)g * C * kRC];
+      y[u] = q[(long)g * C];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (g0 + u < nwg) {
+        acc += x[u];
+        cnt += y[u];
+      }
+  }
+  cent[(long)row * C * kRC + i] =
+      cnt > 0 ? (float)(acc / (double)cnt)
+              : oa::bf16_to_f32(zraw[(long)row * zps + (long)init_idx[c] * kRC + j]) - colmean[row * kRC + j];
+}
+
 
 // a wave copies 1 <= n <= (the LDS array's size) member positions into LDS, eight loads per lane
 // in flight at a time (one at a time, each copy waited on its load)
@@ -673,16 +736,26 @@ __global__ void __launch_bounds__(kSortThreads) csr_sort_kernel(int T, const uin
   }
 }
 
-// One wave per (cluster, query row): the fp64 sums of k, k*k and v over the members in position
-// order (mem, written by csr_sort_kernel; lane l: dims 2l, 2l + 1), the K and V words of 16
-// members requested together.
-__global__ void __launch_bounds__(64) cluster_sums_kernel(const uint16_t* K, const uint16_t* V, long ksh,
-                                                          long kst, int G, int C, const int32_t* cstart,
-                                                          const int32_t* clen, float* Sk, float* Sk2,
-                                                          float* Sv, const int32_t* mem, long ms,
-                                                          float* nb) {
-  __shared__ int s_pos[kMemBuf];
-  const int lane = threadIdx.x;
+// The fp64 sums of k, k*k and v of one (cluster, query row) by W waves: a lane holds 8 dims (16-byte
+// loads) of the members its 16-lane group takes, every (4 W)-th of the list, 4 at a time in flight;
+// the groups' sums are joined by two lane swaps and (W > 1) through LDS.  A group adds its members in
+// position order; sums of bf16 values, and of their squares, are exact in fp64 unless they span more
+// than 2^30 in magnitude, so how the list is split does not show in the fp32 results.
+// Bound by vector issue: 14 fp64 and conversion instructions per member and lane of 8 dims.  With a
+// lane on 2 dims (4-byte loads, a row address per member for every lane) 32 sequences of 32767 tokens
+// took 2215 us, and take 2086 us (by the counters 15 GB of the 17 GB gathered miss the L2s: waves of
+// clusters of different sizes drift apart in position); one such sequence (W = 4) 206 us, and takes 78
+// us.
+template <int W>
+__global__ void __launch_bounds__(64 * W) cluster_sums_kernel(const uint16_t* K, const uint16_t* V, long ksh,
+                                                              long kst, int G, int C, const int32_t* cstart,
+                                                              const int32_t* clen, float* Sk, float* Sk2,
+                                                              float* Sv, const int32_t* mem, long ms,
+                                                              float* nb) {
+  constexpr int kGroups = 4 * W, U = 4;
+  __shared__ double s_part[W > 1 ? W - 1 : 1][3][kD];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int grp = threadIdx.x >> 4, d0 = 8 * (lane & 15);
   // every token's K and V rows are read once per query row of its KV row (each query row has its
   // own clusters).  The G * C workgroups of a KV row run on one XCD, its query rows interleaved,
   // so that they walk the KV row's positions together and the later reads of a row hit that
@@ -700,42 +773,80 @@ __global__ void __launch_bounds__(64) cluster_sums_kernel(const uint16_t* K, con
       c = b % C;
     }
   }
-  const uint16_t* kr = K + (long)(row / G) * ksh + 2 * lane;
-  const uint16_t* vr = V + (long)(row / G) * ksh + 2 * lane;
+  const uint16_t* kr = K + (long)(row / G) * ksh + d0;
+  const uint16_t* vr = V + (long)(row / G) * ksh + d0;
   const int32_t* ml = mem + (long)row * ms + cstart[row * C + c];
   const int cl = clen[row * C + c];
-  if (nb && lane == 0) nb[row * C + c] = (float)cl;   // (when the sort did not write it)
-  double k0 = 0.0, k1 = 0.0, q0 = 0.0, q1 = 0.0, v0 = 0.0, v1 = 0.0;
-  constexpr int U = 16;
-  for (int i0 = 0; i0 < cl; i0 += kMemBuf) {
-    const int n = min(kMemBuf, cl - i0);
-    stage_members(s_pos, ml + i0, n, lane);
-    __syncthreads();
-    for (int k = 0; k < n; k += U) {
-      uint32_t kw[U], vw[U];
+  if (nb && threadIdx.x == 0) nb[row * C + c] = (float)cl;   // (when the sort did not write it)
+  double ks[8], qs[8], vs[8];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const long off = (long)s_pos[min(k + u, n - 1)] * kst;
-        kw[u] = *reinterpret_cast<const uint32_t*>(kr + off);
-        vw[u] = *reinterpret_cast<const uint32_t*>(vr + off);
-      }
+  for (int e = 0; e < 8; ++e) ks[e] = qs[e] = vs[e] = 0.0;
+  // this group's members grp, grp + kGroups, ...: U positions requested a batch ahead of their rows
+  int pos[U];
+  auto next = [&](int m0) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (k + u < n) {
-          const double a0 = (double)__uint_as_float(kw[u] << 16);
-          const double a1 = (double)__uint_as_float(kw[u] & 0xffff0000u);
-          k0 += a0; k1 += a1; q0 += a0 * a0; q1 += a1 * a1;
-          v0 += (double)__uint_as_float(vw[u] << 16);
-          v1 += (double)__uint_as_float(vw[u] & 0xffff0000u);
+    for (int u = 0; u < U; ++u) pos[u] = ml[min(m0 + u * kGroups, cl - 1)];
+  };
+  if (cl > 0) next(grp);
+  for (int m0 = grp; m0 < cl; m0 += U * kGroups) {
+    uint4 kw[U], vw[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long off = (long)pos[u] * kst;
+      kw[u] = *reinterpret_cast<const uint4*>(kr + off);
+      vw[u] = *reinterpret_cast<const uint4*>(vr + off);
+    }
+    next(m0 + U * kGroups);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (m0 + u * kGroups < cl) {
+        float k[8], v[8];
+        oa::unpack8(kw[u], k);
+        oa::unpack8(vw[u], v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const double x = (double)k[e];
+          ks[e] += x;
+          qs[e] = fma(x, x, qs[e]);                // (the square of a bf16 value is exact)
+          vs[e] += (double)v[e];
         }
       }
     }
-    __syncthreads();
   }
-  const long o = ((long)row * C + c) * kD + 2 * lane;
-  Sk[o] = (float)k0; Sk[o + 1] = (float)k1;
-  Sk2[o] = (float)q0; Sk2[o + 1] = (float)q1;
-  Sv[o] = (float)v0; Sv[o + 1] = (float)v1;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    ks[e] = oa::swap32_sum(oa::swap16_sum(ks[e]));
+    qs[e] = oa::swap32_sum(oa::swap16_sum(qs[e]));
+    vs[e] = oa::swap32_sum(oa::swap16_sum(vs[e]));
+  }
+  if (W > 1) {
+    if (wave > 0 && lane < 16) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        s_part[wave - 1][0][d0 + e] = ks[e];
+        s_part[wave - 1][1][d0 + e] = qs[e];
+        s_part[wave - 1][2][d0 + e] = vs[e];
+      }
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 0; w < W - 1; ++w)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        ks[e] += s_part[w][0][d0 + e];
+        qs[e] += s_part[w][1][d0 + e];
+        vs[e] += s_part[w][2][d0 + e];
+      }
+  }
+  // lane group 0 writes Sk, 1 Sk2, 2 Sv (every group holds all three)
+  if (lane >= 48) return;
+  float* out = (lane < 16 ? Sk : lane < 32 ? Sk2 : Sv) + ((long)row * C + c) * kD + d0;
+  float o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = (float)(lane < 16 ? ks[e] : lane < 32 ? qs[e] : vs[e]);
+  *reinterpret_cast<float4*>(out) = make_float4(o[0], o[1], o[2], o[3]);
+  *reinterpret_cast<float4*>(out + 4) = make_float4(o[4], o[5], o[6], o[7]);
 }
 
 }  // namespace
@@ -787,6 +898,33 @@ extern "C" int oa_qgc_project(const void* K, long k_stride_h, long k_stride_t, i
   return OA_LAUNCH_STATUS();
 }
 
+// tiles per wave: up to eight spread the centroids' staging; fewer where the grid would not give
+// every SIMD eight waves
+static int asg_tiles_per_wave(int rows, int T) {
+  const long ntiles = (T + 63) / 64;
+  return (int)std::min<long>(kAsgMaxTiles, std::max<long>(1, ntiles * rows / 8192));
+}
+
+template <bool ACC>
+static void launch_assign(const uint16_t* zraw, const float* colmean, long z_stride, int rows, int T,
+                          const float* cent, int C, int32_t* asg, long asg_stride, uint8_t* asg8,
+                          long asg8_stride, int tpw, double* part, int32_t* pcnt, hipStream_t stream) {
+  const int ntiles = (T + 63) / 64, per = kAsgThreads / 64 * tpw;
+  const dim3 grid((ntiles + per - 1) / per, rows), block(kAsgThreads);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, zraw, colmean, z_stride, T, cent, C, asg, asg_stride, asg8,
+                       asg8_stride, tpw, part, pcnt);
+  };
+  // the centroid blocks a wave holds: the least of these that covers C (padding ranks below)
+  const int cb = (C + 15) / 16;
+  if (cb <= 1) launch(kmeans_assign_kernel<1, ACC>);
+  else if (cb <= 2) launch(kmeans_assign_kernel<2, ACC>);
+  else if (cb <= 4) launch(kmeans_assign_kernel<4, ACC>);
+  else if (cb <= 8) launch(kmeans_assign_kernel<8, ACC>);
+  else if (cb <= 12) launch(kmeans_assign_kernel<12, ACC>);
+  else launch(kmeans_assign_kernel<16, ACC>);
+}
+
 extern "C" int oa_kmeans_assign(const uint16_t* zraw, const float* colmean, long z_stride, int rows,
                                 int T, const float* cent, int C, int32_t* asg, long asg_stride,
                                 uint8_t* asg8, long asg8_stride, void* stream) {
@@ -794,23 +932,39 @@ extern "C" int oa_kmeans_assign(const uint16_t* zraw, const float* colmean, long
       z_stride < (long)T * kRC || z_stride % 4 || asg_stride < T || asg8_stride < T ||
       (reinterpret_cast<uintptr_t>(zraw) & 7))
     return OA_EINVAL;
-  // eight tiles per wave spread the centroids' staging; fewer where the grid would not give every
-  // SIMD eight waves
-  const int ntiles = (T + 63) / 64, waves = kAsgThreads / 64;
-  const int tpw = (int)std::min<long>(kAsgMaxTiles, std::max<long>(1, (long)ntiles * rows / 8192));
-  const dim3 grid((ntiles + waves * tpw - 1) / (waves * tpw), rows), block(kAsgThreads);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, zraw, colmean, z_stride, T, cent, C, asg,
-                       asg_stride, asg8, asg8_stride, tpw);
-  };
-  // the centroid blocks a wave holds: the least of these that covers C (padding ranks below)
-  const int cb = (C + 15) / 16;
-  if (cb <= 1) launch(kmeans_assign_kernel<1>);
-  else if (cb <= 2) launch(kmeans_assign_kernel<2>);
-  else if (cb <= 4) launch(kmeans_assign_kernel<4>);
-  else if (cb <= 8) launch(kmeans_assign_kernel<8>);
-  else if (cb <= 12) launch(kmeans_assign_kernel<12>);
-  else launch(kmeans_assign_kernel<16>);
+  const int tpw = asg_tiles_per_wave(rows, T);
+  launch_assign<false>(zraw, colmean, z_stride, rows, T, cent, C, asg, asg_stride, asg8, asg8_stride, tpw, nullptr,
+                       nullptr, (hipStream_t)stream);
+  return OA_LAUNCH_STATUS();
+}
+
+// a whole Lloyd iteration: part_ws holds a workgroup's sums and counts for each of the grid's
+static int step_groups(int rows, int T) {
+  const int waves = kAsgThreads / 64, tpw = asg_tiles_per_wave(rows, T);
+  return ((T + 63) / 64 + waves * tpw - 1) / (waves * tpw);
+}
+
+extern "C" long oa_kmeans_step_ws(int rows, int T, int C) {
+  if (rows <= 0 || T <= 0 || C <= 0 || C > kMaxC) return OA_EINVAL;
+  return (long)rows * step_groups(rows, T) * C * (kRC * 8 + 4);
+}
+
+extern "C" int oa_kmeans_step(const uint16_t* zraw, const float* colmean, long z_stride, int rows, int T,
+                              float* cent, int C, const int32_t* init_idx, int32_t* asg, long asg_stride,
+                              uint8_t* asg8, long asg8_stride, void* ws, long ws_bytes, void* stream) {
+  if (rows <= 0 || T <= 0 || C <= 0 || C > kMaxC || !zraw || !colmean || !cent || !init_idx || !ws ||
+      z_stride < (long)T * kRC || z_stride % 4 || (!asg != !asg8) || (asg && (asg_stride < T || asg8_stride < T)) ||
+      (reinterpret_cast<uintptr_t>(zraw) & 7) || (reinterpret_cast<uintptr_t>(ws) & 7) ||
+      ws_bytes < oa_kmeans_step_ws(rows, T, C))
+    return OA_EINVAL;
+  const int nwg = step_groups(rows, T);
+  double* part = static_cast<double*>(ws);
+  int32_t* pcnt = reinterpret_cast<int32_t*>(part + (long)rows * nwg * C * kRC);
+  hipStream_t s = (hipStream_t)stream;
+  launch_assign<true>(zraw, colmean, z_stride, rows, T, cent, C, asg, asg_stride, asg8, asg8_stride,
+                      asg_tiles_per_wave(rows, T), part, pcnt, s);
+  hipLaunchKernelGGL(kmeans_mean_kernel, dim3((C * kRC + 255) / 256, rows), dim3(256), 0, s, part, pcnt, nwg, C,
+                     zraw, colmean, z_stride, init_idx, cent);
   return OA_LAUNCH_STATUS();
 }
 
@@ -837,6 +991,20 @@ extern "C" int oa_kmeans_update(const uint16_t* zraw, const float* colmean, long
   return OA_LAUNCH_STATUS();
 }
 
+// one wave per (cluster, row) where those fill the chip (16384 are four waves per SIMD), else four
+static void launch_sums(const void* K, const void* V, long ksh, long kst, int rows, int G, int C,
+                        const int32_t* cstart, const int32_t* clen, float* Sk, float* Sk2, float* Sv,
+                        const int32_t* mem, long ms, float* nb, hipStream_t s) {
+  const uint16_t* k = reinterpret_cast<const uint16_t*>(K);
+  const uint16_t* v = reinterpret_cast<const uint16_t*>(V);
+  if ((long)rows * C >= 16384)
+    hipLaunchKernelGGL(cluster_sums_kernel<1>, dim3(C * rows), dim3(64), 0, s, k, v, ksh, kst, G, C, cstart,
+                       clen, Sk, Sk2, Sv, mem, ms, nb);
+  else
+    hipLaunchKernelGGL(cluster_sums_kernel<4>, dim3(C * rows), dim3(256), 0, s, k, v, ksh, kst, G, C, cstart,
+                       clen, Sk, Sk2, Sv, mem, ms, nb);
+}
+
 extern "C" int oa_cluster_build(const void* K, const void* V, long kv_stride_h, long kv_stride_t, int rows,
                                 int G, int T, const uint8_t* asg8, long asg8_stride, int C, float* nb,
                                 float* Sk, float* Sk2, float* Sv, int32_t* mem, long mem_stride,
@@ -849,10 +1017,7 @@ extern "C" int oa_cluster_build(const void* K, const void* V, long kv_stride_h, 
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(csr_sort_kernel, dim3(rows), dim3(kSortThreads), 0, s, T, asg8, asg8_stride, C, nb,
                      cstart, clen, mem, mem_stride, sort_staged(T, asg8, asg8_stride));
-  hipLaunchKernelGGL(cluster_sums_kernel, dim3(C * rows), dim3(64), 0, s,
-                     reinterpret_cast<const uint16_t*>(K), reinterpret_cast<const uint16_t*>(V),
-                     kv_stride_h, kv_stride_t, G, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride,
-                     static_cast<float*>(nullptr));
+  launch_sums(K, V, kv_stride_h, kv_stride_t, rows, G, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride, nullptr, s);
   return OA_LAUNCH_STATUS();
 }
 
@@ -865,8 +1030,7 @@ extern "C" int oa_cluster_sums(const void* K, const void* V, long kv_stride_h, l
       kv_stride_h % 2 || mem_stride < T || (reinterpret_cast<uintptr_t>(K) & 3) ||
       (reinterpret_cast<uintptr_t>(V) & 3))
     return OA_EINVAL;
-  hipLaunchKernelGGL(cluster_sums_kernel, dim3(C * rows), dim3(64), 0, (hipStream_t)stream,
-                     reinterpret_cast<const uint16_t*>(K), reinterpret_cast<const uint16_t*>(V),
-                     kv_stride_h, kv_stride_t, G, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride, nb);
+  launch_sums(K, V, kv_stride_h, kv_stride_t, rows, G, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride, nb,
+              (hipStream_t)stream);
   return OA_LAUNCH_STATUS();
 }

@@ -6,8 +6,8 @@
 // the keys n_keys - 1, ..., n + i taken back, in that order (index_downdate's fp32 terms).
 // rows_stats_kernel writes every row's statistics at once, and the 2^qsh rows of every sequence then
 // run through each stage as one launch.  One row of one sequence holds 32 of the 256 compute units
-// for a chain of five launches; 64 of them one after the other took 64 x 78 us of device time; in two launches of
-// 32 rows each a stage takes 0.4 ms for all 64.
+// for a chain of five launches: 64 of them one after the other took 64 x 78 us of device time, and take
+// 0.4 ms in two groups of 32.
 #include "oa_common.h"
 #include "oa_rows.h"
 

@@ -69,6 +69,8 @@ SIGNATURES = {
     "oa_qgs_codes": [P, L, L, I, I, P, P, L, P, P, P, P],
     "oa_qgc_project": [P, L, L, I, I, I, P, P, L, P, P, P, P],
     "oa_kmeans_assign": [P, P, L, I, I, P, I, P, L, P, L, P],
+    "oa_kmeans_step_ws": [I, I, I],
+    "oa_kmeans_step": [P, P, L, I, I, P, I, P, P, L, P, L, P, L, P],
     "oa_kmeans_update": [P, P, L, I, I, P, L, I, P, P, P, P, L, P, P, P],
     "oa_cluster_build": [P, P, L, L, I, I, I, P, L, I, P, P, P, P, P, L, P, P, P],
     "oa_cluster_sums": [P, P, L, L, I, I, I, I, P, P, P, P, P, L, P, P, P],
@@ -102,7 +104,7 @@ def load() -> ct.CDLL:
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.argtypes = argtypes
-        fn.restype = ct.c_char_p if name == "oa_error_string" else ct.c_int
+        fn.restype = {"oa_error_string": ct.c_char_p, "oa_kmeans_step_ws": ct.c_long}.get(name, ct.c_int)
     _LIB = lib
     return lib
 

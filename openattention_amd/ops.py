@@ -706,6 +706,30 @@ def kmeans_assign(zraw, colmean, T: int, cent, asg, asg8) -> None:
              asg.stride(0), _ptr(asg8), asg8.stride(0), _stream(dev))
 
 
+def kmeans_step(zraw, colmean, T: int, init, cent, asg=None, asg8=None, ws=None) -> torch.Tensor:
+    """kmeans_assign then kmeans_update's centroids (cent in place) without member lists; asg and asg8
+    both None (not written) or both given.  ws: a byte workspace of a former call with the same sizes,
+    or None; returns the workspace used."""
+    dev = _dev(zraw, colmean, cent, init, asg, asg8)
+    HQ, C = cent.shape[0], cent.shape[1]
+    _zraw(zraw, HQ, T)
+    _need(colmean.is_contiguous() and colmean.shape == (HQ, RANK_C), "colmean: (HQ, 16) contiguous")
+    _need(cent.is_contiguous() and cent.shape[2] == RANK_C, "cent: (HQ, C, 16) contiguous")
+    _need(init.dtype == torch.int32 and init.numel() == C and init.is_contiguous(), "init: (C,) int32")
+    _need((asg is None) == (asg8 is None), "asg and asg8 are given together")
+    if asg is not None:
+        _chk(asg, "asg", torch.int32, (HQ, -T))
+        _chk(asg8, "asg8", torch.uint8, (HQ, -T))
+    need = lib.load().oa_kmeans_step_ws(HQ, T, C)
+    _need(need > 0, "kmeans_step: rows, T and C must be positive, C at most 256")
+    if ws is None or ws.numel() < need:
+        ws = torch.empty(need, device=dev, dtype=torch.uint8)
+    lib.call("oa_kmeans_step", _ptr(zraw), _ptr(colmean), zraw.stride(0), HQ, T, _ptr(cent), C, _ptr(init),
+             _ptr(asg), 0 if asg is None else asg.stride(0), _ptr(asg8), 0 if asg8 is None else asg8.stride(0),
+             _ptr(ws), ws.numel(), _stream(dev))
+    return ws
+
+
 def kmeans_update(zraw, colmean, T: int, asg8, init, cent, mem, cstart, clen, cnt=None) -> None:
     """a12 update of cent (HQ, C, 16) in place; init (C,) int32 initial positions; zP as in
     kmeans_assign; mem (HQ, >=T), cstart, clen (HQ, C) int32 receive the assignment's member lists."""

@@ -366,16 +366,16 @@ def _build_device(st, r0: int, K: torch.Tensor, V: torch.Tensor, T: int, layer: 
     cent.copy_(zraw.index_select(1, init.long()).float() - colmean[:, None, :])
     asg, asg8 = st.asg[q0:q0 + HQ], st.asg8[q0:q0 + HQ]
     mark("kmeans_init")
-    for _ in range(ITERS):
-        ops.kmeans_assign(zraw, colmean, T, cent, asg, asg8)
-        mark("kmeans_assign")
-        ops.kmeans_update(zraw, colmean, T, asg8, init, cent, st.mem[q0:q0 + HQ], st.cstart[q0:q0 + HQ],
-                          st.clen[q0:q0 + HQ])
-        mark("kmeans_update")
-    # a13: cluster statistics; the CSR member lists are the last update's (the assignment did not
-    # change after it), so they are not sorted again
-    ops.cluster_sums(K, V, T, G, C, st.nb[q0:q0 + HQ], st.Sk[q0:q0 + HQ], st.Sk2[q0:q0 + HQ],
-                     st.Sv[q0:q0 + HQ], st.mem[q0:q0 + HQ], st.cstart[q0:q0 + HQ], st.clen[q0:q0 + HQ])
+    # a Lloyd iteration is one call; the assignment itself is only needed from the last
+    ws = None
+    for it in range(ITERS):
+        last = it == ITERS - 1
+        ws = ops.kmeans_step(zraw, colmean, T, init, cent, asg if last else None, asg8 if last else None, ws)
+        mark("kmeans")
+    del ws
+    # a13: the CSR member lists of that assignment and the cluster statistics
+    ops.cluster_build(K, V, T, G, asg8, C, st.nb[q0:q0 + HQ], st.Sk[q0:q0 + HQ], st.Sk2[q0:q0 + HQ],
+                      st.Sv[q0:q0 + HQ], st.mem[q0:q0 + HQ], st.cstart[q0:q0 + HQ], st.clen[q0:q0 + HQ])
     st.reccnt[q0:q0 + HQ] = 0
     mark("cluster_build")
 

@@ -1321,3 +1321,64 @@ def test_kmeans_assign_edges_exact(C, T):
     assert got[4, T - 1] == 0 and 0 <= got[4, 0] < C
     assert (got[:, T:] == -1).all() and (asg8.cpu().numpy()[:, T:] == 255).all()
     assert np.array_equal(asg8.cpu().numpy()[:, :T], got[:, :T].astype(np.uint8))
+
+
+@pytest.mark.parametrize("R,T,C", [(1, 1, 1), (3, 63, 5), (8, 65, 16), (8, 700, 17), (64, 4097, 64), (40, 10007, 100),
+                                   (8, 2050, 129), (8, 1500, 200), (64, 3000, 256)])
+def test_kmeans_step_equals_assign_then_update(R, T, C):
+    """A Lloyd iteration in one call against the assignment and the member-list update: the same ids
+    and the same centroid bits (the fp64 sums are exact, so their order does not show), with empty
+    clusters, ragged tiles, one and several workgroups per row and one tile or more per wave; without
+    asg the ids are not written and the centroids are the same."""
+    print(f"[case] k-means step R={R} T={T} C={C}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(R * 7919 + T * 31 + C)
+    zraw = torch.randn(R, T, 16, device=DEV, generator=g).to(torch.bfloat16)
+    cm = 0.1 * torch.randn(R, 16, device=DEV, generator=g)
+    init = torch.randint(0, T, (C,), device=DEV, generator=g, dtype=torch.int32)
+    cent0 = (zraw.index_select(1, init.long()).float() - cm[:, None]).contiguous()
+    if C > 2:
+        cent0[:, 1] = 40.0                                 # nothing joins it: it returns to its point
+    asg = torch.full((R, T), -1, device=DEV, dtype=torch.int32)
+    asg8 = torch.zeros(R, -(-T // 64) * 64, device=DEV, dtype=torch.uint8)
+    ref = cent0.clone()
+    ops.kmeans_assign(zraw, cm, T, ref, asg, asg8)
+    mem = torch.empty(R, T, device=DEV, dtype=torch.int32)
+    cs, cl = (torch.empty(R, C, device=DEV, dtype=torch.int32) for _ in range(2))
+    ops.kmeans_update(zraw, cm, T, asg8, init, ref, mem, cs, cl)
+    a2, a8 = torch.full_like(asg, -1), torch.zeros_like(asg8)
+    one, two = cent0.clone(), cent0.clone()
+    ws = ops.kmeans_step(zraw, cm, T, init, one, a2, a8)
+    ops.kmeans_step(zraw, cm, T, init, two, ws=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(a2, asg) and torch.equal(a8, asg8)
+    assert torch.equal(one, ref) and torch.equal(two, ref)
+
+
+@pytest.mark.parametrize("HKV_,T,C", [(8, 3000, 64), (64, 300, 64), (65, 700, 70)])
+def test_cluster_sums_layouts_bit_exact(HKV_, T, C):
+    """Cluster statistics with four waves per (cluster, row) and with one (16384 pairs and more), over
+    uneven clusters, an empty one, and K, V rows that start 4 bytes off a 16-byte boundary."""
+    print(f"[case] cluster sums layouts HKV={HKV_} T={T} C={C}", flush=True)
+    rng = np.random.default_rng(HKV_ + T)
+    R = HKV_ * 4
+    pad = torch.from_numpy(rng.standard_normal((2, HKV_, T, D + 2)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    K, V = pad[0, :, :, 2:], pad[1, :, :, 2:]
+    asg = np.minimum((C * rng.random((R, T)) ** 2).astype(np.int64), C - 1)
+    asg[:, asg[0] == 3] = 4
+    asg[asg == 3] = 4
+    asg8 = torch.zeros(R, -(-T // 64) * 64, device=DEV, dtype=torch.uint8)
+    asg8[:, :T] = torch.from_numpy(asg.astype(np.uint8)).to(DEV)
+    nb = torch.empty(R, C, device=DEV)
+    Sk, Sk2, Sv = (torch.full((R, C, D), 7.0, device=DEV) for _ in range(3))
+    mem = torch.empty(R, T, device=DEV, dtype=torch.int32)
+    cs, cl = (torch.empty(R, C, device=DEV, dtype=torch.int32) for _ in range(2))
+    ops.cluster_build(K, V, T, 4, asg8, C, nb, Sk, Sk2, Sv, mem, cs, cl)
+    torch.cuda.synchronize()
+    for h in {0, HKV_ - 1}:
+        k, v = K[h].float().cpu().double().numpy(), V[h].float().cpu().double().numpy()
+        for r in range(4 * h, 4 * h + 4):
+            for c in range(C):
+                m = asg[r] == c
+                assert int(nb[r, c]) == m.sum()
+                for got, x in ((Sk, k), (Sk2, k * k), (Sv, v)):
+                    assert np.array_equal(got[r, c].cpu().numpy(), x[m].sum(0).astype(np.float32)), (r, c)
