@@ -477,6 +477,18 @@ int oa_sym_eig_top(const float* M, long m_stride, int batch, int n, int k, float
                    float* evecs, int* sweeps, void* stream);
 
 /*
+ * Dense causal attention of one sequence's prompt: out[h][t] = softmax over j <= t of
+ * (sm_scale q[h][t] . k[h/4][j]) weighting v[h/4][j], bf16 rows with fp32 scores, softmax and sums and
+ * bf16 weights.  Strides per head and per position in elements (q, k, v: multiples of 8 with 16-byte
+ * aligned bases; out: multiples of 4, 8-byte aligned); heads = 4 kv_heads.  Replaces the dense prefill
+ * branch of the hook (inference/graph_runner.py:472-475).
+ */
+int oa_prefill_attn(const void* q, long q_stride_h, long q_stride_t, const void* k, long k_stride_h,
+                    long k_stride_t, const void* v, long v_stride_h, long v_stride_t, int heads,
+                    int kv_heads, int T, int head_dim, float sm_scale, void* out, long out_stride_h,
+                    long out_stride_t, void* stream);
+
+/*
  * One decode step, or one group of question rows, in one call: oa_index_prep (update = 1) or
  * oa_qgs_prep (update = 0), then oa_qgs_scan_heads, oa_topk_gate_fill, oa_topq_heads and
  * oa_residual_flash with these arguments, launched in order on the stream; the same outputs as those

@@ -76,6 +76,7 @@ SIGNATURES = {
     "oa_cluster_sums": [P, P, L, L, I, I, I, I, P, P, P, P, P, L, P, P, P],
     "oa_query_metric": [P, I, L, L, I, I, P, I, P, P, Dd, P, I, P, P, P],
     "oa_sym_eig_top": [P, L, I, I, I, P, P, P, P],
+    "oa_prefill_attn": [P, L, L, P, L, L, P, L, L, I, I, I, I, F, P, L, L, P],
     "oa_step": [ct.POINTER(StepArgs), P],
 }
 

@@ -53,12 +53,15 @@ def prefill_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tenso
     """Dense causal attention of the prefill rows of one sequence, as the deployed hook's prefill
     branch computes it (graph_runner.py:472-475): query (1, HQ, Q, D) at positions K - Q .. K - 1
     of key, value (1, HKV, K, D); returns (1, HQ, Q, D) in query's dtype.  GQA groups are
-    expanded.  When Q == K the fused flash / memory-efficient kernels run on the cache's dtype;
-    otherwise (or where those kernels are unavailable) blocks of query rows run in fp32, so the
-    score matrix never exceeds (HQ, block, K)."""
+    expanded.  When Q == K this library's matrix-core kernel takes bf16 rows of its head layout
+    (ops.prefill_attn_ok) and the fused flash / memory-efficient kernels the others; otherwise (or
+    where those kernels are unavailable) blocks of query rows run in fp32, so the score matrix never
+    exceeds (HQ, block, K)."""
     Gq = query.shape[1] // key.shape[1]
     Q, K = query.shape[2], key.shape[2]
     if Q == K:
+        if ops.prefill_attn_ok(query, key, value, scale):
+            return ops.prefill_attn(query, key, value, scale)
         from torch.nn.attention import SDPBackend, sdpa_kernel
         try:
             with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):

@@ -594,6 +594,41 @@ def dense_decode(q, K, V, n_dev, out=None, sm_scale: float | None = None, nsplit
     return out
 
 
+def prefill_attn_ok(q, k, v, sm_scale: float = 1.0) -> bool:
+    """Whether prefill_attn takes these arguments: a scale that is not negative (the running maximum is
+    taken before it is applied), plain bf16 HIP tensors of Llama-3.1-8B's head layout,
+    one sequence, rows of dims contiguous, 16-byte aligned, and nothing that would have to see the
+    operation (autograd in either mode, a functional transform, a tracer)."""
+    if (not sm_scale >= 0 or q.dim() != 4 or k.dim() != 4 or q.shape[0] != 1 or k.shape[0] != 1 or k.shape != v.shape
+            or q.shape[3] != HEAD_DIM or k.shape[3] != HEAD_DIM or q.shape[1] != GROUP * k.shape[1]
+            or q.shape[2] != k.shape[2] or q.shape[2] < 1):
+        return False
+    for t in (q, k, v):
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != torch.bfloat16
+                or t.device.type != "cuda" or t.device != q.device or t.stride(3) != 1
+                or t.stride(1) % 8 or t.stride(2) % 8 or t.stride(2) < HEAD_DIM or t.stride(2) > 1 << 24
+                or torch._C._functorch.is_functorch_wrapped_tensor(t) or t.data_ptr() % 16):
+            return False
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        return False
+    return torch.autograd.forward_ad._current_level < 0 and not torch.compiler.is_compiling()
+
+
+def prefill_attn(q, k, v, sm_scale: float) -> torch.Tensor:
+    """Dense causal attention of one prompt (oa_prefill_attn): q (1, HQ, T, 128), k, v (1, HKV, T, 128)
+    bf16, any head and position strides that prefill_attn_ok admits -> (1, HQ, T, 128), a view of
+    position-major rows."""
+    dev = _dev(q, k, v)
+    _need(prefill_attn_ok(q, k, v, sm_scale), "q, k, v: one sequence of bf16 rows of 128 aligned dims, "
+          "HQ = 4 HKV, a scale >= 0")
+    _, HQ, T, _ = q.shape
+    out = torch.empty(1, T, HQ, HEAD_DIM, device=dev, dtype=torch.bfloat16)
+    lib.call("oa_prefill_attn", _ptr(q), q.stride(1), q.stride(2), _ptr(k), k.stride(1), k.stride(2), _ptr(v),
+             v.stride(1), v.stride(2), HQ, k.shape[1], T, HEAD_DIM, float(sm_scale), _ptr(out), out.stride(2),
+             out.stride(1), _stream(dev))
+    return out.transpose(1, 2)
+
+
 # ================================================================== prefill index build
 def qgs_codes(K, T: int, U, codes, scale, amax_ws, zc_ws=None) -> None:
     """a11 of one request: K (HKV, >=T, 128) bf16; U (HKV, 128, 32) fp32; codes (HKV, Lmax, 32)

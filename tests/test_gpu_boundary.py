@@ -328,3 +328,73 @@ def test_question_rows_in_groups_equal_rows_one_by_one(B, N, Q, rho):
         for x, y in zip(a[1:], b[1:]):
             assert torch.equal(x, y), a[0]
     assert torch.equal(o1, o2)
+
+
+@pytest.mark.parametrize("T,heads,layout", [(1, 32, "head"), (31, 32, "token"), (32, 8, "head"), (33, 4, "token"),
+                                            (64, 32, "token"), (65, 8, "head"), (97, 8, "token"), (700, 32, "token"),
+                                            (1027, 4, "head")])
+def test_prefill_attn_against_fp64(T, heads, layout):
+    """The matrix-core prefill attention against fp64 softmax attention: tile edges, one to 33 tiles
+    (odd and even), head-major and position-major rows, scores that raise the running maximum late (a
+    scale that makes the last keys by far the largest) and a scale of 0.  bf16 output rounds to 2^-9
+    relative and the weights of a row to 2^-9 each, so a row is within 2^-8 of its largest terms:
+    1e-2 of the row's norm, and 6e-3 over all rows."""
+    print(f"[case] prefill attention T={T} heads={heads} {layout}", flush=True)
+    from openattention_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(T)
+    kv = heads // 4
+
+    def rows(h):
+        x = torch.randn(1, T, h, 128, device="cuda", generator=g).to(torch.bfloat16)
+        return x.transpose(1, 2) if layout == "token" else x.transpose(1, 2).contiguous()
+
+    q, k, v = rows(heads), rows(kv), rows(kv)
+    for scale, late in ((128 ** -0.5, False), (0.5, True), (0.0, False)):
+        kk = k.clone() if layout == "head" else k.transpose(1, 2).clone().transpose(1, 2)
+        if late:
+            kk = kk * torch.linspace(0.01, 3.0, T, device="cuda", dtype=torch.bfloat16)[None, None, :, None]
+            kk = kk if layout == "head" else kk.transpose(1, 2).contiguous().transpose(1, 2)
+        assert ops.prefill_attn_ok(q, kk, v)
+        o = ops.prefill_attn(q, kk, v, scale)
+        torch.cuda.synchronize()
+        z = q[0].double() @ kk[0].repeat_interleave(4, 0).double().transpose(1, 2).contiguous() * scale
+        z.masked_fill_(torch.ones(T, T, device="cuda", dtype=torch.bool).triu(1), float("-inf"))
+        ref = torch.softmax(z, -1) @ v[0].repeat_interleave(4, 0).double()
+        err = (o[0].double() - ref).norm(dim=-1) / ref.norm(dim=-1)
+        rel = ((o[0].double() - ref).norm() / ref.norm()).item()
+        print(f"  scale {scale:.3f}: rel {rel:.2e}, worst row {err.max().item():.2e}")
+        assert o.shape == q.shape and rel < 6e-3 and err.max() < 1e-2
+
+
+def test_prefill_attention_keeps_the_general_path():
+    """What the matrix-core kernel does not take still runs as before: gradients, forward-mode tangents,
+    vmap, other dtypes, rows off 16 bytes, several query heads per KV head other than four."""
+    from torch.autograd import forward_ad
+    from openattention_amd import ops
+    from openattention_amd.method import prefill_attention
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(1, h, 48, 128, device="cuda", generator=g).to(torch.bfloat16) for h in (8, 2, 2))
+    assert ops.prefill_attn_ok(q, k, v)
+    base = prefill_attention(q, k, v, 0.1).float()
+    qr = q.clone().requires_grad_(True)
+    assert not ops.prefill_attn_ok(qr, k, v)
+    prefill_attention(qr, k, v, 0.1).float().sum().backward()
+    assert qr.grad is not None and qr.grad.abs().sum() > 0
+    with torch.no_grad():
+        assert ops.prefill_attn_ok(qr, k, v)
+    with forward_ad.dual_level():
+        assert not ops.prefill_attn_ok(q, k, v)
+    assert not ops.prefill_attn_ok(q, k, v, -0.1) and not ops.prefill_attn_ok(q, k, v, float("nan"))
+    z = -0.1 * (q[0].double() @ k[0].repeat_interleave(4, 0).double().transpose(1, 2).contiguous())
+    z.masked_fill_(torch.ones(48, 48, device="cuda", dtype=torch.bool).triu(1), float("-inf"))
+    ref = torch.softmax(z, -1) @ v[0].repeat_interleave(4, 0).double()
+    assert (prefill_attention(q, k, v, -0.1)[0].double() - ref).norm() < 1e-2 * ref.norm()
+    seen = []
+    torch.vmap(lambda x: seen.append(ops.prefill_attn_ok(x[None], k, v)) or x)(q)
+    assert seen == [False]
+    for a, b, c in ((q.half(), k.half(), v.half()), (q, k.repeat_interleave(2, 1), v.repeat_interleave(2, 1)),
+                    (torch.nn.functional.pad(q, (1, 0))[..., 1:], k, v)):
+        assert not ops.prefill_attn_ok(a, b, c)
+        o = prefill_attention(a, b, c, 0.1).float()
+        assert o.shape == base.shape and torch.isfinite(o).all()
+    assert (prefill_attention(q.half(), k.half(), v.half(), 0.1).float() - base).norm() < 1e-2 * base.norm()
