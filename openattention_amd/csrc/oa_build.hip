@@ -78,64 +78,110 @@ __global__ void __launch_bounds__(64) clear_u32_kernel(uint32_t* p, int n) {
 
 // pass 1: per (KV row, coordinate) the maximum |zc| over the tokens, as float bits (|zc| >= 0,
 // so the unsigned maximum of the bits is the float maximum); zc itself into zc_ws when given
-// (128 bytes per token), so that pass 2 quantizes without a second fma chain
-// The block's 256 key rows are staged through LDS, 64 dims at a time (coalesced 128-byte row
-// segments, rows padded to 144 bytes so that a 16-lane phase of row reads hits distinct banks):
-// a lane walking its own row straight from memory touched 64 lines per load and lost them to
-// the other rows before its next step (5.5x the keys' bytes fetched).  U's rows come through
-// scalar loads (the same for every lane; the fmas take them from SGPRs) rather than LDS
-// broadcasts, which bounded the pass by LDS bandwidth.  The fma chain over d is token_zc's, in
-// the same order.
-constexpr int kZcDims = 64;                    // dims staged per pass
+// (128 bytes per token), so that pass 2 quantizes without a second fma chain.
+// The fma chains run on the fp32 matrix cores: v_mfma_f32_32x32x1_2b_f32 adds one product per output
+// with one rounding, an fma, so that 128 of them over d = 0..127 are token_zc's chains bit for bit
+// (subnormal products included) at twice the vector rate.  A is U (coordinate lane % 32), B dimension d
+// of the wave's 64 tokens (token lane), and a lane ends with coordinates 8 (r / 4) + 4 (lane / 32) + r % 4
+// of tokens lane % 32 and 32 + lane % 32.  U lies in LDS by fours of d: as 128 registers it left two
+// waves per SIMD, the next keys went through scratch and the matrix cores waited for them (1229 us
+// against the figure below).  The key rows reach LDS 64 dims at a time in coalesced 128-byte segments
+// (rows padded to 144 bytes: a 16-lane phase of row reads hits distinct banks), the next segment
+// requested while one is used; a wave takes up to kZcTiles tiles of 64 tokens.  At 256 rows of 32767
+// tokens: 1310 us with the chains on the vector units, 731 us now, 3.2 GB of keys and zc at 4.4 TB/s
+// beside 0.5 ms of matrix instructions; at 16 rows of 10007 tokens 42 -> 26 us.
+constexpr int kZcDims = 64;                    // dims staged per segment
 constexpr int kZcRowQ = kZcDims / 8 + 1;       // uint4 per staged row (8 + 1 pad)
+constexpr int kZcTiles = 8;                    // 64-token tiles per wave
+typedef __attribute__((__vector_size__(32 * sizeof(float)))) float float32v;
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t uint32x4v;
 
-__global__ void __launch_bounds__(kCodeThreads) codes_amax_kernel(const uint16_t* __restrict__ K, long ksh,
-                                                                  long kst, int T,
-                                                                  const float* __restrict__ U,
-                                                                  uint32_t* __restrict__ amax,
-                                                                  float* __restrict__ zc_ws) {
+__global__ void __launch_bounds__(kCodeThreads, 3) codes_amax_kernel(const uint16_t* __restrict__ K, long ksh,
+                                                                     long kst, int T,
+                                                                     const float* __restrict__ U,
+                                                                     uint32_t* __restrict__ amax,
+                                                                     float* __restrict__ zc_ws, int tiles) {
   __shared__ uint32_t s_m[kRQ];
-  __shared__ uint4 s_k[kCodeThreads * kZcRowQ];
+  __shared__ uint4 s_k[kCodeThreads / 64][64 * kZcRowQ];
+  __shared__ float4 s_u[kD / 4][kRQ];
   const int h = blockIdx.y;
-  const float* __restrict__ Uh = U + (long)h * kD * kRQ;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int hi = lane >> 5, n32 = lane & 31;
+  const float* Uh = U + (long)h * kD * kRQ;
   if (threadIdx.x < kRQ) s_m[threadIdx.x] = 0u;
-  const int t0 = blockIdx.x * kCodeThreads;
-  const int t = t0 + threadIdx.x;
+  for (int i = threadIdx.x; i < kD / 4 * kRQ; i += kCodeThreads) {
+    const float* up = Uh + (i / kRQ) * 4 * kRQ + i % kRQ;
+    s_u[i / kRQ][i % kRQ] = make_float4(up[0], up[kRQ], up[2 * kRQ], up[3 * kRQ]);
+  }
+  __syncthreads();
   const uint16_t* kh = K + (long)h * ksh;
-  float z[kRQ];
+  const int ntiles = (T + 63) / 64;
+  const int tile0 = (blockIdx.x * (kCodeThreads / 64) + wave) * tiles;
+  const int tend = min(ntiles, tile0 + tiles);
+  // a segment's 512 16-byte words: lane takes word lane % 8 of rows lane / 8 + 8 j
+  uint32x4v seg[8];
+  auto fetch = [&](int tile, int half) {
 #pragma unroll
-  for (int r = 0; r < kRQ; ++r) z[r] = 0.f;
-  for (int d0 = 0; d0 < kD; d0 += kZcDims) {
-    if (d0) __syncthreads();   // every lane has read the previous dims
+    for (int j = 0; j < 8; ++j)
+      seg[j] = *reinterpret_cast<const uint32x4v*>(kh + (long)min(tile * 64 + (lane >> 3) + 8 * j, T - 1) * kst +
+                                                   half * kZcDims + 8 * (lane & 7));
+  };
+  uint32_t mx[16];
 #pragma unroll
-    for (int j = 0; j < kZcDims / 8; ++j) {
-      const int i = threadIdx.x + j * kCodeThreads;
-      const int r = i / (kZcDims / 8), c = i % (kZcDims / 8);
-      s_k[r * kZcRowQ + c] =
-          *reinterpret_cast<const uint4*>(kh + (long)min(t0 + r, T - 1) * kst + d0 + 8 * c);
+  for (int r = 0; r < 16; ++r) mx[r] = 0u;
+  if (tile0 < tend) fetch(tile0, 0);
+#pragma unroll 1
+  for (int tile = tile0; tile < tend; ++tile) {
+    float32v acc = {};
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      // (one wave's LDS: its reads of the last segment precede these writes in order)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        *reinterpret_cast<uint32x4v*>(&s_k[wave][((lane >> 3) + 8 * j) * kZcRowQ + (lane & 7)]) = seg[j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+      fetch(min(tile + half, ntiles - 1), half ^ 1);
+#pragma unroll
+      for (int c = 0; c < kZcDims / 8; ++c) {
+        float kv[8];
+        oa::unpack8(s_k[wave][lane * kZcRowQ + c], kv);
+        const float4 ua = s_u[half * (kZcDims / 4) + 2 * c][n32], ub = s_u[half * (kZcDims / 4) + 2 * c + 1][n32];
+        const float u[8] = {ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(u[e], kv[e], acc, 0, 0, 0);
+      }
     }
-    __syncthreads();
-    for (int c = 0; c < kZcDims / 8; ++c) {
-      float kv[8];
-      oa::unpack8(s_k[threadIdx.x * kZcRowQ + c], kv);
 #pragma unroll
-      for (int dd = 0; dd < 8; ++dd) {
-        const float* ud = Uh + (d0 + 8 * c + dd) * kRQ;
+    for (int b = 0; b < 2; ++b) {
+      const int t = tile * 64 + 32 * b + n32;
+      if (t < T) {
 #pragma unroll
-        for (int r = 0; r < kRQ; ++r) z[r] = fmaf(kv[dd], ud[r], z[r]);
+        for (int r = 0; r < 16; ++r) mx[r] = max(mx[r], __float_as_uint(fabsf(acc[16 * b + r])));
+        if (zc_ws) {
+          float4* zo = reinterpret_cast<float4*>(zc_ws + ((long)h * T + t) * kRQ + 4 * hi);
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            zo[2 * g] = make_float4(acc[16 * b + 4 * g], acc[16 * b + 4 * g + 1], acc[16 * b + 4 * g + 2],
+                                    acc[16 * b + 4 * g + 3]);
+        }
       }
     }
   }
-  const bool in = t < T;
-  if (zc_ws && in) {
-    float4* zo = reinterpret_cast<float4*>(zc_ws + ((long)h * T + t) * kRQ);
+  __syncthreads();                               // s_m is cleared
 #pragma unroll
-    for (int r4 = 0; r4 < kRQ / 4; ++r4) zo[r4] = make_float4(z[4 * r4], z[4 * r4 + 1], z[4 * r4 + 2], z[4 * r4 + 3]);
-  }
-#pragma unroll
-  for (int r = 0; r < kRQ; ++r) {
-    const unsigned m = oa::wave_max_u32(in ? __float_as_uint(fabsf(z[r])) : 0u);
-    if ((threadIdx.x & 63) == 0) atomicMax(&s_m[r], m);
+  for (int r = 0; r < 16; ++r) {
+    // the maximum over the 32 lanes that hold this coordinate
+    uint32_t v = mx[r];
+    v = max(v, oa::dpp_u32<0xB1, 0xf>(v));
+    v = max(v, oa::dpp_u32<0x4E, 0xf>(v));
+    v = max(v, oa::dpp_u32<0x141, 0xf>(v));
+    v = max(v, oa::dpp_u32<0x140, 0xf>(v));
+    const auto x = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = max((uint32_t)x[0], (uint32_t)x[1]);
+    if (n32 == 0) atomicMax(&s_m[8 * (r >> 2) + 4 * hi + (r & 3)], v);
   }
   __syncthreads();
   if (threadIdx.x < kRQ) atomicMax(&amax[h * kRQ + threadIdx.x], s_m[threadIdx.x]);
@@ -864,8 +910,13 @@ extern "C" int oa_qgs_codes(const void* K, long k_stride_h, long k_stride_t, int
   hipLaunchKernelGGL(clear_u32_kernel, dim3(std::min(64, (kv_rows * kRQ + 63) / 64)), dim3(64), 0, s,
                      amax_ws, kv_rows * kRQ);
   const dim3 grid((T + kCodeThreads - 1) / kCodeThreads, kv_rows);
-  hipLaunchKernelGGL(codes_amax_kernel, grid, dim3(kCodeThreads), 0, s, k, k_stride_h, k_stride_t, T, U,
-                     amax_ws, zc_ws);
+  // tiles per wave: eight spread the block's load of U; fewer where the grid would leave a SIMD with
+  // less than four waves
+  const int ntiles = (T + 63) / 64;
+  const int tiles = (int)std::min<long>(kZcTiles, std::max<long>(1, (long)ntiles * kv_rows / 4096));
+  const int per = kCodeThreads / 64 * tiles;
+  hipLaunchKernelGGL(codes_amax_kernel, dim3((ntiles + per - 1) / per, kv_rows), dim3(kCodeThreads), 0, s, k,
+                     k_stride_h, k_stride_t, T, U, amax_ws, zc_ws, tiles);
   hipLaunchKernelGGL(codes_write_kernel, grid, dim3(kCodeThreads), 0, s, k, k_stride_h, k_stride_t, T, U,
                      amax_ws, codes, codes_stride_h, scale, zc_ws);
   return OA_LAUNCH_STATUS();

@@ -883,6 +883,39 @@ def test_build_codes_bit_exact(T):
         assert np.array_equal(codes.cpu().numpy(), rc)
 
 
+@pytest.mark.parametrize("T,rows", [(1, 1), (31, 3), (33, 1), (63, 2), (64, 2), (65, 3), (321, 5), (8257, 37),
+                                    (2113, 260), (2113, 970)])
+def test_codes_chains_on_the_matrix_cores_bit_exact(T, rows):
+    """The products' chains against the restatement's fma chains, bit for bit, at the edges of a wave's
+    64-token tiles and of the tiles per wave, with padded key rows: ordinary values, one row of values
+    whose products are subnormal and one that spans the exponent range."""
+    print(f"[case] codes chains T={T} rows={rows}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(T + rows)
+    Kd = torch.zeros(rows, T + 2, D + 8, device=DEV, dtype=torch.bfloat16)
+    Kd[:, :T, :D] = torch.randn(rows, T, D, device=DEV, generator=gen, dtype=torch.bfloat16)
+    U = torch.randn(rows, D, 32, device=DEV, generator=gen)
+    if rows > 1:
+        U[1] *= 2.0**-120
+        Kd[1] *= 2.0**-12
+    if rows > 2:
+        Kd[2, :T, :D] *= 2.0 ** torch.randint(-40, 40, (T, D), device=DEV, generator=gen).to(torch.bfloat16)
+    codes = torch.zeros(rows, T, 32, device=DEV, dtype=torch.int8)
+    scale = torch.zeros(rows, 32, device=DEV)
+    ws = torch.empty(rows * 32, device=DEV, dtype=torch.int32)
+    zc = torch.full((rows, T, 32), float("nan"), device=DEV)
+    ops.qgs_codes(Kd[:, :, :D], T, U, codes, scale, ws, zc)
+    torch.cuda.synchronize()
+    pick = [r for r in (0, 1, 2, rows // 2, rows - 1) if r < rows]
+    K = Kd[pick][:, :T, :D].contiguous().view(torch.int16).cpu().numpy().view(np.uint16)
+    rc, rs = O.qgs_codes(K, T, U[pick].cpu().numpy())
+    assert np.array_equal(scale.cpu().numpy()[pick], rs)
+    assert np.array_equal(codes.cpu().numpy()[pick], rc)
+    # the kept zc itself: pass 2 without it forms the chains on the vector units
+    again = torch.zeros_like(codes)
+    ops.qgs_codes(Kd[:, :, :D], T, U, again, scale, ws, None)
+    assert torch.equal(again, codes)
+
+
 @pytest.mark.parametrize("T,G_", [(4095, 4), (1000, 4), (1000, 2)])
 def test_build_projection_and_kmeans(T, G_):
     """QGC projection on the bf16 matrix cores: bf16(k W) agrees with the exact-sum restatement
