@@ -41,8 +41,10 @@ __device__ __forceinline__ void gate_row(const GateArgs& a, int row, float* s_sc
   const int lane = tid & 63;
   const int kvr = row / a.G;
   constexpr int kBatch = 4;     // larger batches spill at the 64-VGPR cap
-  float sk[kBatch][2], s2[kBatch][2], nbv[kBatch];
+  float sk[kBatch][2], s2[kBatch][2], ntl;      // ntl: n_c of this lane's cluster of the batch
+  const int lc = kGateWaves * (lane % kBatch);
   auto issue = [&](int c0) {
+    ntl = a.nb[(long)row * a.nb_stride + min(c0 + lc, a.C - 1)];
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int c = min(c0 + kGateWaves * i, a.C - 1);
@@ -51,7 +53,6 @@ __device__ __forceinline__ void gate_row(const GateArgs& a, int row, float* s_sc
       sk[i][1] = a.Sk[base + lane + 64];
       s2[i][0] = a.Sk2[base + lane];
       s2[i][1] = a.Sk2[base + lane + 64];
-      nbv[i] = a.nb[(long)row * a.nb_stride + c];
     }
   };
   for (int c = tid; c < a.C; c += kGateThreads) s_selmask[c] = 0ull;
@@ -76,6 +77,18 @@ __device__ __forceinline__ void gate_row(const GateArgs& a, int row, float* s_sc
     kw0 = *reinterpret_cast<const uint4*>(a.K + (long)kvr * a.k_sb + (long)tok0 * a.k_ss + (e0 % kW) * 8);
   if (tok1 >= 0)
     kw1 = *reinterpret_cast<const uint4*>(a.K + (long)kvr * a.k_sb + (long)tok1 * a.k_ss + (e1 % kW) * 8);
+  // a batch as if its clusters held no selected token (most do not)
+  auto batch = [&](int c0) {
+    float zb, sv, qs;
+    gate_dots_batch<kBatch>(a, sk, s2, ntl, q_lo, q_hi, qq_lo, qq_hi, lane, &zb, &sv, &qs);
+    if (lane < kBatch && c0 + lc < a.C) {
+      s_zbar[c0 + lc] = zb;
+      s_s2[c0 + lc] = sv;
+      s_nt[c0 + lc] = ntl;
+      s_qsk[c0 + lc] = qs;
+    }
+  };
+  // one cluster that holds some, again with its mask
   auto dots = [&](float k0, float k1, float t0, float t1, float nbc, int c,
                   unsigned long long mask) {
     float zb, sv, nt, qs;
@@ -84,16 +97,23 @@ __device__ __forceinline__ void gate_row(const GateArgs& a, int row, float* s_sc
       s_zbar[c] = zb;
       s_s2[c] = sv;
       s_nt[c] = nt;
-      s_qsk[c] = qs;
     }
   };
-  // ---- the first batch as if its clusters held no selected token (most do not) while the
-  // selected keys arrive; a cluster that holds one is done again below
+  auto redo = [&](int c0) {
+    if (!__any(c0 + lc < a.C && s_selmask[min(c0 + lc, kMaxC - 1)] != 0ull)) return;
+    // (the batch's stores to the same words come first: one wave's LDS is in order)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int i = 0; i < kBatch; ++i) {
-    const int c = wave + kGateWaves * i;
-    if (c < a.C) dots(sk[i][0], sk[i][1], s2[i][0], s2[i][1], nbv[i], c, 0ull);
-  }
+    for (int i = 0; i < kBatch; ++i) {
+      const int c = c0 + kGateWaves * i;
+      if (c < a.C && s_selmask[c])
+        dots(sk[i][0], sk[i][1], s2[i][0], s2[i][1],
+             __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ntl), i)), c, s_selmask[c]);
+    }
+  };
+  // ---- the first batch while the selected keys arrive
+  if (wave < a.C) batch(wave);
   // ---- selected keys into LDS; per cluster, the mask of its selected tokens
   if (cm >= 0) atomicOr(&s_selmask[cm], 1ull << tid);
   if (e0 < n_sel * kW) {
@@ -109,19 +129,12 @@ __device__ __forceinline__ void gate_row(const GateArgs& a, int row, float* s_sc
     for (int j = 0; j < 8; ++j) s_k[(e1 / kW) * OA_D + (e1 % kW) * 8 + j] = x[j];
   }
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kBatch; ++i) {
-    const int c = wave + kGateWaves * i;
-    if (c < a.C && s_selmask[c]) dots(sk[i][0], sk[i][1], s2[i][0], s2[i][1], nbv[i], c, s_selmask[c]);
-  }
+  if (wave < a.C) redo(wave);
   // ---- the other batches, all loads of a batch in flight
   for (int c0 = wave + kGateWaves * kBatch; c0 < a.C; c0 += kGateWaves * kBatch) {
     issue(c0);
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i) {
-      const int c = c0 + kGateWaves * i;
-      if (c < a.C) dots(sk[i][0], sk[i][1], s2[i][0], s2[i][1], nbv[i], c, s_selmask[c]);
-    }
+    batch(c0);
+    redo(c0);
   }
   __syncthreads();
   // ---- scalar tails, one cluster per thread
@@ -562,7 +575,7 @@ struct FixLds {
   unsigned long long selmask[kMaxC];
   int sel[kMaxSel];
   int hit[kMaxSel];
-  float zb[kMaxSel], s2[kMaxSel], hnt[kMaxSel];
+  alignas(16) unsigned long long list[oa_sel::kTopList];   // the top-k wave's
   int nhit;
 };
 
@@ -641,6 +654,8 @@ __device__ __forceinline__ void fix_finish(const GateArgs& a, int row, FixLds& L
       s2[i][1] = a.Sk2[base + lane + 64];
       nbv[i] = a.nb[(long)row * a.nb_stride + c];
     }
+    // lane i keeps the i-th hit's values, for the scalar tail of one cluster per lane
+    float zbl = 0.f, svl = 0.f, ntl = 0.f;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int h = h0 + kWv * i;
@@ -648,23 +663,20 @@ __device__ __forceinline__ void fix_finish(const GateArgs& a, int row, FixLds& L
         float zb, sv, nt, qs;
         gate_dots(a, sk[i][0], sk[i][1], s2[i][0], s2[i][1], nbv[i], q_lo, q_hi, qq_lo, qq_hi,
                   L.selmask[L.hit[h]], s_k, lane, &zb, &sv, &nt, &qs);
-        if (lane == 0) {
-          L.zb[h] = zb;
-          L.s2[h] = sv;
-          L.hnt[h] = nt;
-        }
+        zbl = lane == i ? zb : zbl;
+        svl = lane == i ? sv : svl;
+        ntl = lane == i ? nt : ntl;
       }
     }
-  }
-  __syncthreads();
-  // the scalar tails, one hit cluster per thread
-  if (tid < nhit) {
-    const int c = L.hit[tid];
-    const float sc = gate_score(L.zb[tid], L.s2[tid], L.hnt[tid]);
-    L.score[c] = sc;
-    L.nt[c] = L.hnt[tid];
-    a.score[(long)row * a.out_stride + c] = sc;
-    a.n_t[(long)row * a.out_stride + c] = L.hnt[tid];
+    const int hl = h0 + kWv * lane;
+    if (lane < kBatch && hl < nhit) {
+      const int c = L.hit[hl];
+      const float sc = gate_score(zbl, svl, ntl);
+      L.score[c] = sc;
+      L.nt[c] = ntl;
+      a.score[(long)row * a.out_stride + c] = sc;
+      a.n_t[(long)row * a.out_stride + c] = ntl;
+    }
   }
   __syncthreads();
   if (wave == 0) waterfill_row<NS>(L.score, L.nt, quota_row, a.C, budget, lane, L.cw);
@@ -691,7 +703,7 @@ __global__ void __launch_bounds__(kFixThreads) topk_fix_fill_kernel(TopkArgs t, 
   if (threadIdx.x < 64)
     oa_sel::topk_reg_row<TPL, KR, true>(t.H, t.h_stride, t.TM, t.tm_stride, t.ntiles, sel,
                                         a.sel_stride, *t.n_dev, t.ns, t.nl, t.k_top, t.rs, row,
-                                        threadIdx.x, L.sel);
+                                        threadIdx.x, L.list, L.sel);
   else
     fix_load(a, row, L, 64, kFixThreads - 64, false);
   __syncthreads();
@@ -703,26 +715,25 @@ __global__ void __launch_bounds__(kFixThreads) topk_fix_fill_kernel(TopkArgs t, 
 // Wave 0 runs the row's register top-k while waves 1 .. W-1 compute the clusters' pooled
 // ErrorGate dot products (gate_dots with an empty mask): wave w takes the batches of kPoolBatch
 // consecutive clusters w - 1, w - 1 + (W - 1), ... (a fixed split: every loop bound depends on
-// the wave index and C only), all of a batch's loads in flight.  Then every cluster's scalar
-// tail (one per thread), the clusters holding a selected token done again with their masks
-// (fix_finish), and the fill on wave 0.  Every cluster's score and n_t, and q . Sk, are
-// written out.
+// the wave index and C only), all of a batch's loads in flight, and then its clusters' scalar tails,
+// one per lane (a wave has at most 24 of 64 clusters, 40 of 256).  Then the clusters holding a selected
+// token are done again with their masks (fix_finish), and the fill runs on wave 0.  Every cluster's
+// score and n_t, and q . Sk, are written out.  (32 rows of 64 clusters: 25.4 -> 21.5 us with the ranked
+// top-k and the scalar tails beside it; what is left is the chain of top-k, correction and fill.)
 constexpr int kPoolBatch = 8;
-struct Gate2Lds {
-  FixLds f;
-  float zb[kMaxC], s2[kMaxC], nt[kMaxC];
-};
 
 template <int W>
-__device__ __forceinline__ void pooled_batches(const GateArgs& a, int row, Gate2Lds& L) {
+__device__ __forceinline__ void pooled_batches(const GateArgs& a, int row, FixLds& L) {
   constexpr int nGW = W - 1;
   const int gw = (int)(threadIdx.x >> 6) - 1;       // 0 .. W-2
   const int lane = threadIdx.x & 63;
   const float q_lo = oa::bf16_to_f32(a.q[(long)row * a.q_stride + lane]);
   const float q_hi = oa::bf16_to_f32(a.q[(long)row * a.q_stride + lane + 64]);
   const float qq_lo = q_lo * q_lo, qq_hi = q_hi * q_hi;
-  for (int c0 = gw * kPoolBatch; c0 < a.C; c0 += nGW * kPoolBatch) {
-    float sk[kPoolBatch][2], s2[kPoolBatch][2], nbv[kPoolBatch];
+  float zbl = 0.f, svl = 0.f, ntl = 0.f;            // of this lane's cluster
+  int cl = -1, slot = 0;
+  for (int c0 = gw * kPoolBatch; c0 < a.C; c0 += nGW * kPoolBatch, ++slot) {
+    float sk[kPoolBatch][2], s2[kPoolBatch][2];
 #pragma unroll
     for (int i = 0; i < kPoolBatch; ++i) {
       const int c = min(c0 + i, a.C - 1);
@@ -731,53 +742,45 @@ __device__ __forceinline__ void pooled_batches(const GateArgs& a, int row, Gate2
       sk[i][1] = a.Sk[base + lane + 64];
       s2[i][0] = a.Sk2[base + lane];
       s2[i][1] = a.Sk2[base + lane + 64];
-      nbv[i] = a.nb[(long)row * a.nb_stride + c];
     }
-#pragma unroll
-    for (int i = 0; i < kPoolBatch; ++i) {
-      const int c = c0 + i;
-      if (c < a.C) {
-        float zb, sv, nt, qs;
-        gate_dots(a, sk[i][0], sk[i][1], s2[i][0], s2[i][1], nbv[i], q_lo, q_hi, qq_lo, qq_hi, 0ull,
-                  nullptr, lane, &zb, &sv, &nt, &qs);
-        if (lane == 0) {
-          L.zb[c] = zb;
-          L.s2[c] = sv;
-          L.nt[c] = nt;
-          if (a.qsk) a.qsk[(long)row * a.C + c] = qs;
-        }
-      }
+    const int c = c0 + lane % kPoolBatch;           // lane l's cluster of the batch
+    const float nt = a.nb[(long)row * a.nb_stride + min(c, a.C - 1)];
+    float zb, sv, qs;
+    gate_dots_batch<kPoolBatch>(a, sk, s2, nt, q_lo, q_hi, qq_lo, qq_hi, lane, &zb, &sv, &qs);
+    if (c < a.C) {
+      if (lane / kPoolBatch == slot) { zbl = zb; svl = sv; ntl = nt; cl = c; }
+      if (a.qsk && lane < kPoolBatch) a.qsk[(long)row * a.C + c] = qs;
     }
+  }
+  if (cl >= 0) {
+    L.score[cl] = gate_score(zbl, svl, ntl);
+    L.nt[cl] = ntl;
+    L.selmask[cl] = 0ull;
   }
 }
 
 template <int NS, int TPL, int KR, int W>
 __global__ void __launch_bounds__(64 * W) topk_gate2_fill_kernel(TopkArgs t, GateArgs a, int32_t* sel,
                                                                   float* __restrict__ quota, double budget) {
-  __shared__ Gate2Lds L;
+  static_assert((64 * NS / kPoolBatch + W - 2) / (W - 1) * kPoolBatch <= 64, "a wave's clusters fit its lanes");
+  __shared__ FixLds L;
   constexpr int kThr = 64 * W;
   const int row = oa::xcd_row(blockIdx.x, gridDim.x);   // a KV row's query rows share one L2
   const int tid = threadIdx.x;
   if (tid < 64)
     oa_sel::topk_reg_row<TPL, KR, true>(t.H, t.h_stride, t.TM, t.tm_stride, t.ntiles, sel,
-                                        a.sel_stride, *t.n_dev + oa::row_extra(row, a.qsh), t.ns, t.nl, t.k_top, t.rs, row, tid,
-                                        L.f.sel);
+                                        a.sel_stride, *t.n_dev + oa::row_extra(row, a.qsh), t.ns, t.nl,
+                                        t.k_top, t.rs, row, tid, L.list, L.sel);
   else
     pooled_batches<W>(a, row, L);
-  if (tid == 0) L.f.nhit = 0;
+  if (tid == 0) L.nhit = 0;
   __syncthreads();
-  for (int c = tid; c < a.C; c += kThr) {
-    L.f.score[c] = gate_score(L.zb[c], L.s2[c], L.nt[c]);
-    L.f.nt[c] = L.nt[c];
-    L.f.selmask[c] = 0ull;
-  }
-  __syncthreads();
-  fix_finish<NS, kThr>(a, row, L.f, quota + (long)row * a.C, budget);
+  fix_finish<NS, kThr>(a, row, L, quota + (long)row * a.C, budget);
   // the rows' pooled values of the clusters no selected token touched (fix_finish wrote the others)
   for (int c = tid; c < a.C; c += kThr) {
-    if (L.f.selmask[c]) continue;
-    a.score[(long)row * a.out_stride + c] = L.f.score[c];
-    a.n_t[(long)row * a.out_stride + c] = L.f.nt[c];
+    if (L.selmask[c]) continue;
+    a.score[(long)row * a.out_stride + c] = L.score[c];
+    a.n_t[(long)row * a.out_stride + c] = L.nt[c];
   }
 }
 
@@ -938,8 +941,8 @@ int oa_rows::topk_gate_fill(uint16_t* H, long h_stride, const float* TM, long tm
       hipLaunchKernelGGL((topk_gate2_fill_kernel<NS, T, KK, 16>), g, dim3(1024), lds, s, t, a, sel, quota, bd); \
     else if (wv == 8)                                                                           \
       hipLaunchKernelGGL((topk_gate2_fill_kernel<NS, T, KK, 8>), g, dim3(512), lds, s, t, a, sel, quota, bd); \
-    else                                                                                        \
-      hipLaunchKernelGGL((topk_gate2_fill_kernel<NS, T, KK, 4>), g, dim3(256), lds, s, t, a, sel, quota, bd); \
+    else   /* kFuseRows rows or more: C <= 64 only */                                           \
+      hipLaunchKernelGGL((topk_gate2_fill_kernel<1, T, KK, 4>), g, dim3(256), lds, s, t, a, sel, quota, bd); \
   } while (0)
 #define OA_TG2_NS(NS)                                                                           \
   do {                                                                                          \

@@ -79,6 +79,70 @@ __device__ __forceinline__ void gate_dots(const GateArgs& a, float sk_lo, float 
   *nt_out = nt;
 }
 
+// wave_sum of NB (4 or 8) values at once: lane l ends with the sum of p[l % NB].  The levels m = 1, 2
+// (and 4) halve the number of values instead of leaving two lanes with the same one: a lane keeps the
+// value its bit selects and adds its partner's copy of it, the sum the butterfly forms (addition is
+// commutative), in NB + 2 additions where NB butterflies take 6 NB.
+__device__ __forceinline__ float lane_xor4(float v) {
+  const int b = __float_as_int(v);
+  const int lo = __builtin_amdgcn_update_dpp(b, b, 0x104, 0xf, 0x5, false);    // row_shl:4 into quads 0, 2
+  return __int_as_float(__builtin_amdgcn_update_dpp(lo, b, 0x114, 0xf, 0xa, false));   // row_shr:4 into 1, 3
+}
+template <int NB>
+__device__ __forceinline__ float wave_sums(const float (&p)[NB], int lane) {
+  static_assert(NB == 4 || NB == 8, "values per batch");
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
+  float t[NB / 2], u[NB / 4];
+#pragma unroll
+  for (int k = 0; k < NB / 2; ++k)
+    t[k] = (b0 ? p[2 * k + 1] : p[2 * k]) + oa::dpp_f32<0xB1>(b0 ? p[2 * k] : p[2 * k + 1]);
+#pragma unroll
+  for (int k = 0; k < NB / 4; ++k)
+    u[k] = (b1 ? t[2 * k + 1] : t[2 * k]) + oa::dpp_f32<0x4E>(b1 ? t[2 * k] : t[2 * k + 1]);
+  float v = NB == 8 ? (b2 ? u[NB / 4 - 1] : u[0]) + lane_xor4(b2 ? u[0] : u[NB / 4 - 1]) : u[0] + lane_xor4(u[0]);
+  v = v + oa::dpp_f32<0x128>(v);                   // row_ror:8, m = 8
+  return oa::swap32_sum(oa::swap16_sum(v));
+}
+
+// gate_dots with an empty mask of NB clusters together: lane l holds cluster l % NB's n_c in nt and
+// ends with that cluster's values.  The same arithmetic bit for bit: the divisions by n_c share one
+// reciprocal per cluster, formed by its lane, and the sums over the dimensions come from wave_sums.
+// (One cluster at a time the pass was bound by instruction issue, three butterflies and four divisions'
+// checks a cluster: at 1024 rows of 64 clusters its waves, not the top-k's, held the fused launch, which
+// takes 38.5 us with this and the ranked top-k against 45; oa_errorgate 59 us against 62 at 1024 rows of
+// 256 clusters, which is 4.5 TB/s, and 30 against 33.5 at 256 rows.)
+template <int NB>
+__device__ __forceinline__ void gate_dots_batch(const GateArgs& a, const float (&sk)[NB][2],
+                                                const float (&s2)[NB][2], float nt, float q_lo, float q_hi,
+                                                float qq_lo, float qq_hi, int lane, float* zbar_out,
+                                                float* s2_out, float* qsk_out) {
+  const float den_l = fmaxf(nt, 1.0f);
+  const float r_l = 1.0f / den_l;
+  float pq[NB], pz[NB], ps[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const float sl = sk[i][0], sh = sk[i][1], ml = s2[i][0], mh = s2[i][1];
+    const float den = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(den_l), i));
+    pq[i] = fmaf(q_hi, sh, q_lo * sl);
+    float kb_lo, kb_hi, ks_lo, ks_hi;
+    if (__all(div_fast_ok(sl) && div_fast_ok(sh) && div_fast_ok(ml) && div_fast_ok(mh))) {
+      const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r_l), i));
+      kb_lo = div_den(sl, den, r); kb_hi = div_den(sh, den, r);
+      ks_lo = div_den(ml, den, r); ks_hi = div_den(mh, den, r);
+    } else {
+      kb_lo = sl / den; kb_hi = sh / den;
+      ks_lo = ml / den; ks_hi = mh / den;
+    }
+    const float v_lo = fmaxf(ks_lo - kb_lo * kb_lo, 0.f);
+    const float v_hi = fmaxf(ks_hi - kb_hi * kb_hi, 0.f);
+    pz[i] = fmaf(q_hi, kb_hi, q_lo * kb_lo);
+    ps[i] = fmaf(qq_hi, v_hi, qq_lo * v_lo);
+  }
+  *qsk_out = wave_sums<NB>(pq, lane);
+  *zbar_out = a.sc * wave_sums<NB>(pz, lane);
+  *s2_out = a.sc2 * wave_sums<NB>(ps, lane);
+}
+
 // the scalar tail of one cluster's wl1 score
 __device__ __forceinline__ float gate_score(float zbar, float s2, float nt) {
   if (!(nt >= 2.0f)) s2 = 0.f;
@@ -104,7 +168,7 @@ __device__ __forceinline__ void gate_pooled_unit(const GateArgs& a, int row, int
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
-  float sk[kPer][2], s2[kPer][2], nbv[kPer];
+  float sk[kPer][2], s2[kPer][2];
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int c = min(c0 + wave + 4 * i, a.C - 1);
@@ -113,26 +177,18 @@ __device__ __forceinline__ void gate_pooled_unit(const GateArgs& a, int row, int
     sk[i][1] = a.Sk[base + lane + 64];
     s2[i][0] = a.Sk2[base + lane];
     s2[i][1] = a.Sk2[base + lane + 64];
-    nbv[i] = a.nb[(long)row * a.nb_stride + c];
   }
+  const int j = wave + 4 * (lane % kPer);       // this lane's cluster: its slot in the unit
+  const float nt = a.nb[(long)row * a.nb_stride + min(c0 + j, a.C - 1)];
   const float q_lo = oa::bf16_to_f32(a.q[(long)row * a.q_stride + lane]);
   const float q_hi = oa::bf16_to_f32(a.q[(long)row * a.q_stride + lane + 64]);
-  const float qq_lo = q_lo * q_lo, qq_hi = q_hi * q_hi;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int j = wave + 4 * i;                 // the cluster's slot in the unit
-    const int c = c0 + j;
-    if (c < a.C) {
-      float zb, sv, nt, qs;
-      gate_dots(a, sk[i][0], sk[i][1], s2[i][0], s2[i][1], nbv[i], q_lo, q_hi, qq_lo, qq_hi, 0ull,
-                nullptr, lane, &zb, &sv, &nt, &qs);
-      if (lane == 0) {
-        s_zb[j] = zb;
-        s_s2[j] = sv;
-        s_nt[j] = nt;
-        if (a.qsk) a.qsk[(long)row * a.C + c] = qs;
-      }
-    }
+  float zb, sv, qs;
+  gate_dots_batch<kPer>(a, sk, s2, nt, q_lo, q_hi, q_lo * q_lo, q_hi * q_hi, lane, &zb, &sv, &qs);
+  if (lane < kPer && c0 + j < a.C) {
+    s_zb[j] = zb;
+    s_s2[j] = sv;
+    s_nt[j] = nt;
+    if (a.qsk) a.qsk[(long)row * a.C + c0 + j] = qs;
   }
   __syncthreads();
   if (tid < kPoolClusters && c0 + tid < a.C) {

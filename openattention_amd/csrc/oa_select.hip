@@ -205,14 +205,32 @@ __device__ __forceinline__ int lanes_below(unsigned long long m, int lane) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
-// Radix-select variant for rows of at most 64*TPL tiles and k_top <= kMaxTop.  The k-th largest
-// tile key T is found bit by bit from ballot counts over the tile keys held in registers (lane
-// l: tiles l, l + 64, ...); the chosen tiles are those above T and the lowest-index ones equal
-// to it.  Every top-k token scores at least T (k chosen tiles each hold a token that does), so
-// only candidates whose key reaches T join the candidate list (with HEADS: whose head reaches
-// T's head, exact scores then recomputed for the list alone).  The k-th largest candidate key
-// (score key << 32 | ~position: distinct) is found the same way, and the k winners are written
-// in descending key order, as repeated wave maxima would give them.
+// the number of the list's m distinct keys above x; a list of at most kRankList is ranked this way (past
+// it the bit search's fixed cost is the lower one)
+constexpr int kRankList = 256;
+__device__ __forceinline__ int rank_in(const unsigned long long* list, int m, unsigned long long x) {
+  int r0 = 0, r1 = 0, i = 0;
+  for (; i + 4 <= m; i += 4) {
+    const unsigned long long y0 = list[i], y1 = list[i + 1], y2 = list[i + 2], y3 = list[i + 3];
+    r0 += (y0 > x ? 1 : 0) + (y1 > x ? 1 : 0);
+    r1 += (y2 > x ? 1 : 0) + (y3 > x ? 1 : 0);
+  }
+  for (; i < m; ++i) r0 += list[i] > x ? 1 : 0;
+  return r0 + r1;
+}
+
+// Variant for rows of at most 64*TPL tiles and k_top <= kMaxTop.  The k-th of the distinct lane maxima
+// (lane l holds tiles l, l + 64, ...) bounds the k-th largest tile key from below; the tiles at or above
+// it, k and some, are listed and ranked by counting the larger keys (each list entry against the others,
+// over broadcast LDS reads).  Where the list is long (many equal maxima) the k-th largest tile key T is
+// found bit by bit from ballot counts over the tile keys instead; the chosen tiles are those above T and
+// the lowest-index ones equal to it, the same set.  Every top-k token scores at least T (k chosen tiles
+// each hold a token that does), so only candidates whose key reaches T join the candidate list (with
+// HEADS: whose head reaches T's head, exact scores then recomputed for the list alone).  The candidate
+// keys (score key << 32 | ~position: distinct) are ranked the same way, or the k-th largest found bit by
+// bit where they are many, and the k winners are written in descending key order, as repeated wave
+// maxima would give them.  The searches are chains of dependent wave operations: at 256 rows of 2048
+// tiles, k = 38, bit by bit alone 50 us, ranked 19 us.
 // Sink, local and unwritten positions are candidates scoring -inf (the register variant's and
 // graph_runner.py:145-151's rule): a row with fewer than k_top live positions is filled with the
 // lowest such positions, so the list always holds at least k_top candidates, each below
@@ -226,6 +244,7 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
   __shared__ int s_tile[kMaxTop];
   __shared__ unsigned long long s_ck[kMaxTop * 64];   // candidate positions, then their keys
   __shared__ unsigned long long s_win[kMaxTop];
+  __shared__ uint32_t s_T;
   const int row = oa::xcd_row(blockIdx.x, gridDim.x);   // a KV row's query rows share one L2
   const int lane = threadIdx.x;
   const int n = *n_dev + oa::row_extra(row, rs.qsh);
@@ -244,30 +263,62 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
   for (int j = 0; j < TPL; ++j) tv[j] = TM[(long)row * tm_stride + min(j * 64 + lane, ntiles - 1)];
 #pragma unroll
   for (int j = 0; j < TPL; ++j) tk[j] = j * 64 + lane < ntiles ? oa::float_key(tv[j]) : 0u;
-  // ---- T: the largest key value reached by at least k tiles
-  uint32_t T = 0u;
-  for (int bit = 31; bit >= 0; --bit) {
-    const uint32_t cand = T | (1u << bit);
-    int cnt = 0;
+  // ---- the tiles at or above the k-th distinct lane maximum
+  uint32_t cur = 0u, bound = 0u;
 #pragma unroll
-    for (int j = 0; j < TPL; ++j) cnt += __popcll(__ballot(tk[j] >= cand));
-    if (cnt >= k_top) T = cand;
+  for (int j = 0; j < TPL; ++j) cur = max(cur, tk[j]);
+  for (int i = 0; i < k_top; ++i) {
+    bound = oa::wave_max_u32(cur);
+    cur = cur == bound ? 0u : cur;
   }
-  int need = k_top;
-#pragma unroll
-  for (int j = 0; j < TPL; ++j) need -= __popcll(__ballot(tk[j] > T));
-  // ---- the chosen tiles, in tile order: above T, then equal to T while need lasts
-  int nt = 0;
+  int nl_t = 0;
 #pragma unroll
   for (int j = 0; j < TPL; ++j) {
-    const unsigned long long meq = __ballot(tk[j] == T);
-    const bool take = tk[j] > T || (tk[j] == T && lanes_below(meq, lane) < need);
-    need -= min(need, __popcll(meq));
-    const unsigned long long mt = __ballot(take);
-    if (take) s_tile[nt + lanes_below(mt, lane)] = j * 64 + lane;
-    nt += __popcll(mt);
+    const int t = j * 64 + lane;
+    const bool in = t < ntiles && tk[j] >= bound;
+    const unsigned long long m = __ballot(in);
+    if (!m) continue;                               // uniform
+    if (in) s_ck[nl_t + lanes_below(m, lane)] = ((unsigned long long)tk[j] << 32) | (0xffffffffu - (unsigned)t);
+    nl_t += __popcll(m);
   }
   __syncthreads();
+  uint32_t T = 0u;
+  if (nl_t <= kRankList) {
+    for (int i0 = 0; i0 < nl_t; i0 += 64) {
+      const unsigned long long x = s_ck[min(i0 + lane, nl_t - 1)];
+      const int rank = rank_in(s_ck, nl_t, x);
+      if (i0 + lane < nl_t && rank < k_top) {
+        s_tile[rank] = (int)(0xffffffffu - (unsigned)x);
+        if (rank == k_top - 1) s_T = (uint32_t)(x >> 32);
+      }
+    }
+    __syncthreads();
+    T = s_T;
+  } else {
+    // ---- T: the largest key value reached by at least k tiles
+    for (int bit = 31; bit >= 0; --bit) {
+      const uint32_t cand = T | (1u << bit);
+      int cnt = 0;
+#pragma unroll
+      for (int j = 0; j < TPL; ++j) cnt += __popcll(__ballot(tk[j] >= cand));
+      if (cnt >= k_top) T = cand;
+    }
+    int need = k_top;
+#pragma unroll
+    for (int j = 0; j < TPL; ++j) need -= __popcll(__ballot(tk[j] > T));
+    // ---- the chosen tiles, in tile order: above T, then equal to T while need lasts
+    int nt = 0;
+#pragma unroll
+    for (int j = 0; j < TPL; ++j) {
+      const unsigned long long meq = __ballot(tk[j] == T);
+      const bool take = tk[j] > T || (tk[j] == T && lanes_below(meq, lane) < need);
+      need -= min(need, __popcll(meq));
+      const unsigned long long mt = __ballot(take);
+      if (take) s_tile[nt + lanes_below(mt, lane)] = j * 64 + lane;
+      nt += __popcll(mt);
+    }
+    __syncthreads();
+  }
   // ---- candidates: column lane of every chosen tile whose key (head) reaches T's (every
   // tile's value is requested before any is used: one round of loads)
   uint32_t cv[kMaxTop];
@@ -323,6 +374,21 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
     }
     __syncthreads();
   }
+  int32_t* sr = sel + (long)row * sel_stride;
+  if (lane < ns) sr[lane] = lane;
+  if (lane < nl) sr[ns + lane] = n - nl + lane;
+  if (nc <= kRankList) {
+    for (int i0 = 0; i0 < nc; i0 += 64) {
+      const unsigned long long x = s_ck[min(i0 + lane, nc - 1)];
+      const int rank = rank_in(s_ck, nc, x);
+      if (i0 + lane < nc && rank < k_top) {
+        const int pos = (int)(0xffffffffu - (unsigned)x);
+        sr[ns + nl + rank] = pos;
+        mark_selected<HEADS>(Sv, s_stride, row, pos);
+      }
+    }
+    return;
+  }
   // ---- the k-th largest candidate key: 32 score bits, then the position bits (positions are
   // below 2^24, so bits 24..31 of ~position are all ones)
   unsigned long long T2 = 0xff000000ull;
@@ -341,9 +407,6 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
     nw += __popcll(m);
   }
   __syncthreads();
-  int32_t* sr = sel + (long)row * sel_stride;
-  if (lane < ns) sr[lane] = lane;
-  if (lane < nl) sr[ns + lane] = n - nl + lane;
   if (lane < k_top) {
     const unsigned long long x = s_win[lane];
     int rank = 0;
@@ -364,9 +427,10 @@ __global__ void __launch_bounds__(64) topk_select_reg_kernel(void* __restrict__ 
                                                              long sel_stride,
                                                              const int* __restrict__ n_dev, int ns,
                                                              int nl, int k_top, Rescore rs) {
+  __shared__ __align__(16) unsigned long long s_list[kTopList];
   const int row = oa::xcd_row(blockIdx.x, gridDim.x);   // a KV row's query rows share one L2
   topk_reg_row<TPL, KR, HEADS>(Sv, s_stride, TM, tm_stride, ntiles, sel, sel_stride,
-                               *n_dev + oa::row_extra(row, rs.qsh), ns, nl, k_top, rs, row, threadIdx.x);
+                               *n_dev + oa::row_extra(row, rs.qsh), ns, nl, k_top, rs, row, threadIdx.x, s_list);
 }
 
 }  // namespace

@@ -604,6 +604,52 @@ def test_topk_rows_with_ties_large_k(n, k):
     assert np.array_equal(after, marked)
 
 
+@pytest.mark.parametrize("n,k", [(64, 1), (640, 9), (4096, 16), (36864, 9), (36929, 16), (131072, 17), (262000, 64)])
+def test_topk_lists_and_their_overflow(n, k):
+    """The ranked lists of tiles and candidates against the restatement where they are short, just fit
+    (64 and 256 keys) and just do not, over fp32 rows and over key heads: rows with that many equal tile
+    maxima, all of the best scores in one tile, several equal scores in each best tile, fewer than k
+    scores above -inf, and codes of three distinct tokens (every score tied)."""
+    print(f"[case] topk lists n={n} k={k}", flush=True)
+    rng = np.random.default_rng(n + k)
+    ns, nl, R = 1, 2, 8
+    ncols = -(-(n + 30) // 64) * 64
+    nt = ncols // 64
+    S = rng.normal(size=(R, ncols)).astype(np.float32)
+    for r, m in ((1, 64), (2, 65), (3, 256), (4, 257)):
+        S[r, rng.permutation(nt)[:m] * 64 + 7] = 50.0
+    S[5, 64 * (nt // 2):64 * (nt // 2) + 64] += 100.0
+    for t in rng.permutation(nt)[:k + 2]:
+        S[6, t * 64 + 5:t * 64 + 13] = 60.0
+    S[7, k // 2 + 1:] = -np.inf
+    S[:, :ns] = -np.inf
+    S[:, n - nl:] = -np.inf
+    want = O.topk_select(S, n, ns, nl, k)
+    sel = torch.empty(R, ns + nl + k, device=DEV, dtype=torch.int32)
+    n_dev = torch.tensor([n], device=DEV, dtype=torch.int32)
+    St = torch.from_numpy(S).to(DEV)
+    ops.topk_select(St, St.view(R, nt, 64).amax(2), sel, n_dev, ns, nl, k)
+    assert np.array_equal(sel.cpu().numpy(), want)
+
+    codes = rng.integers(-127, 128, (2, ncols, 32), dtype=np.int8)
+    codes[1] = codes[1, rng.integers(0, 3, ncols)]
+    codes[:, n:] = 0
+    U = rng.normal(size=(2, D, 32)).astype(np.float32)
+    scale = rng.uniform(0.5, 2.0, (2, 32)).astype(np.float32)
+    q16 = f32_to_bf16(rng.normal(size=(2 * G, D)).astype(np.float32))
+    _, fexp_ref, Z = O.qgs_prep(q16, U, scale, G)
+    want = O.topk_select(O.qgs_scores(codes, Z, fexp_ref, G, n, ns, nl), n, ns, nl, k)
+    limbs = torch.zeros(2, 16, 32, device=DEV, dtype=torch.int8)
+    fexp = torch.zeros(2 * G, device=DEV, dtype=torch.int32)
+    ops.qgs_prep(np_bf16(q16, DEV), _f32(U), _f32(scale), limbs, fexp)
+    H = torch.empty(2 * G, ncols, device=DEV, dtype=torch.int16)
+    TM = torch.empty(2 * G, nt, device=DEV)
+    codes_t = torch.from_numpy(codes).to(DEV)
+    ops.qgs_scan_heads(codes_t, limbs, fexp, H, TM, n_dev, ns, nl)
+    ops.topk_select_heads(H, TM, sel, n_dev, ns, nl, k, codes_t, limbs, fexp)
+    assert np.array_equal(sel.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("Lmax,n,ns,nl,k", [
     (140000, 12, 3, 3, 20),      # radix kernel (k > 16, 2188 tiles): 6 live positions for 20
     (140000, 500, 3, 3, 0),      # radix kernel at k = 0: sink and local only
