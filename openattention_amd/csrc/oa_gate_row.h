@@ -79,31 +79,6 @@ __device__ __forceinline__ void gate_dots(const GateArgs& a, float sk_lo, float 
   *nt_out = nt;
 }
 
-// wave_sum of NB (4 or 8) values at once: lane l ends with the sum of p[l % NB].  The levels m = 1, 2
-// (and 4) halve the number of values instead of leaving two lanes with the same one: a lane keeps the
-// value its bit selects and adds its partner's copy of it, the sum the butterfly forms (addition is
-// commutative), in NB + 2 additions where NB butterflies take 6 NB.
-__device__ __forceinline__ float lane_xor4(float v) {
-  const int b = __float_as_int(v);
-  const int lo = __builtin_amdgcn_update_dpp(b, b, 0x104, 0xf, 0x5, false);    // row_shl:4 into quads 0, 2
-  return __int_as_float(__builtin_amdgcn_update_dpp(lo, b, 0x114, 0xf, 0xa, false));   // row_shr:4 into 1, 3
-}
-template <int NB>
-__device__ __forceinline__ float wave_sums(const float (&p)[NB], int lane) {
-  static_assert(NB == 4 || NB == 8, "values per batch");
-  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
-  float t[NB / 2], u[NB / 4];
-#pragma unroll
-  for (int k = 0; k < NB / 2; ++k)
-    t[k] = (b0 ? p[2 * k + 1] : p[2 * k]) + oa::dpp_f32<0xB1>(b0 ? p[2 * k] : p[2 * k + 1]);
-#pragma unroll
-  for (int k = 0; k < NB / 4; ++k)
-    u[k] = (b1 ? t[2 * k + 1] : t[2 * k]) + oa::dpp_f32<0x4E>(b1 ? t[2 * k] : t[2 * k + 1]);
-  float v = NB == 8 ? (b2 ? u[NB / 4 - 1] : u[0]) + lane_xor4(b2 ? u[0] : u[NB / 4 - 1]) : u[0] + lane_xor4(u[0]);
-  v = v + oa::dpp_f32<0x128>(v);                   // row_ror:8, m = 8
-  return oa::swap32_sum(oa::swap16_sum(v));
-}
-
 // gate_dots with an empty mask of NB clusters together: lane l holds cluster l % NB's n_c in nt and
 // ends with that cluster's values.  The same arithmetic bit for bit: the divisions by n_c share one
 // reciprocal per cluster, formed by its lane, and the sums over the dimensions come from wave_sums.
@@ -138,9 +113,9 @@ __device__ __forceinline__ void gate_dots_batch(const GateArgs& a, const float (
     pz[i] = fmaf(q_hi, kb_hi, q_lo * kb_lo);
     ps[i] = fmaf(qq_hi, v_hi, qq_lo * v_lo);
   }
-  *qsk_out = wave_sums<NB>(pq, lane);
-  *zbar_out = a.sc * wave_sums<NB>(pz, lane);
-  *s2_out = a.sc2 * wave_sums<NB>(ps, lane);
+  *qsk_out = oa::wave_sums<NB>(pq, lane);
+  *zbar_out = a.sc * oa::wave_sums<NB>(pz, lane);
+  *s2_out = a.sc2 * oa::wave_sums<NB>(ps, lane);
 }
 
 // the scalar tail of one cluster's wl1 score

@@ -38,22 +38,19 @@ __device__ __forceinline__ void index_codes_row(const IdxArgs& a, int r, int lan
   const float k_lo = oa::bf16_to_f32(kp[lane]), k_hi = oa::bf16_to_f32(kp[lane + 64]);
   if (r % a.G == 0) {
     const float* Ub = a.U + (long)kvr * OA_D * RQ;
-    float ul[RQ], uh[RQ];
+    float p[RQ], uh[RQ];
 #pragma unroll
     for (int j = 0; j < RQ; j += 4) {
       const float4 x = *reinterpret_cast<const float4*>(Ub + lane * RQ + j);
       const float4 y = *reinterpret_cast<const float4*>(Ub + (lane + 64) * RQ + j);
-      ul[j] = x.x; ul[j + 1] = x.y; ul[j + 2] = x.z; ul[j + 3] = x.w;
+      p[j] = x.x; p[j + 1] = x.y; p[j + 2] = x.z; p[j + 3] = x.w;
       uh[j] = y.x; uh[j + 1] = y.y; uh[j + 2] = y.z; uh[j + 3] = y.w;
     }
-    int8_t mycode = 0;
+    const float sc = a.scale[(long)kvr * RQ + lane % RQ];
 #pragma unroll
-    for (int j = 0; j < RQ; ++j) {
-      const float zc = oa::dot128_canon(k_lo, ul[j], k_hi, uh[j]);
-      float code = rintf(zc / a.scale[(long)kvr * RQ + j]);
-      code = fminf(fmaxf(code, -127.f), 127.f);
-      if (lane == j) mycode = (int8_t)(int)code;
-    }
+    for (int j = 0; j < RQ; ++j) p[j] = fmaf(k_hi, uh[j], k_lo * p[j]);
+    const float code = rintf(oa::wave_sums<RQ>(p, lane) / sc);
+    const int8_t mycode = (int8_t)(int)fminf(fmaxf(code, -127.f), 127.f);
     if (lane < RQ) a.codes[((long)kvr * a.Lmax_codes + pos) * RQ + lane] = mycode;
   }
 }
@@ -82,12 +79,14 @@ __device__ __forceinline__ void index_assign_row(const IdxArgs& a, int r, int la
     const float4 x = *reinterpret_cast<const float4*>(cb + (long)min(lane, a.C - 1) * RC + j);
     c0[j] = x.x; c0[j + 1] = x.y; c0[j + 2] = x.z; c0[j + 3] = x.w;
   }
+  // the canonical dot products: component lane % 16 in the lane, then all 16 read into scalars
+  const float cm = a.colmean[(long)r * RC + lane % RC];
   float zp[RC];
 #pragma unroll
-  for (int j = 0; j < RC; ++j) {
-    const float d = oa::dot128_canon(k_lo, wl[j], k_hi, wh[j]);
-    zp[j] = oa::bf16_round(d) - a.colmean[(long)r * RC + j];
-  }
+  for (int j = 0; j < RC; ++j) wl[j] = fmaf(k_hi, wh[j], k_lo * wl[j]);
+  const float zl = oa::bf16_round(oa::wave_sums<RC>(wl, lane)) - cm;
+#pragma unroll
+  for (int j = 0; j < RC; ++j) zp[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(zl), j));
   float best = -INFINITY;
   int bidx = 0x7fffffff;
   for (int c = lane; c < a.C; c += 64) {

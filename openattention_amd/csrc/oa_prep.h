@@ -25,23 +25,19 @@ __device__ __forceinline__ void qgs_prep_row(const uint16_t* __restrict__ q, lon
   const float q_hi = bf16_to_f32(q[(long)row * q_stride + lane + 64]);
   const float* Ub = U + (long)(kvr >> qsh) * OA_D * RQ;
   // lane l holds rows l and l+64 of U (32 contiguous floats each)
-  float ul[RQ], uh[RQ], sc[RQ];
+  float p[RQ], uh[RQ];
 #pragma unroll
   for (int j = 0; j < RQ; j += 4) {
     const float4 a = *reinterpret_cast<const float4*>(Ub + lane * RQ + j);
     const float4 b = *reinterpret_cast<const float4*>(Ub + (lane + 64) * RQ + j);
-    ul[j] = a.x; ul[j + 1] = a.y; ul[j + 2] = a.z; ul[j + 3] = a.w;
+    p[j] = a.x; p[j + 1] = a.y; p[j + 2] = a.z; p[j + 3] = a.w;
     uh[j] = b.x; uh[j + 1] = b.y; uh[j + 2] = b.z; uh[j + 3] = b.w;
   }
+  const float sc = scale[(long)(kvr >> qsh) * RQ + lane % RQ];
+  // the canonical dot products (dot128_canon's terms), component lane % 32 left in the lane
 #pragma unroll
-  for (int j = 0; j < RQ; ++j) sc[j] = scale[(long)(kvr >> qsh) * RQ + j];
-  float myz = 0.f;
-#pragma unroll
-  for (int j = 0; j < RQ; ++j) {
-    const float d = dot128_canon(q_lo, ul[j], q_hi, uh[j]);
-    const float z = d * sc[j];
-    if (lane == j) myz = z;
-  }
+  for (int j = 0; j < RQ; ++j) p[j] = fmaf(q_hi, uh[j], q_lo * p[j]);
+  const float myz = wave_sums<RQ>(p, lane) * sc;
   float a = (lane < RQ) ? fabsf(myz) : 0.f;
   float emax = wave_max(a);
   int F = 0;
