@@ -48,6 +48,7 @@
 // global memory (L2 / Infinity Cache) in each pass.  Rows are read in groups of four
 // positions, so both row strides are multiples of 4 and hold round_up(Lmax, 4) entries.
 #include <algorithm>
+#include <type_traits>
 
 #include "oa_common.h"
 #include "oa_score.h"
@@ -249,13 +250,13 @@ __device__ __forceinline__ void scan_row(const int* row, int j, RowScan<BPT>& r)
 }
 // the same over one of the linear-bin kernel's rows of 16 * BPT bins without pad words: thread j
 // holds bins [j*BPT, (j+1)*BPT); bin 0 (non-members) counts nothing
-template <int BPT>
-__device__ __forceinline__ void scan_row_dense(const int* row, int j, RowScan<BPT>& r) {
-  const int* h = row + j * BPT;
+template <int BPT, class T>
+__device__ __forceinline__ void scan_row_dense(const T* row, int j, RowScan<BPT>& r) {
+  const T* h = row + j * BPT;
   r.ls = 0;
 #pragma unroll
   for (int b = 0; b < BPT; ++b) {
-    r.x[b] = (b == 0 && j == 0) ? 0 : h[b];
+    r.x[b] = (b == 0 && j == 0) ? 0 : (int)h[b];
     r.ls += r.x[b];
   }
   int v = r.ls;
@@ -900,7 +901,7 @@ __global__ void __launch_bounds__(kThreads) topq_marked_kernel(TopqArgs a) {
 // HEADS: the score rows hold 16-bit key heads (oa_qgs_scan_heads), which are all the kernel
 // keeps of a score anyway; exact scores come from the codes (oa::qgs_score).
 // Returns true for a row it leaves to the key-prefix algorithm (marked kRowMarked).
-template <int PPT, int LB, bool HEADS, bool TILE>
+template <int PPT, int LB, bool N16, bool HEADS, bool TILE>
 __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, unsigned long long* dyn) {
   static_assert(HEADS || !TILE, "the tile range comes with the head rows");
   __shared__ int s_w[kMaxC];
@@ -923,6 +924,10 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
   constexpr int NB = 1 << LB;
   constexpr int HS = NB + 16;
   constexpr int bpt = HS / 16;
+  // N16: a row of one segment (at most 36864 positions) counts in 16 bits, two bins per word: more bins
+  // than 32-bit counts in the same LDS, and so fewer members in a boundary bin
+  static_assert(!N16 || PPT <= 36, "16-bit counts hold one segment");
+  typedef uint16_t __attribute__((may_alias)) count16;
   int* s_hist = reinterpret_cast<int*>(dyn);                                  // hwords
   unsigned long long* s_g = reinterpret_cast<unsigned long long*>(s_hist);    // after T1
   int* s_out = s_hist;                                                        // after P5
@@ -1048,7 +1053,7 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
     s_t[c] = 0; s_above[c] = 0; s_bcnt[c] = 0; s_klo[c] = 0u; s_khi[c] = ~0u;
     s_sel[c] = 0xffffffffu; s_mode[c] = kModeNone; s_goff[c] = 0; s_gcur[c] = 0; s_ccur[c] = 0;
   }
-  for (int i = tid; i < (C * HS) / 4; i += kThreads) reinterpret_cast<int4*>(s_hist)[i] = make_int4(0, 0, 0, 0);
+  for (int i = tid; i < (C * HS) / (N16 ? 8 : 4); i += kThreads) reinterpret_cast<int4*>(s_hist)[i] = make_int4(0, 0, 0, 0);
   if (tid == 0) { s_gused = 0; s_fail = a.force_mark; }
   if (HEADS && tid < 32) s_lw[tid] = lwv;
 
@@ -1119,6 +1124,10 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
   // positions wholly past n are skipped (uniform); in the group holding n the positions past it
   // (clamped loads: copies of one cluster id) count in per-lane trash words, not all in one bin 0
   const int trash = C * HS + lane;
+  auto count = [&](int i) {
+    if (!N16) atomicAdd(&s_hist[i], 1);
+    else atomicAdd(&s_hist[i >> 1], 1 << ((i & 1) * 16));
+  };
   for (int sg = 0; sg < nseg; ++sg) {
     // with the tile range the row's t are formed here, group by group as the loads arrive
     if (TILE ? sg > 0 : nseg > 1) issue(sg);
@@ -1140,8 +1149,8 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
           a0 = b0 ? a0 : trash;
           a1 = b1 ? a1 : trash;
         }
-        atomicAdd(&s_hist[a0], 1);
-        atomicAdd(&s_hist[a1], 1);
+        count(a0);
+        count(a1);
         if (!kMulti) kh[j] = (uint32_t)b0 | ((uint32_t)b1 << 16);
       }
     }
@@ -1155,7 +1164,8 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
     const int j = tid & 15;
     const int w = c < C ? s_w[c] : 0;
     RowScan<bpt> r;
-    scan_row_dense(s_hist + min(c, C - 1) * HS, j, r);
+    if (!N16) scan_row_dense(s_hist + min(c, C - 1) * HS, j, r);
+    else scan_row_dense(reinterpret_cast<const count16*>(s_hist) + min(c, C - 1) * HS, j, r);
     const int m = __shfl(r.sfx, 0, 16);
     if (c < C && w > 0) {
       const int t = min(w, m);
@@ -1252,21 +1262,21 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
   return false;
 }
 
-template <int PPT, int LB, bool HEADS, bool TILE>
+template <int PPT, int LB, bool N16, bool HEADS, bool TILE>
 // up to 64 VGPRs for the single-segment instantiations: two workgroups (rows) per unit
 __global__ void __launch_bounds__(kThreads, PPT <= 36 ? 8 : 4) topq_linear_kernel(TopqArgs a) {
   extern __shared__ unsigned long long dyn[];
-  topq_linear_body<PPT, LB, HEADS, TILE>(a, blockIdx.x, dyn);
+  topq_linear_body<PPT, LB, N16, HEADS, TILE>(a, blockIdx.x, dyn);
 }
 
 // Fewer rows than compute units (one workgroup per unit, so its LDS and registers are free):
 // the linear-bin algorithm and, on a row it cannot finish, the key-prefix algorithm in the same
 // workgroup, instead of a second launch over every row.  lin and pre are the two algorithms'
 // arguments (LDS layouts); the dynamic LDS holds either's.
-template <int PPT, int LB, int PLB, bool TILE>
+template <int PPT, int LB, bool N16, int PLB, bool TILE>
 __global__ void __launch_bounds__(kThreads) topq_small_kernel(TopqArgs lin, TopqArgs pre) {
   extern __shared__ unsigned long long dyn[];
-  if (topq_linear_body<PPT, LB, true, TILE>(lin, blockIdx.x, dyn)) {   // uniform
+  if (topq_linear_body<PPT, LB, N16, true, TILE>(lin, blockIdx.x, dyn)) {   // uniform
     // the row's exact scores (S32) written above are read back by every wave
     __threadfence();
     __syncthreads();
@@ -1294,21 +1304,23 @@ int launch_lb(const TopqArgs& a, int rows, int Lmax, size_t lds, hipStream_t s) 
   return launch_row<44, LB>(a, rows, lds, s);
 }
 
-template <int PPT, int LB, bool HEADS, bool TILE>
+template <int PPT, int LB, bool N16, bool HEADS, bool TILE>
 int launch_linear(const TopqArgs& a, int rows, size_t lds, hipStream_t s) {
-  const hipError_t e = hipFuncSetAttribute((const void*)topq_linear_kernel<PPT, LB, HEADS, TILE>,
+  const hipError_t e = hipFuncSetAttribute((const void*)topq_linear_kernel<PPT, LB, N16, HEADS, TILE>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL((topq_linear_kernel<PPT, LB, HEADS, TILE>), dim3(rows), dim3(kThreads), lds, s, a);
+  hipLaunchKernelGGL((topq_linear_kernel<PPT, LB, N16, HEADS, TILE>), dim3(rows), dim3(kThreads), lds, s, a);
   return OA_LAUNCH_STATUS();
 }
 
-template <int LB, bool HEADS, bool TILE>
+template <int LB, bool N16, bool HEADS, bool TILE>
 int launch_linear_lb(const TopqArgs& a, int rows, int Lmax, size_t lds, hipStream_t s) {
-  if (Lmax <= kThreads * 8) return launch_linear<8, LB, HEADS, TILE>(a, rows, lds, s);
-  if (Lmax <= kThreads * 16) return launch_linear<16, LB, HEADS, TILE>(a, rows, lds, s);
-  if (Lmax <= kThreads * 36) return launch_linear<36, LB, HEADS, TILE>(a, rows, lds, s);
-  return launch_linear<44, LB, HEADS, TILE>(a, rows, lds, s);
+  if constexpr (LB == 7 || N16) {
+    if (Lmax <= kThreads * 8) return launch_linear<8, LB, N16, HEADS, TILE>(a, rows, lds, s);
+    if (Lmax <= kThreads * 16) return launch_linear<16, LB, N16, HEADS, TILE>(a, rows, lds, s);
+    if (N16 || Lmax <= kThreads * 36) return launch_linear<36, LB, N16, HEADS, TILE>(a, rows, lds, s);
+  }
+  if constexpr (!N16) return launch_linear<44, LB, false, HEADS, TILE>(a, rows, lds, s);
 }
 
 // The one-launch kernel holds both algorithms' static LDS; the key-prefix algorithm's gathered
@@ -1316,9 +1328,9 @@ int launch_linear_lb(const TopqArgs& a, int rows, int Lmax, size_t lds, hipStrea
 // LDS (hipFuncGetAttributes).  Returns kNotLaunched when the list would be too short to run the
 // key-prefix algorithm in the same workgroup: the caller then takes two launches.
 constexpr int kNotLaunched = -1001;
-template <int PPT, int LB, int PLB, bool TILE>
+template <int PPT, int LB, bool N16, int PLB, bool TILE>
 int launch_small(const TopqArgs& lin, TopqArgs pre, int rows, size_t lds_lin, hipStream_t s) {
-  const void* fn = (const void*)topq_small_kernel<PPT, LB, PLB, TILE>;
+  const void* fn = (const void*)topq_small_kernel<PPT, LB, N16, PLB, TILE>;
   hipFuncAttributes fa;
   const hipError_t ea = hipFuncGetAttributes(&fa, fn);
   if (ea != hipSuccess) return (int)ea;
@@ -1331,15 +1343,15 @@ int launch_small(const TopqArgs& lin, TopqArgs pre, int rows, size_t lds_lin, hi
   if ((long)lds + (long)fa.sharedSizeBytes > kLdsLimit) return kNotLaunched;
   const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL((topq_small_kernel<PPT, LB, PLB, TILE>), dim3(rows), dim3(kThreads), lds, s, lin, pre);
+  hipLaunchKernelGGL((topq_small_kernel<PPT, LB, N16, PLB, TILE>), dim3(rows), dim3(kThreads), lds, s, lin, pre);
   return OA_LAUNCH_STATUS();
 }
-template <int LB, int PLB, bool TILE>
+template <int LB, bool N16, int PLB, bool TILE>
 int launch_small_ppt(const TopqArgs& lin, const TopqArgs& pre, int rows, int Lmax, size_t lds_lin,
                      hipStream_t s) {
-  if (Lmax <= kThreads * 8) return launch_small<8, LB, PLB, TILE>(lin, pre, rows, lds_lin, s);
-  if (Lmax <= kThreads * 16) return launch_small<16, LB, PLB, TILE>(lin, pre, rows, lds_lin, s);
-  return launch_small<36, LB, PLB, TILE>(lin, pre, rows, lds_lin, s);
+  if (Lmax <= kThreads * 8) return launch_small<8, LB, N16, PLB, TILE>(lin, pre, rows, lds_lin, s);
+  if (Lmax <= kThreads * 16) return launch_small<16, LB, N16, PLB, TILE>(lin, pre, rows, lds_lin, s);
+  return launch_small<36, LB, N16, PLB, TILE>(lin, pre, rows, lds_lin, s);
 }
 
 }  // namespace
@@ -1371,40 +1383,45 @@ int topq_launch(TopqArgs a, int rows, int C, int Lmax, int E, bool lin, bool hea
   const bool tile = heads && a.TM != nullptr && (Lmax + 63) / 64 <= kTileLd * kThreads;
   if (lin) {
     // linear-bin kernel, dynamic LDS: histogram -> staged keys -> output row | chosen words.
-    // 7 bits for C <= 64, 6 for C <= 128, else 5: two workgroups' LDS fits one unit.  Rows
-    // longer than one register segment run one workgroup per unit anyway (their VGPRs), and
-    // keep 6 bits (smaller boundary bins: fewer rows overflow the staging space)
+    // 7 bits for C <= 64, two workgroups' LDS in one unit.  Above, 16-bit counts (a row of one register
+    // segment) keep 7 bits to C = 128 and 6 to 256 in the LDS of 6 and 5 in 32; longer rows run one
+    // workgroup per unit anyway (their VGPRs) and take 6 bits in 32.  16-bit counts cost three instructions
+    // a position and pay by a smaller boundary bin (fewer keys recomputed, fewer rows that overflow the
+    // staging space): at 1024 rows of 32768 positions, C = 256 and E = 2877 the kernel went from 127 to
+    // 117 us with them, at C = 64 and E = 216 (7 bits either way) from 50 to 53
     TopqArgs al = a;
-    al.lb = C <= 64 ? 7 : (C <= 128 || Lmax > kThreads * 36 ? 6 : 5);
-    al.hwords = (int)((std::max<long>((long)C * ((1 << al.lb) + 16) + 64, a.cpow) + 3) & ~3L);
+    const bool n16 = C > 64 && Lmax <= kThreads * 36;
+    al.lb = C <= 64 || (n16 && C <= 128) ? 7 : 6;
+    const long bins = (long)C * ((1 << al.lb) + 16);
+    al.hwords = (int)((std::max<long>((n16 ? bins / 2 : bins) + 64, a.cpow) + 3) & ~3L);
     al.gcap = al.hwords / 2;
     const size_t lds_lin = 4 * (size_t)al.hwords + 4 * (size_t)a.cpow;
     if (heads && pre && rows < kSmallRows && Lmax <= kThreads * 36) {
       // one launch: the key-prefix algorithm's gathered list shrinks by the linear-bin
       // algorithm's static LDS, which the same workgroup holds (path 3, every row marked, then
       // runs every row through the key-prefix algorithm in this kernel)
-      int st1 = kNotLaunched;
-      if (tile) {
-        if (al.lb == 7 && a.lb == 8) st1 = launch_small_ppt<7, 8, true>(al, a, rows, Lmax, lds_lin, s);
-        else if (al.lb == 6 && a.lb == 7) st1 = launch_small_ppt<6, 7, true>(al, a, rows, Lmax, lds_lin, s);
-        else if (al.lb == 5 && a.lb == 6) st1 = launch_small_ppt<5, 6, true>(al, a, rows, Lmax, lds_lin, s);
-      } else {
-        if (al.lb == 7 && a.lb == 8) st1 = launch_small_ppt<7, 8, false>(al, a, rows, Lmax, lds_lin, s);
-        else if (al.lb == 6 && a.lb == 7) st1 = launch_small_ppt<6, 7, false>(al, a, rows, Lmax, lds_lin, s);
-        else if (al.lb == 5 && a.lb == 6) st1 = launch_small_ppt<5, 6, false>(al, a, rows, Lmax, lds_lin, s);
-      }
+      int st1;
+      if (tile)
+        st1 = a.lb == 8 ? launch_small_ppt<7, false, 8, true>(al, a, rows, Lmax, lds_lin, s)
+              : a.lb == 7 ? launch_small_ppt<7, true, 7, true>(al, a, rows, Lmax, lds_lin, s)
+                          : launch_small_ppt<6, true, 6, true>(al, a, rows, Lmax, lds_lin, s);
+      else
+        st1 = a.lb == 8 ? launch_small_ppt<7, false, 8, false>(al, a, rows, Lmax, lds_lin, s)
+              : a.lb == 7 ? launch_small_ppt<7, true, 7, false>(al, a, rows, Lmax, lds_lin, s)
+                          : launch_small_ppt<6, true, 6, false>(al, a, rows, Lmax, lds_lin, s);
       if (st1 != kNotLaunched) return st1;
     }
     int st;
-    if (tile) st = al.lb == 7 ? launch_linear_lb<7, true, true>(al, rows, Lmax, lds_lin, s)
-                   : al.lb == 6 ? launch_linear_lb<6, true, true>(al, rows, Lmax, lds_lin, s)
-                                : launch_linear_lb<5, true, true>(al, rows, Lmax, lds_lin, s);
-    else if (heads) st = al.lb == 7 ? launch_linear_lb<7, true, false>(al, rows, Lmax, lds_lin, s)
-                    : al.lb == 6 ? launch_linear_lb<6, true, false>(al, rows, Lmax, lds_lin, s)
-                                 : launch_linear_lb<5, true, false>(al, rows, Lmax, lds_lin, s);
-    else st = al.lb == 7 ? launch_linear_lb<7, false, false>(al, rows, Lmax, lds_lin, s)
-              : al.lb == 6 ? launch_linear_lb<6, false, false>(al, rows, Lmax, lds_lin, s)
-                           : launch_linear_lb<5, false, false>(al, rows, Lmax, lds_lin, s);
+    auto linear = [&](auto h, auto t) {
+      constexpr bool hd = decltype(h)::value, tl = decltype(t)::value;
+      if (!n16) return al.lb == 7 ? launch_linear_lb<7, false, hd, tl>(al, rows, Lmax, lds_lin, s)
+                                  : launch_linear_lb<6, false, hd, tl>(al, rows, Lmax, lds_lin, s);
+      return al.lb == 7 ? launch_linear_lb<7, true, hd, tl>(al, rows, Lmax, lds_lin, s)
+                        : launch_linear_lb<6, true, hd, tl>(al, rows, Lmax, lds_lin, s);
+    };
+    st = tile ? linear(std::true_type{}, std::true_type{})
+         : heads ? linear(std::true_type{}, std::false_type{})
+                 : linear(std::false_type{}, std::false_type{});
     if (st || !pre) return st;
     a.marked_only = 1;
   }

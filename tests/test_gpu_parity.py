@@ -482,6 +482,36 @@ def test_topq_deep_histogram_levels(n, C, E, seed, grid, path):
     assert np.array_equal(got, ref), f"rows differ: {np.nonzero((got != ref).any(1))[0]}"
 
 
+@pytest.mark.parametrize("n,C,E", [(8100, 65, 300), (16300, 128, 1000), (36800, 129, 2877), (36560, 256, 4096),
+                                   (36605, 256, 4096)])
+def test_topq_counts_of_one_segment(n, C, E):
+    """Top-q at the cluster counts on either side of the histogram's layouts and at the longest row whose
+    counts are 16 bits: rows with every member in one cluster, in one bin (an equal score, which counts
+    n positions in one bin and leaves the row to the key-prefix kernel) and in two neighbouring bins."""
+    print(f"[case] topq counts n={n} C={C} E={E}", flush=True)
+    rng = np.random.default_rng(n + C)
+    R, Lmax = 5, -(-(n + 260) // 64) * 64
+    S = rng.standard_normal((R, Lmax)).astype(np.float32)
+    asg = rng.integers(0, C, size=(R, Lmax)).astype(np.int32)
+    asg[1:4] = C - 1
+    S[2] = 1.5
+    S[3] = np.where(rng.random(Lmax) < 0.5, 1.0, 2.0)
+    S[4, : n // 2] = 7.0
+    sel = np.stack([rng.choice(n, 16, replace=False) for _ in range(R)]).astype(np.int32)
+    for r in range(R):
+        S[r, sel[r]] = -np.inf
+    S[:, n:] = -np.inf
+    quota = rng.integers(0, 2 * max(E // C, 1) + 2, size=(R, C)).astype(np.float32)
+    quota[1:4, C - 1] = E // 2
+    n_dev = torch.tensor([n], device=DEV, dtype=torch.int32)
+    ref = O.topq(S, asg, sel, quota, n, E)
+    got = torch.full((R, E), 12345, device=DEV, dtype=torch.int32)
+    ops.topq(_f32(S), torch.from_numpy(asg.astype(np.uint8)).to(DEV), _f32(quota), got, n_dev, path=0)
+    torch.cuda.synchronize()
+    got = got.cpu().numpy()
+    assert np.array_equal(got, ref), f"rows differ: {np.nonzero((got != ref).any(1))[0]}"
+
+
 @pytest.mark.parametrize("n,C,E,seed", [(32768, 64, 216, 11), (30000, 128, 700, 12), (50000, 256, 2000, 13)])
 def test_topq_linear_bins_and_marked_rows(n, C, E, seed):
     """The linear-bin kernel alone (path 2) on Gaussian scores resolves every row and equals the
