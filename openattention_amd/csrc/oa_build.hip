@@ -20,8 +20,9 @@
 //   codes    zc_r = fma chain over d = 0..127 in fp32 (z = fma(k_d, U_dr, z), from z = 0);
 //   colmean  per 64-token tile an fp64 sum in a fixed lane order, the tiles summed in order,
 //            then one rounding of sum / T to fp32;
-//   update   per cluster an fp64 sum of the members in position order, one rounding of
-//            sum / count to fp32;
+//   update   per cluster an fp64 sum of the members, one rounding of sum / count to fp32: in position
+//            order in oa_kmeans_update, in no fixed order in oa_kmeans_step (an fp64 sum of fp32 terms
+//            of like magnitude drops bits far below the fp32 mean's last one);
 //   sums     per cluster fp64 sums of k, k*k and v over the members in position order, one
 //            rounding to fp32.
 // The two matrix products of the QGC step (k W and zP . c) run on the bf16 matrix cores with

@@ -1053,7 +1053,8 @@ __device__ __forceinline__ bool topq_linear_body(const TopqArgs& a, int row, uns
     s_t[c] = 0; s_above[c] = 0; s_bcnt[c] = 0; s_klo[c] = 0u; s_khi[c] = ~0u;
     s_sel[c] = 0xffffffffu; s_mode[c] = kModeNone; s_goff[c] = 0; s_gcur[c] = 0; s_ccur[c] = 0;
   }
-  for (int i = tid; i < (C * HS) / (N16 ? 8 : 4); i += kThreads) reinterpret_cast<int4*>(s_hist)[i] = make_int4(0, 0, 0, 0);
+  for (int i = tid; i < (C * HS) / (N16 ? 8 : 4); i += kThreads)
+    reinterpret_cast<int4*>(s_hist)[i] = make_int4(0, 0, 0, 0);
   if (tid == 0) { s_gused = 0; s_fail = a.force_mark; }
   if (HEADS && tid < 32) s_lw[tid] = lwv;
 

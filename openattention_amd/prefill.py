@@ -13,9 +13,9 @@ multibin.py:1894):
   a11  codes: oa_qgs_codes (zc = k U, scale = max(max_t |zc| / 127, 1e-12), codes =
        clamp(rint(zc / scale), -127, 127); static_top_k.py:174-181).
   a12  oa_qgc_project (zP = bf16(k W) - colmean on the bf16 matrix cores), then 4 Lloyd
-       iterations of oa_kmeans_assign (bf16 distance bf16(bf16(zP . c) - bf16(|c|^2 / 2)), ties
-       to the lower cluster) and oa_kmeans_update (member means; an empty cluster keeps its
-       initial point) (methods_eager.py:526-547).
+       iterations of oa_kmeans_step (bf16 distance bf16(bf16(zP . c) - bf16(|c|^2 / 2)), ties to
+       the lower cluster; then the member means, an empty cluster keeping its initial point)
+       (methods_eager.py:526-547).
   a13  oa_cluster_build: n_b, sum k, sum k^2, sum v per cluster and the CSR member lists
        (ours_fastbuild.py:293-301).
 The a11-a13 stages run only on the HIP kernels (a tensor on another device raises).  The

@@ -482,6 +482,36 @@ def test_topq_deep_histogram_levels(n, C, E, seed, grid, path):
     assert np.array_equal(got, ref), f"rows differ: {np.nonzero((got != ref).any(1))[0]}"
 
 
+@pytest.mark.parametrize("C", [1, 3, 4, 5, 8, 33, 64, 65, 255])
+def test_errorgate_batches_of_clusters_bit_exact(C):
+    """The ErrorGate's batches of four clusters at ragged cluster counts: empty clusters (zero sums, the
+    dividing path), sums beyond the shared reciprocal's range on both sides, one member, a cluster of
+    selected tokens only; score and tail count equal the restatement bit for bit."""
+    print(f"[case] errorgate batches C={C}", flush=True)
+    rng = np.random.default_rng(C)
+    BH, Lmax, ns = 2, 256, 5
+    R = BH * G
+    q16 = f32_to_bf16(rng.normal(size=(R, D)).astype(np.float32))
+    K16 = f32_to_bf16(rng.normal(size=(BH, Lmax, D)).astype(np.float32))
+    asg = rng.integers(0, C, (R, Lmax)).astype(np.int32)
+    sel = np.stack([rng.choice(Lmax, ns, replace=False) for _ in range(R)]).astype(np.int32)
+    nb = rng.integers(1, 60, (R, C)).astype(np.float32)
+    Sk = (rng.normal(size=(R, C, D)) * nb[..., None]).astype(np.float32)
+    Sk2 = (np.abs(rng.normal(size=(R, C, D))) * nb[..., None]).astype(np.float32)
+    Sk[1], Sk2[1], nb[1] = 0.0, 0.0, 0.0
+    Sk[2, :, ::5] *= np.float32(2.0**-110)
+    Sk[3, :, 7] = np.float32(2.0**105)
+    nb[4] = 1.0
+    nb[5, asg[5, sel[5]]] = 3.0
+    wants, wantn = O.errorgate(q16, K16, asg, sel, Sk, Sk2, nb, G, SC, SC * SC)
+    score = torch.empty(R, C, device=DEV)
+    n_t = torch.empty(R, C, device=DEV)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+    ops.errorgate(np_bf16(q16, DEV), _bf16_dev(K16), dev(asg), dev(sel), dev(Sk), dev(Sk2), dev(nb), score, n_t, SC)
+    assert np.array_equal(n_t.cpu().numpy(), wantn)
+    assert np.array_equal(score.cpu().numpy(), wants, equal_nan=True)
+
+
 @pytest.mark.parametrize("n,C,E", [(8100, 65, 300), (16300, 128, 1000), (36800, 129, 2877), (36560, 256, 4096),
                                    (36605, 256, 4096)])
 def test_topq_counts_of_one_segment(n, C, E):
