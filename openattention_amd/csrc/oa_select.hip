@@ -201,9 +201,6 @@ __global__ void __launch_bounds__(kScanThreads) qgs_scan_gate_kernel(ScanArgs sa
 // sel = [0..ns) ++ [n-nl..n) ++ top, and the selected tokens' scores are set to -inf so the
 // within-cluster top-q ranks them last.
 constexpr int kMaxTilesLds = 4096;   // Lmax <= 262144
-__device__ __forceinline__ int lanes_below(unsigned long long m, int lane) {
-  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-}
 
 // the number of the list's m distinct keys above x; a list of at most kRankList is ranked this way (past
 // it the bit search's fixed cost is the lower one)
@@ -278,7 +275,7 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
     const bool in = t < ntiles && tk[j] >= bound;
     const unsigned long long m = __ballot(in);
     if (!m) continue;                               // uniform
-    if (in) s_ck[nl_t + lanes_below(m, lane)] = ((unsigned long long)tk[j] << 32) | (0xffffffffu - (unsigned)t);
+    if (in) s_ck[nl_t + lanes_below(m)] = ((unsigned long long)tk[j] << 32) | (0xffffffffu - (unsigned)t);
     nl_t += __popcll(m);
   }
   __syncthreads();
@@ -311,10 +308,10 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
 #pragma unroll
     for (int j = 0; j < TPL; ++j) {
       const unsigned long long meq = __ballot(tk[j] == T);
-      const bool take = tk[j] > T || (tk[j] == T && lanes_below(meq, lane) < need);
+      const bool take = tk[j] > T || (tk[j] == T && lanes_below(meq) < need);
       need -= min(need, __popcll(meq));
       const unsigned long long mt = __ballot(take);
-      if (take) s_tile[nt + lanes_below(mt, lane)] = j * 64 + lane;
+      if (take) s_tile[nt + lanes_below(mt)] = j * 64 + lane;
       nt += __popcll(mt);
     }
     __syncthreads();
@@ -344,7 +341,7 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
       q = (uint32_t)(key >> 32) >= T;
     }
     const unsigned long long m = __ballot(q);
-    if (q) s_ck[nc + lanes_below(m, lane)] = HEADS ? (unsigned long long)pos : key;
+    if (q) s_ck[nc + lanes_below(m)] = HEADS ? (unsigned long long)pos : key;
     nc += __popcll(m);
   }
   __syncthreads();
@@ -403,7 +400,7 @@ __global__ void __launch_bounds__(64) topk_select_kernel(void* __restrict__ Sv, 
   for (int i0 = 0; i0 < nc; i0 += 64) {
     const bool w = i0 + lane < nc && s_ck[i0 + lane] >= T2;
     const unsigned long long m = __ballot(w);
-    if (w) s_win[nw + lanes_below(m, lane)] = s_ck[i0 + lane];
+    if (w) s_win[nw + lanes_below(m)] = s_ck[i0 + lane];
     nw += __popcll(m);
   }
   __syncthreads();

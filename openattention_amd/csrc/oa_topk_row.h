@@ -27,15 +27,6 @@ struct Rescore {
   int qsh = 0;                      // question rows per KV row (oa_common.h)
 };
 
-// candidate score of position pos of a query-head row (sink, local and unwritten: -inf)
-template <bool HEADS>
-__device__ __forceinline__ float cand_score(const void* Sv, long s_stride, int row, int pos, int ns,
-                                            int dead_hi, const Rescore& rs, const int* lw,
-                                            double inv) {
-  if (!HEADS) return static_cast<const float*>(Sv)[(long)row * s_stride + pos];
-  if (pos < ns || pos >= dead_hi) return -INFINITY;
-  return oa::qgs_score(rs.codes, rs.lmax, oa::row_kv(row, rs.qsh), pos, lw, inv);
-}
 template <bool HEADS>
 __device__ __forceinline__ void mark_selected(void* Sv, long s_stride, int row, int pos) {
   if (HEADS) static_cast<uint16_t*>(Sv)[(long)row * s_stride + pos] = oa::kNegInfHead;
@@ -51,10 +42,10 @@ __device__ __forceinline__ double load_limbs(const Rescore& rs, int row, int* lw
   return ldexp(1.0, -rs.fexp[row]);
 }
 
-// The wave's list of candidate keys (one per lane at most), in its own 64 LDS words.  lanes_below:
-// the set bits of m below this lane.
+// The wave's list of candidate keys (one per lane at most), in its own 64 LDS words.  lanes_below: the
+// set bits of m below this lane.
 constexpr int kTopList = 64;
-__device__ __forceinline__ int lanes_below_m(unsigned long long m) {
+__device__ __forceinline__ int lanes_below(unsigned long long m) {
   return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 __device__ __forceinline__ void list_sync() {      // one wave's LDS: in order, the compiler told
@@ -64,7 +55,7 @@ __device__ __forceinline__ void list_sync() {      // one wave's LDS: in order, 
 __device__ __forceinline__ void list_push(unsigned long long* list, int& m, bool in, unsigned long long x) {
   const unsigned long long bal = __ballot(in);
   if (!bal) return;                                 // uniform
-  const int i = m + lanes_below_m(bal);
+  const int i = m + lanes_below(bal);
   if (in && i < kTopList) list[i] = x;
   m += __popcll(bal);
 }
