@@ -384,6 +384,10 @@ class OursHIP(Method):
         B, H, Q, _ = q.shape
         if H != HQ or B != self.B or out.shape != q.shape:
             raise ValueError(f"q and out must be ({self.B}, {HQ}, Q, {D})")
+        if not 1 <= n_keys <= self.Lmax:
+            raise ValueError(f"n_keys={n_keys} outside [1, Lmax={self.Lmax}]")
+        if K.shape[0] != B * HKV or K.shape[1] < n_keys or V.shape != K.shape:
+            raise ValueError(f"K, V must be ({B * HKV}, >= n_keys={n_keys}, {D}) with equal shapes")
         counts = self.bud.counts(n_keys)
         ns, nl, k_top = counts
         if n_keys - Q + 1 - ns - nl < k_top:
