@@ -46,6 +46,16 @@ def _dev(*ts: torch.Tensor) -> torch.device:
     return dev
 
 
+def _on(dev: torch.device, *ts: torch.Tensor) -> None:
+    """_dev's checks of further tensors against the device it returned (by index: a step checks 17 of
+    them, on the host path of every eager call)."""
+    i = dev.index
+    for t in ts:
+        if t is not None and t.get_device() != i:
+            _dev(t)
+            raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
+
+
 def _need(cond: bool, msg: str) -> None:
     if not cond:
         raise ValueError(msg)
@@ -428,6 +438,11 @@ def step(K, V, st, n_dev, q, w, sel, out, ns: int, nl: int, k_top: int, sm_scale
     (update False): 2^qshift question rows per sequence, rows laid out ((kv << qshift) + i) * 4 + head
     in q, sel, out and w; stats = (nb, Sk, Sk2, Sv) receives their statistics."""
     dev = _dev(K, V, n_dev, q, w.limbs, w.fexp, w.H, w.TM, w.S, w.score, w.n_t, w.quota, w.exp_idx, sel, out)
+    _on(dev, w.qsk, w.TMn, st.codes, st.asg, st.asg8, st.nb, st.Sk, st.Sk2, st.Sv, st.U, st.scale)
+    if update:
+        _on(dev, st.W, st.colmean, st.cent, st.reclist, st.reccnt)
+    if stats is not None:
+        _on(dev, *stats)
     BH, Lk, _ = K.shape
     Lmax = st.codes.shape[1]
     R, C = st.nb.shape

@@ -4,7 +4,8 @@ import types
 import pytest
 import torch
 
-from openattention_amd.method import OursHIP
+from openattention_amd import ops
+from openattention_amd.method import RMAX, OursHIP
 
 
 def test_rows_step_refuses_keys_past_the_cache():
@@ -25,3 +26,44 @@ def test_rows_step_refuses_keys_past_the_cache():
         with pytest.raises(ValueError, match="n_keys|K, V"):
             rows(*args)
     assert int(n_dev) == 0
+
+
+def _moved(ns, name):
+    """A copy of the namespace with one tensor on the host."""
+    t = getattr(ns, name)
+    return types.SimpleNamespace(**{**vars(ns), name: torch.empty(t.shape, dtype=t.dtype, device="cpu")})
+
+
+@pytest.mark.parametrize("rows", [False, True])
+def test_step_refuses_tensors_on_another_device(rows):
+    """A step whose index, work buffers or row statistics are not on the keys' device raises for each of
+    its tensors before a pointer is taken (stand-in device tensors, which have no pointer to take)."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    ns, nl, k, Lmax = 1, 1, 2, 256
+    with FakeTensorMode():
+        m = OursHIP(types.SimpleNamespace(rho=0.01), 1, Lmax, "cuda", n_layers=1)
+        m.TMn = torch.empty_like(m.TM)
+        st = types.SimpleNamespace(**vars(m.st[0]))
+        w = types.SimpleNamespace(**{f: getattr(m, f) for f in ("limbs", "fexp", "H", "TM", "TMn", "S", "score", "n_t",
+                                                                "quota", "qsk", "exp_idx")})
+        K = torch.empty(8, Lmax, 128, device="cuda", dtype=torch.bfloat16)
+        q = torch.empty(32, 128, device="cuda", dtype=torch.bfloat16)
+        sel = torch.empty(32, ns + nl + k, device="cuda", dtype=torch.int32)
+        n_dev = torch.empty(1, device="cuda", dtype=torch.int32)
+        stats = {f: torch.empty_like(getattr(st, f)) for f in ("nb", "Sk", "Sk2", "Sv")} if rows else {}
+
+        def call(st=st, w=w, stats=stats):
+            ops.step(K, K, st, n_dev, q, w, sel, m.out, ns, nl, k, 0.1, m.E, RMAX, update=not rows, later=int(rows),
+                     stats=tuple(stats.values()) or None)
+
+        used = ["codes", "U", "scale", "asg", "asg8", "nb", "Sk", "Sk2", "Sv"]
+        used += [] if rows else ["W", "colmean", "cent", "reclist", "reccnt"]
+        for f in used:
+            with pytest.raises(RuntimeError, match="HIP device"):
+                call(st=_moved(st, f))
+        for f in vars(w):
+            with pytest.raises(RuntimeError, match="HIP device"):
+                call(w=_moved(w, f))
+        for f in stats:
+            with pytest.raises(RuntimeError, match="HIP device"):
+                call(stats={**stats, f: torch.empty(stats[f].shape, device="cpu")})
