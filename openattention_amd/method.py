@@ -459,8 +459,11 @@ class OursHIP(Method):
                     for j in range(nq - 1, -1, -1):
                         record.append((i0 + j, row(sel, j).clone(), row(w["quota"], j).clone(),
                                        row(w["exp_idx"], j).clone()))
-                if i0 == 0:
+                if i0 == 0:      # the method's own result buffers hold the last row run, row 0, as after a step
                     self.last_sel = row(sel, 0)
+                    for f in ("score", "n_t", "quota", "exp_idx"):
+                        getattr(self, f).copy_(row(w[f], 0))
+                    self.out.copy_(row(o, 0))
         finally:
             n_dev.fill_(n_keys)
         return out

@@ -398,3 +398,28 @@ def test_prefill_attention_keeps_the_general_path():
         o = prefill_attention(a, b, c, 0.1).float()
         assert o.shape == base.shape and torch.isfinite(o).all()
     assert (prefill_attention(q.half(), k.half(), v.half(), 0.1).float() - base).norm() < 1e-2 * base.norm()
+
+
+@pytest.mark.parametrize("B,Q", [(1, 5), (2, 37)])
+def test_question_rows_leave_the_first_rows_results(B, Q):
+    """After a multi-row call the method's result buffers (selection, scores, tail counts, quotas,
+    expanded set, output rows) hold the last row run, row 0: what the same rows run one after the other
+    leave."""
+    print(f"[case] results after question rows B={B} Q={Q}", flush=True)
+    from openattention_amd.method import OursHIP
+    N = 3000
+    K, V, _, qq, _ = synth.make_layer(11, B, N, N, 64, DEV, n_question=max(Q, 8))
+    static = synth.static_metric(1)
+    got = {}
+    for mode in ("fused", "separate"):
+        m = OursHIP(types.SimpleNamespace(rho=0.03), B, N, DEV, n_layers=1, static=static, gate_mode=mode)
+        build_rows(m.st[0], K, V, qq, N, static["M"][0], static["inv_freq"], 1.0, 0)
+        for t in (m.score, m.n_t, m.quota, m.exp_idx, m.out):
+            t.fill_(7)
+        n_dev = torch.zeros(1, device=DEV, dtype=torch.int32)
+        out = torch.empty(B, HQ, Q, D, device=DEV, dtype=torch.bfloat16)
+        m.rows_step(m.st[0], K.view(-1, N, D), V.view(-1, N, D), qq[:, :, :Q].contiguous(), n_dev, N, out)
+        assert torch.equal(m.out.view(B, HQ, D), out[:, :, 0])
+        got[mode] = [t.clone() for t in (m.last_sel, m.score, m.n_t, m.quota, m.exp_idx, m.out)]
+    for a, b in zip(got["fused"], got["separate"]):
+        assert torch.equal(a, b)
