@@ -27,7 +27,12 @@ G = HQ // HKV
 SC = D ** -0.5
 RMAX = 256
 SCAN_TILE = 64
-ROWS_FULL = 1024           # query-head rows of a multi-row call's launch (4 per compute unit)
+# query-head rows of a multi-row call's launch (4 per compute unit).  A batch of more than half of it (17
+# sequences up) leaves one question row to a group, which would copy every cluster's statistics for each
+# row: 16 rows of 32 sequences of 32K tokens took 3.6 ms that way and take 3.0 one after the other with
+# the keys taken back in place (C = 64; 10.5 and 8.4 ms at C = 256); 16 sequences, two rows a group, 1.67
+# ms against 1.97 (4.82 against 4.82 at C = 256)
+ROWS_FULL = 1024
 TOPQ_SEGMENT = 36 * 1024   # positions the top-q kernel holds in registers at once (36 per thread)
 
 
@@ -393,9 +398,10 @@ class OursHIP(Method):
         if n_keys - Q + 1 - ns - nl < k_top:
             raise ValueError(f"{n_keys} keys leave the first of {Q} causal rows too few positions for "
                              f"sink {ns} + local {nl} + top-k {k_top}")
-        if self.fused and self.gate_mode == "fused" and self.groups == 1:
-            return self._rows_grouped(st, K, V, q, n_dev, n_keys, out, record, counts)
-        snap = (st.nb.clone(), st.Sk.clone(), st.Sk2.clone(), st.Sv.clone())
+        sh = self._rows_shift(Q)
+        if sh > 0:
+            return self._rows_grouped(st, K, V, q, n_dev, n_keys, out, record, counts, sh)
+        snap = (st.nb.clone(), st.Sk.clone(), st.Sk2.clone(), st.Sv.clone()) if Q > 1 else ()
         try:
             for i in range(Q - 1, -1, -1):
                 n_i = n_keys - Q + i + 1
@@ -412,7 +418,14 @@ class OursHIP(Method):
             n_dev.fill_(n_keys)
         return out
 
-    def _rows_grouped(self, st, K, V, q, n_dev, n_keys, out, record, counts):
+    def _rows_shift(self, Q: int) -> int:
+        """log2 of the question rows that a launch of a Q-row call takes together (0: one after the
+        other): the most that ROWS_FULL holds."""
+        if not (self.fused and self.gate_mode == "fused" and self.groups == 1):
+            return 0
+        return max(0, min(ROWS_FULL // self.R, Q).bit_length() - 1)
+
+    def _rows_grouped(self, st, K, V, q, n_dev, n_keys, out, record, counts, sh_max):
         """rows_step with the rows taken in groups of a power of two, each group one launch per stage
         over every sequence's rows (ops.step's question rows; every row's statistics formed beside the
         index, which is not changed).  The group is the largest whose rows fill the chip, ROWS_FULL
@@ -421,9 +434,6 @@ class OursHIP(Method):
         B, _, Q, _ = q.shape
         ns, nl, k_top = counts
         NS, C = ns + nl + k_top, self.Cn
-        sh_max = max(0, (max(1, ROWS_FULL // self.R)).bit_length() - 1)
-        while sh_max and (1 << sh_max) > Q:
-            sh_max -= 1
         # work buffers of the largest group, shared by all (a smaller group uses their first rows)
         R = self.R << sh_max
         f32 = dict(device=q.device, dtype=torch.float32)

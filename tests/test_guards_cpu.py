@@ -67,3 +67,24 @@ def test_step_refuses_tensors_on_another_device(rows):
         for f in stats:
             with pytest.raises(RuntimeError, match="HIP device"):
                 call(stats={**stats, f: torch.empty(stats[f].shape, device="cpu")})
+
+
+def test_question_rows_are_grouped_where_a_group_holds_two():
+    """Rows per launch of a multi-row call: the largest power of two that 1024 query-head rows and the
+    call hold; a batch that leaves one row to a launch runs its rows one after the other in place."""
+    for B, want in ((1, 5), (2, 4), (3, 3), (8, 2), (16, 1), (17, 0), (32, 0)):
+        m = OursHIP(types.SimpleNamespace(rho=0.01), B, 128, "meta", n_layers=1)
+        assert m._rows_shift(64) == want
+        assert [m._rows_shift(Q) for Q in (1, 2, 3)] == [0, min(want, 1), min(want, 1)]
+    for kw in (dict(fused=False), dict(gate_mode="separate")):
+        assert OursHIP(types.SimpleNamespace(rho=0.01), 1, 128, "meta", n_layers=1, **kw)._rows_shift(64) == 0
+
+    m = OursHIP(types.SimpleNamespace(rho=0.01), 32, 128, "cpu", n_layers=1)
+    ran = []
+    m.step = lambda st, K, V, q, n_dev, n, counts, update_index: ran.append(n) or m.out
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(ops, "index_downdate", lambda K, V, st, n_dev: ran.append("back"))
+        K = torch.zeros(256, 128, 128, dtype=torch.bfloat16)
+        q = torch.zeros(32, 32, 3, 128, dtype=torch.bfloat16)
+        m.rows_step(m.st[0], K, K, q, torch.zeros(1, dtype=torch.int32), 128, torch.empty_like(q))
+    assert ran == [128, "back", 127, "back", 126]
