@@ -33,6 +33,7 @@ SCAN_TILE = 64
 # the keys taken back in place (C = 64; 10.5 and 8.4 ms at C = 256); 16 sequences, two rows a group, 1.67
 # ms against 1.97 (4.82 against 4.82 at C = 256)
 ROWS_FULL = 1024
+ROWS_BYTES = 1 << 30       # most bytes of a group's work buffers (they grow with the index's capacity)
 TOPQ_SEGMENT = 36 * 1024   # positions the top-q kernel holds in registers at once (36 per thread)
 
 
@@ -420,10 +421,17 @@ class OursHIP(Method):
 
     def _rows_shift(self, Q: int) -> int:
         """log2 of the question rows that a launch of a Q-row call takes together (0: one after the
-        other): the most that ROWS_FULL holds."""
+        other): the most that ROWS_FULL holds and whose work buffers fit ROWS_BYTES.  At 1024 rows and 64
+        clusters those are 0.3 GB at 32K positions, 0.9 GB at 128K; beyond, half the rows: one 128K
+        sequence of 192 clusters, 1.1 GB, 1.42 ms for 64 rows against 1.26, and 9.0 one by one."""
         if not (self.fused and self.gate_mode == "fused" and self.groups == 1):
             return 0
-        return max(0, min(ROWS_FULL // self.R, Q).bit_length() - 1)
+        sh = max(0, min(ROWS_FULL // self.R, Q).bit_length() - 1)
+        row = 6 * self.SW + 4 * self.ntiles * (1 if self.TMn is None else 2)      # H and S, TM and TMn
+        row += 4 * self.Cn * (3 * D + 5) + 4 * self.exp_idx.shape[1]             # statistics and maps, exp_idx
+        while sh and (self.R << sh) * row > ROWS_BYTES:
+            sh -= 1
+        return sh
 
     def _rows_grouped(self, st, K, V, q, n_dev, n_keys, out, record, counts, sh_max):
         """rows_step with the rows taken in groups of a power of two, each group one launch per stage

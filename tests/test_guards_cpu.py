@@ -88,3 +88,26 @@ def test_question_rows_are_grouped_where_a_group_holds_two():
         q = torch.zeros(32, 32, 3, 128, dtype=torch.bfloat16)
         m.rows_step(m.st[0], K, K, q, torch.zeros(1, dtype=torch.int32), 128, torch.empty_like(q))
     assert ran == [128, "back", 127, "back", 126]
+
+
+@pytest.mark.parametrize("rho,Lmax", [(0.01, 32896), (0.10, 32896), (0.01, 131200), (0.10, 131200), (0.01, 262144)])
+def test_question_rows_work_buffers_are_bounded(rho, Lmax):
+    """What a group of question rows allocates stays within its bound whatever the index's capacity, in
+    the largest group that does."""
+    from openattention_amd import method as M
+    m = OursHIP(types.SimpleNamespace(rho=rho), 1, Lmax, "meta", n_layers=1)
+    sh = m._rows_shift(64)
+    got = []
+
+    def bytes_of(st, K, V, n_dev, q, w, sel, *a, stats, **kw):
+        ts = [t for t in vars(w).values() if t is not None] + list(stats)
+        got.append(sum(t.numel() * t.element_size() for t in ts))
+
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(ops, "step", lambda K, V, st, *a, **kw: bytes_of(st, K, V, *a, **kw))
+        q = torch.empty(1, 32, 64, 128, dtype=torch.bfloat16, device="meta")
+        K = torch.empty(8, Lmax, 128, dtype=torch.bfloat16, device="meta")
+        m.rows_step(m.st[0], K, K, q, torch.empty(1, dtype=torch.int32, device="meta"), Lmax, torch.empty_like(q))
+    small = 32 << sh << 10          # limbs, fexp: under 1 KB a row
+    assert max(got) <= M.ROWS_BYTES + small
+    assert sh == 5 or 2 * max(got) + small > M.ROWS_BYTES
