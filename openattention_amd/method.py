@@ -13,6 +13,7 @@ only computes (ns, nl, k_top) from n, which the reference also keys its graphs b
 """
 from __future__ import annotations
 
+import copy
 import types
 
 import torch
@@ -33,6 +34,7 @@ SCAN_TILE = 64
 # the keys taken back in place (C = 64; 10.5 and 8.4 ms at C = 256); 16 sequences, two rows a group, 1.67
 # ms against 1.97 (4.82 against 4.82 at C = 256)
 ROWS_FULL = 1024
+ROWS_WALK = 1024           # keys past which a group's statistics start from those of the group before
 ROWS_BYTES = 1 << 30       # most bytes of a group's work buffers (they grow with the index's capacity)
 TOPQ_SEGMENT = 36 * 1024   # positions the top-q kernel holds in registers at once (36 per thread)
 
@@ -383,9 +385,11 @@ class OursHIP(Method):
         n_i = n_keys - Q + i + 1 keys before it (multibin.py:2210-2218 keeps raw > NEG only);
         the sink / local / top-k sizes come from the call's key count, as the maskers size them
         from seq_len_keys (maskers/base.py:152-158), and the local window ends at the row.
-        The rows run from the last to the first; after row i the key at n_i - 1 leaves the
-        cluster statistics (ops.index_downdate), so row i - 1 sees those of [0, n_{i-1}); the
-        statistics are restored afterwards and n_dev is left at n_keys.  Writes and returns out
+        The rows run from the last to the first, row i over the cluster statistics of [0, n_i): in
+        groups (_rows_grouped), whose statistics are formed beside the index, or, where a launch would
+        hold one row (_rows_shift), one after the other, the key at n_i - 1 leaving the index's own
+        statistics after row i (ops.index_downdate) and these restored afterwards.  Either way the
+        index is left as it was, n_dev at n_keys and the result buffers at row 0's.  Writes and returns out
         (B, HQ, Q, D).  record, when a list, receives (i, sel, quota, exp_idx) copies per row."""
         B, H, Q, _ = q.shape
         if H != HQ or B != self.B or out.shape != q.shape:
@@ -438,7 +442,10 @@ class OursHIP(Method):
         over every sequence's rows (ops.step's question rows; every row's statistics formed beside the
         index, which is not changed).  The group is the largest whose rows fill the chip, ROWS_FULL
         query-head rows: 64 rows of one 32K sequence took 64 chains of 5 launches at 32 of 256 compute
-        units, 5.0 ms of device time (8.9 ms with the host's 600 launches), and take 0.4 ms."""
+        units, 5.0 ms of device time (8.9 ms with the host's 600 launches), and take 0.4 ms.  A group's
+        statistics walk back over the keys after it from those of all keys, or, ROWS_WALK keys on, from
+        a copy of an earlier group's first row: 8192 rows of one sequence 55 ms, and 174 with every walk
+        from the last key."""
         B, _, Q, _ = q.shape
         ns, nl, k_top = counts
         NS, C = ns + nl + k_top, self.Cn
@@ -459,17 +466,19 @@ class OursHIP(Method):
         qr = q.view(B, HKV, G, Q, D).permute(0, 1, 3, 2, 4)
         outr = out.view(B, HKV, G, Q, D).permute(0, 1, 3, 2, 4)
         i0 = Q
+        base, held = st, n_keys       # the statistics the next group starts from, and how many keys they hold
         try:
             while i0 > 0:
                 sh = min(sh_max, i0.bit_length() - 1)
                 nq = 1 << sh
                 i0 -= nq
                 Rg = self.R << sh
-                n_dev.fill_(n_keys - Q + i0 + 1)
+                n_first = n_keys - Q + i0 + 1
+                n_dev.fill_(n_first)
                 wg = types.SimpleNamespace(**{k: None if t is None else t[:Rg if k != "limbs" else Rg // G]
                                               for k, t in w.items()})
-                ops.step(K, V, st, n_dev, qr[:, :, i0:i0 + nq].reshape(Rg, D), wg, sel[:Rg], o[:Rg], ns, nl, k_top,
-                         self.sm_scale, self.E, RMAX, update=False, qshift=sh, later=Q - i0 - nq,
+                ops.step(K, V, base, n_dev, qr[:, :, i0:i0 + nq].reshape(Rg, D), wg, sel[:Rg], o[:Rg], ns, nl, k_top,
+                         self.sm_scale, self.E, RMAX, update=False, qshift=sh, later=held - n_first - nq + 1,
                          stats=tuple(t[:Rg] for t in stats))
                 outr[:, :, i0:i0 + nq] = o[:Rg].view(B, HKV, nq, G, D)
                 row = lambda t, j: t[:Rg].view(B * HKV, nq, G, -1)[:, j].reshape(self.R, -1)  # noqa: E731
@@ -477,6 +486,13 @@ class OursHIP(Method):
                     for j in range(nq - 1, -1, -1):
                         record.append((i0 + j, row(sel, j).clone(), row(w["quota"], j).clone(),
                                        row(w["exp_idx"], j).clone()))
+                if i0 > 0 and held - n_first >= ROWS_WALK:
+                    base = copy.copy(st)
+                    for f, t in zip(("nb", "Sk", "Sk2", "Sv"), stats):
+                        u = torch.empty_like(getattr(st, f))
+                        u.view(B * HKV, G, -1).copy_(t[:Rg].view(B * HKV, nq, G, -1)[:, 0])
+                        setattr(base, f, u)
+                    held = n_first
                 if i0 == 0:      # the method's own result buffers hold the last row run, row 0, as after a step
                     self.last_sel = row(sel, 0)
                     for f in ("score", "n_t", "quota", "exp_idx"):

@@ -423,3 +423,33 @@ def test_question_rows_leave_the_first_rows_results(B, Q):
         got[mode] = [t.clone() for t in (m.last_sel, m.score, m.n_t, m.quota, m.exp_idx, m.out)]
     for a, b in zip(got["fused"], got["separate"]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,N,Q,walk", [(1, 1200, 203, 1024), (1, 1200, 203, 64), (2, 900, 130, 96)])
+def test_question_rows_past_64_keys(B, N, Q, walk, monkeypatch):
+    """More question rows than the 64 cluster ids that a wave takes back at a time, with every group's
+    statistics walked back from the last key and from an earlier group's first row: the same
+    selections, quotas, expanded sets and output bits as the rows one after the other."""
+    print(f"[case] question rows past 64 keys B={B} N={N} Q={Q} walk={walk}", flush=True)
+    from openattention_amd.method import OursHIP
+    monkeypatch.setattr(M, "ROWS_WALK", walk)
+    K, V, _, qq, _ = synth.make_layer(13, B, N, N, 64, DEV, n_question=Q)
+    static = synth.static_metric(1)
+    got = {}
+    for mode in ("fused", "separate"):
+        m = OursHIP(types.SimpleNamespace(rho=0.03), B, N, DEV, n_layers=1, static=static, gate_mode=mode)
+        build_rows(m.st[0], K, V, qq, N, static["M"][0], static["inv_freq"], 1.0, 0)
+        before = m.st[0].to_numpy()
+        n_dev = torch.zeros(1, device=DEV, dtype=torch.int32)
+        out = torch.empty(B, HQ, Q, D, device=DEV, dtype=torch.bfloat16)
+        rec = []
+        m.rows_step(m.st[0], K.view(-1, N, D), V.view(-1, N, D), qq, n_dev, N, out, record=rec)
+        torch.cuda.synchronize()
+        after = m.st[0].to_numpy()
+        assert all(np.array_equal(before[f], after[f]) for f in before)
+        got[mode] = (out, sorted(rec, key=lambda t: t[0]))
+    (o1, r1), (o2, r2) = got["fused"], got["separate"]
+    assert [t[0] for t in r1] == list(range(Q))
+    for a, b in zip(r1, r2):
+        assert all(torch.equal(x, y) for x, y in zip(a[1:], b[1:])), a[0]
+    assert torch.equal(o1, o2)

@@ -111,3 +111,29 @@ def test_question_rows_work_buffers_are_bounded(rho, Lmax):
     small = 32 << sh << 10          # limbs, fexp: under 1 KB a row
     assert max(got) <= M.ROWS_BYTES + small
     assert sh == 5 or 2 * max(got) + small > M.ROWS_BYTES
+
+
+def test_question_rows_walk_back_a_bounded_number_of_keys():
+    """A group's statistics start from those of an earlier group's first row once the walk from the last
+    key would be long: the keys a long call's groups walk over grow with its rows, not with their
+    square, and each group's count fits the statistics it starts from."""
+    from openattention_amd import method as M
+    Q, n_keys = 5000, 6000
+    m = OursHIP(types.SimpleNamespace(rho=0.01), 1, 6016, "meta", n_layers=1)
+    st, n_dev, calls = m.st[0], types.SimpleNamespace(at=[]), []
+    n_dev.fill_ = n_dev.at.append
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(ops, "step", lambda K, V, st, *a, qshift, later, **kw: calls.append((st, qshift, later)))
+        q = torch.empty(1, 32, Q, 128, dtype=torch.bfloat16, device="meta")
+        K = torch.empty(8, n_keys, 128, dtype=torch.bfloat16, device="meta")
+        m.rows_step(st, K, K, q, n_dev, n_keys, torch.empty_like(q))
+    assert n_dev.at[-1] == n_keys and sum(1 << c[1] for c in calls) == Q
+    held, end, last = n_keys, n_keys, st
+    for (base, sh, later), n_first in zip(calls, n_dev.at):
+        if base is not last:         # copied after the group before, from the row that saw `end` keys
+            held, last = end + 1, base
+            assert base.codes is st.codes and base.Sk is not st.Sk and base.Sk.shape == st.Sk.shape
+        assert n_first + (1 << sh) - 1 + later == held and n_first + (1 << sh) - 1 == end
+        end = n_first - 1
+        assert later <= M.ROWS_WALK
+    assert last is not st
