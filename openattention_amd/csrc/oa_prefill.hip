@@ -25,6 +25,7 @@
 // 32 x 32 scores of a wave against 512 matrix cycles.  32768 positions, 32 heads: 9.2 ms, 953 TFLOP/s
 // (a large bf16 product reaches 1326 on this card); the library kernel it replaces took 16.9 ms and
 // another 0.34 ms to expand the KV heads.
+#include <cfloat>
 #include <type_traits>
 
 #include "oa_common.h"
@@ -150,7 +151,8 @@ __global__ void __launch_bounds__(kThreads, 2) prefill_attn_kernel(PrefillArgs a
   for (int d = 0; d < 4; ++d) O[d] = float16v(0.f);
 #pragma unroll
   for (int s = 0; s < 8; ++s) S0 = mfma(key_op(s_k, s), Q[s], S0);
-  float m = -1e30f, l = 0.f;             // running maximum (scaled by c) and sum of the lane's keys
+  float m = -FLT_MAX, l = 0.f;           // running maximum (scaled by c) and sum of the lane's keys
+  bool big = false;                      // a lane's maximum is past 2^24 (uniform)
   oa::lds_barrier();                     // K(0) has been read: its place takes K(2)
 
   // iteration i (parity odd = i & 1): K(i + 1), V(i - 1) are in the other parity's tiles
@@ -196,11 +198,18 @@ __global__ void __launch_bounds__(kThreads, 2) prefill_attn_kernel(PrefillArgs a
           alpha = __builtin_amdgcn_exp2f(m - mn);
           l *= alpha;
           m = mn;
+          // m rounds S c, so that the fma below leaves up to half its last place: past 2^24 more than
+          // the exponential should see, and an infinity in time.  There S c is rounded first, as m is
+          big = __any(fabsf(m) >= 16777216.f);
+        }
+        if (!MASK && big) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) S[r] *= a.c;
         }
       } else {
 #pragma unroll
         for (int r = (s - 2) * 16 / 6; r < (s - 1) * 16 / 6; ++r) {
-          const float p1 = __builtin_amdgcn_exp2f(MASK ? S[r] - m : fmaf(S[r], a.c, -m));
+          const float p1 = __builtin_amdgcn_exp2f(MASK ? S[r] - m : fmaf(S[r], big ? 1.f : a.c, -m));
           l += p1;
           if (r & 1) {                   // (pinned here: left alone they all sink below the products)
             uint32_t w = pack2(p0, p1);

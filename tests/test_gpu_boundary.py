@@ -453,3 +453,39 @@ def test_question_rows_past_64_keys(B, N, Q, walk, monkeypatch):
     for a, b in zip(r1, r2):
         assert all(torch.equal(x, y) for x, y in zip(a[1:], b[1:])), a[0]
     assert torch.equal(o1, o2)
+
+
+@pytest.mark.parametrize("T", [20, 97, 300])
+def test_prefill_attention_of_extreme_scores(T):
+    """Prefill rows whose scores are of any finite size: every score far below -1e30, near -1e16 with equal
+    keys, and 2^20 to 2^60 with one key a row ahead of the rest by more than rounding.  One key or all
+    equal keys hold such a row's weight, so the answer is that key's value or the values' mean."""
+    print(f"[case] prefill attention extreme scores T={T}", flush=True)
+    from openattention_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(T)
+    v = torch.randn(1, 2, T, 128, device=DEV, generator=g).to(torch.bfloat16)
+    one = torch.ones(1, 8, T, 128, device=DEV, dtype=torch.bfloat16)
+    mean = v.double().cumsum(2) / torch.arange(1, T + 1, device=DEV, dtype=torch.float64)[:, None]
+    for a, b in ((1e16, -1e16), (2.0 ** 40, 2.0 ** 70), (2.0 ** 12, 2.0 ** 14), (1.0, -(2.0 ** 30))):
+        q, k = one * a, (one * b)[:, :2].clone()
+        o = ops.prefill_attn(q, k, v, 128 ** -0.5)
+        ref = mean.repeat_interleave(4, 1)
+        assert torch.isfinite(o).all(), (a, b)
+        assert (o.double() - ref).norm() < 1e-2 * ref.norm(), (a, b)
+    for e in (20, 40, 60):
+        # key j's score grows with j: every row's own key takes all the weight
+        k = (one[:, :2].float() * (1 + torch.arange(T, device=DEV)[:, None] / 128)).to(torch.bfloat16)
+        distinct = torch.cat([k.new_ones(1, 2, 1, 128, dtype=torch.bool), k[:, :, 1:] > k[:, :, :-1]], 2).all(-1)
+        for sign in (1, -1):
+            q = one * sign * 2.0 ** e
+            o = ops.prefill_attn(q, k, v, 128 ** -0.5)
+            assert torch.isfinite(o).all(), (e, sign)
+            want = v if sign > 0 else v[:, :, :1].expand_as(v)
+            rows = distinct if sign > 0 else torch.arange(T, device=DEV).expand(1, 2, T) < 1
+            if sign < 0:          # (keys equal to the first in bf16 share its weight)
+                rows = (k[..., 0] > k[:, :, :1, 0]) | rows
+                same = (k[..., 0] == k[:, :, :1, 0]).sum(2, keepdim=True).expand(1, 2, T)
+                rows = rows & (same == 1)
+            got = o.view(1, 2, 4, T, 128)
+            for h in range(4):
+                assert torch.equal(got[:, :, h][rows], want[rows]), (e, sign, h)
