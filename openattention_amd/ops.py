@@ -14,6 +14,8 @@ on a HIP device and the kernel library must be built.
 from __future__ import annotations
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from openattention_amd import lib
 
@@ -609,24 +611,36 @@ def dense_decode(q, K, V, n_dev, out=None, sm_scale: float | None = None, nsplit
     return out
 
 
+def _watched() -> bool:
+    """Whether something on this thread has to see a torch operation that is run now, which a library
+    call would hide from it: a tracer, a dispatch or function mode (a default device is none), autocast
+    to another type."""
+    if (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._ops._len_torch_dispatch_stack_pre_dispatch()
+            or torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16):
+        return True
+    return torch._C._len_torch_function_stack() > 0 and any(
+        not isinstance(m, DeviceContext) for m in _get_current_function_mode_stack())
+
+
 def prefill_attn_ok(q, k, v, sm_scale: float = 1.0) -> bool:
     """Whether prefill_attn takes these arguments: a scale that is not negative (the running maximum is
-    taken before it is applied), plain bf16 HIP tensors of Llama-3.1-8B's head layout,
-    one sequence, rows of dims contiguous, 16-byte aligned, and nothing that would have to see the
-    operation (autograd in either mode, a functional transform, a tracer)."""
-    if (not sm_scale >= 0 or q.dim() != 4 or k.dim() != 4 or q.shape[0] != 1 or k.shape[0] != 1 or k.shape != v.shape
+    taken before it is applied), plain bf16 tensors on the current HIP device, of Llama-3.1-8B's head
+    layout, one sequence, rows of dims contiguous, 16-byte aligned, and nothing that would have to see
+    the operation (autograd in either mode, a functional transform, what _watched names)."""
+    if (sm_scale is None or not sm_scale >= 0 or _watched() or q.dim() != 4 or k.dim() != 4 or q.shape[0] != 1 or k.shape[0] != 1 or k.shape != v.shape
             or q.shape[3] != HEAD_DIM or k.shape[3] != HEAD_DIM or q.shape[1] != GROUP * k.shape[1]
             or q.shape[2] != k.shape[2] or q.shape[2] < 1):
         return False
     for t in (q, k, v):
         if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != torch.bfloat16
-                or t.device.type != "cuda" or t.device != q.device or t.stride(3) != 1
+                or t.device.type != "cuda" or t.device != q.device or t.is_neg() or t.stride(3) != 1
                 or t.stride(1) % 8 or t.stride(2) % 8 or t.stride(2) < HEAD_DIM or t.stride(2) > 1 << 24
                 or torch._C._functorch.is_functorch_wrapped_tensor(t) or t.data_ptr() % 16):
             return False
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
         return False
-    return torch.autograd.forward_ad._current_level < 0 and not torch.compiler.is_compiling()
+    return torch.autograd.forward_ad._current_level < 0 and q.device.index == torch.cuda.current_device()
 
 
 def prefill_attn(q, k, v, sm_scale: float) -> torch.Tensor:

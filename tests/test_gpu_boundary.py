@@ -489,3 +489,73 @@ def test_prefill_attention_of_extreme_scores(T):
             got = o.view(1, 2, 4, T, 128)
             for h in range(4):
                 assert torch.equal(got[:, :, h][rows], want[rows]), (e, sign, h)
+
+
+def test_prefill_attention_is_seen_by_modes():
+    """Dispatch and function modes meet the prefill attention's operation, autocast to another type gives
+    that type, a lazily negated query and a default scale are taken as torch takes them; a default device
+    and bf16 autocast keep the matrix-core kernel."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from openattention_amd import ops
+    from openattention_amd.method import prefill_attention
+    g = torch.Generator(device=DEV).manual_seed(5)
+    other = [torch.randn(1, h, 48, 128, device=DEV, generator=g).to(torch.bfloat16) for h in (8, 2, 2)]
+
+    def f(q, k, v):
+        return prefill_attention(q, k, v, 0.1)
+
+    want = f(*other)
+
+    def same(got):
+        return (got.float() - want.float()).norm() < 1e-2 * want.float().norm()
+
+    names = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            names.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Dispatch, Function):
+        names.clear()
+        with mode():
+            assert same(f(*other))
+        assert any("attention" in n for n in names), (mode, names)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert f(*other).dtype == torch.float16 and same(f(*other))
+    assert same(f(torch._neg_view(-other[0]), *other[1:]))
+    with torch.device(DEV), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert ops.prefill_attn_ok(*other)
+    assert (prefill_attention(*other, None).float() - prefill_attention(*other, 128 ** -0.5).float()).norm() < \
+        1e-2 * want.float().norm()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("T,at", [(31, 30), (200, 131), (200, 199)])
+def test_prefill_attention_with_a_value_that_is_not_finite(bad, T, at):
+    """An infinity or NaN in one value row: the positions before its 32-key tile do not meet it (those of
+    its own tile may, by a weight of 0), those from it on do, and the other dimensions and heads are
+    untouched; in a key row: exactly the positions from it on may change."""
+    print(f"[case] prefill attention with {bad} at {at} of {T}", flush=True)
+    from openattention_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(at)
+    q, k, v = (torch.randn(1, h, T, 128, device=DEV, generator=g).to(torch.bfloat16) for h in (8, 2, 2))
+    base = ops.prefill_attn(q, k, v, 0.1)
+    assert torch.isfinite(base).all()
+    vv, kk = v.clone(), k.clone()
+    vv[0, 1, at, 5] = bad
+    o = ops.prefill_attn(q, k, vv, 0.1)
+    hit = torch.zeros_like(o, dtype=torch.bool)
+    hit[0, 4:, at // 32 * 32:, 5] = True
+    assert torch.equal(o[~hit], base[~hit]) and not torch.isfinite(o[0, 4:, at:, 5]).any()
+    kk[0, 0, at, 7] = bad
+    o = ops.prefill_attn(q, kk, v, 0.1)
+    hit = torch.zeros_like(o, dtype=torch.bool)
+    hit[0, :4, at:] = True
+    assert torch.equal(o[~hit], base[~hit])

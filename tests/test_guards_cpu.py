@@ -137,3 +137,48 @@ def test_question_rows_walk_back_a_bounded_number_of_keys():
         end = n_first - 1
         assert later <= M.ROWS_WALK
     assert last is not st
+
+
+def test_tracers_and_modes_are_noticed():
+    """What follows torch's operations (a tracer, make_fx with its dispatch mode before or after
+    decomposition, a dispatch or function mode, autocast to another type) is noticed, so that the prefill
+    attention stays a torch operation under it; a default device and bf16 autocast are not."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    x, seen = torch.zeros(3), []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    def f(t):
+        seen.append(ops._watched())
+        return t + 1
+
+    f(x)
+    with torch.device("cpu"):
+        f(x)
+    assert seen == [False, False]
+    torch.jit.trace(f, (x,), check_trace=False)
+    make_fx(f)(x)
+    make_fx(f, pre_dispatch=True)(x)
+    with Dispatch():
+        seen.append(ops._watched())
+    with Function(), torch.device("cpu"):
+        seen.append(ops._watched())
+    was, dt = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+    try:
+        torch.set_autocast_enabled("cuda", True)
+        torch.set_autocast_dtype("cuda", torch.float16)
+        seen.append(ops._watched())
+        torch.set_autocast_dtype("cuda", torch.bfloat16)
+        assert not ops._watched()
+    finally:
+        torch.set_autocast_enabled("cuda", was)
+        torch.set_autocast_dtype("cuda", dt)
+    assert len(seen) == 8 and all(seen[2:])
