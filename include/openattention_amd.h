@@ -390,6 +390,15 @@ int oa_qgc_project(const void* K, long k_stride_h, long k_stride_t, int rows, in
                    uint16_t* zraw_out, void* stream);
 
 /*
+ * oa_qgc_project which also writes each column's bound word for oa_kmeans_step_max: zmax (rows, 16), the
+ * fp32 bits of its largest |bf16(k W)|, with the sign bit set (and those of the largest bf16) where one
+ * is not finite.  max_ws: rows * ceil(T / 512) * 16 words of scratch.
+ */
+int oa_qgc_project_max(const void* K, long k_stride_h, long k_stride_t, int rows, int G, int T,
+                       const void* W, float* zP, long zp_stride, float* colmean, double* tile_ws,
+                       uint16_t* zraw_out, uint32_t* max_ws, uint32_t* zmax, void* stream);
+
+/*
  * k-means assignment: asg_t = argmax_c bf16(bf16(bf16(zP_t) . bf16(c)) - bf16(|c|^2 / 2)), ties
  * to the lower cluster, written as int32 and uint8; zP_t = zraw_t - colmean (fp32, formed from
  * the stored bf16 projection).  zraw (rows, z_stride) as oa_qgc_project writes it; cent
@@ -401,15 +410,22 @@ int oa_kmeans_assign(const uint16_t* zraw, const float* colmean, long z_stride, 
                      long asg8_stride, void* stream);
 
 /*
- * A whole k-means iteration in two launches: oa_kmeans_assign's assignment, then oa_kmeans_update's
- * centroids in cent (in place), with no member lists.  The fp64 sums are formed per workgroup (exact,
- * so equal to the position-order sums, unless a column spans more than 2^14 times its mean).  asg and
- * asg8 both NULL (not written) or both given.  ws: oa_kmeans_step_ws(rows, T, C) bytes, 8-byte aligned.
+ * A whole k-means iteration: oa_kmeans_assign's assignment, then the members' means in cent (in place)
+ * as oa_kmeans_update forms them, with no member lists.  The sums are exact over 2048 tokens at a time
+ * (a value that is not exact in 2^-51 of its column's largest counts to that unit), then added in fp64
+ * in order: the same bits at every call and in every batch.  asg and asg8 both NULL (not written) or
+ * both given.  ws: oa_kmeans_step_ws(rows, T, C) bytes, 8-byte aligned.  oa_kmeans_step_max: with the
+ * bound words of oa_qgc_project_max for this zraw and colmean; oa_kmeans_step (or zmax NULL) reads zraw
+ * once more for them.
  */
 long oa_kmeans_step_ws(int rows, int T, int C);
 int oa_kmeans_step(const uint16_t* zraw, const float* colmean, long z_stride, int rows, int T, float* cent,
                    int C, const int32_t* init_idx, int32_t* asg, long asg_stride, uint8_t* asg8,
                    long asg8_stride, void* ws, long ws_bytes, void* stream);
+int oa_kmeans_step_max(const uint16_t* zraw, const float* colmean, const uint32_t* zmax, long z_stride,
+                       int rows, int T, float* cent, int C, const int32_t* init_idx, int32_t* asg,
+                       long asg_stride, uint8_t* asg8, long asg8_stride, void* ws, long ws_bytes,
+                       void* stream);
 
 /*
  * k-means update: centroid = mean of the members' zP rows (fp64 sum in position order, one

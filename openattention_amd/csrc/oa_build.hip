@@ -20,9 +20,9 @@
 //   codes    zc_r = fma chain over d = 0..127 in fp32 (z = fma(k_d, U_dr, z), from z = 0);
 //   colmean  per 64-token tile an fp64 sum in a fixed lane order, the tiles summed in order,
 //            then one rounding of sum / T to fp32;
-//   update   per cluster an fp64 sum of the members, one rounding of sum / count to fp32: in position
-//            order in oa_kmeans_update, in no fixed order in oa_kmeans_step (an fp64 sum of fp32 terms
-//            of like magnitude drops bits far below the fp32 mean's last one);
+//   update   per cluster the sum of the members, one rounding of sum / count to fp32: in fp64 in position
+//            order in oa_kmeans_update; in oa_kmeans_step exact over 2048 tokens (kmeans_assign_kernel
+//            says how), then in fp64 in order;
 //   sums     per cluster fp64 sums of k, k*k and v over the members in position order, one
 //            rounding to fp32.
 // The two matrix products of the QGC step (k W and zP . c) run on the bf16 matrix cores with
@@ -30,6 +30,7 @@
 // hardware's, so the CPU restatement matches them up to an agreement rate (ties of the bf16
 // result), not bit for bit.
 #include <algorithm>
+#include <cfloat>
 #include <type_traits>
 
 #include "oa_common.h"
@@ -246,7 +247,7 @@ template <int NG>
 __global__ void __launch_bounds__(64) qgc_project_kernel(const uint16_t* K, long ksh, long kst, int G,
                                                          int T, const uint16_t* W, float* zP,
                                                          long zps, uint16_t* zraw_out, double* tsum,
-                                                         int ntiles) {
+                                                         int ntiles, uint32_t* wmax) {
   __shared__ uint4 s_z[NG][64 * kRC / 8];         // the tile's bf16(k W), token rows of 32 bytes
   const int lane = threadIdx.x;
   const int row0 = NG == 1 ? (int)blockIdx.y : (int)blockIdx.y * G;
@@ -261,6 +262,9 @@ __global__ void __launch_bounds__(64) qgc_project_kernel(const uint16_t* K, long
       for (int e = 0; e < 8; ++e)
         bw[g][ch][e] = bits_bf16(W[(long)(row0 + g) * kD * kRC + (ch * 32 + 8 * (lane >> 4) + e) * kRC + (lane & 15)]);
   const int tend = min(ntiles, (int)(blockIdx.x + 1) * kProjTiles);
+  uint32_t mx[NG];   // this lane's column: the largest |bf16(k W)|, as float bits
+#pragma unroll
+  for (int g = 0; g < NG; ++g) mx[g] = 0u;
 #pragma unroll 1
   for (int tile = blockIdx.x * kProjTiles; tile < tend; ++tile) {
   double cs[NG];   // this lane's column (lane % 16) partial over its tokens, in block order
@@ -290,6 +294,7 @@ __global__ void __launch_bounds__(64) qgc_project_kernel(const uint16_t* K, long
         if (t < T) {
           if (zP) zP[(long)(row0 + g) * zps + (long)t * kRC + (lane & 15)] = v;
           cs[g] += (double)v;
+          mx[g] = max(mx[g], __float_as_uint(fabsf(v)));
         }
       }
     }
@@ -320,13 +325,28 @@ __global__ void __launch_bounds__(64) qgc_project_kernel(const uint16_t* K, long
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
   }
+  if (wmax)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const auto r16 = __builtin_amdgcn_permlane16_swap(mx[g], mx[g], false, false);
+      const uint32_t v = max(r16[0], r16[1]);
+      const auto r32 = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+      if (lane < 16) wmax[((long)(row0 + g) * gridDim.x + blockIdx.x) * kRC + lane] = max(r32[0], r32[1]);
+    }
 }
+
+// A column's bound word: the bits of a largest |bf16(k W)| that is finite, with kOddColumn where some
+// value of the column is not
+constexpr uint32_t kOddColumn = 0x80000000u;
 
 // colmean from the tile sums (tiles in order, fp64): one wave per row, lane j < 16 a column; the
 // sums of 16 tiles are requested together and then added in tile order (one load in flight at a
 // time left the pass bound by memory latency: 0.21 ms at 512 tiles, 0.44 ms at 2048)
+// Lanes 16 .. 31: the bound word of column lane - 16 from the nw waves' maxima (a value that is not finite
+// makes the column's mean so too, and every zP: what is finite beside it does not matter then).
 __global__ void __launch_bounds__(64) qgc_colmean_kernel(int T, const double* tsum, int ntiles,
-                                                         float* colmean) {
+                                                         float* colmean, const uint32_t* wmax, int nw,
+                                                         uint32_t* zmax) {
   constexpr int kBatch = 16;
   const int row = blockIdx.x;
   const int j = threadIdx.x;
@@ -343,6 +363,12 @@ __global__ void __launch_bounds__(64) qgc_colmean_kernel(int T, const double* ts
     }
     for (; k < ntiles; ++k) s += p[(long)k * kRC];
     colmean[row * kRC + j] = (float)(s / (double)T);
+  } else if (zmax && j < 2 * kRC) {
+    const uint32_t* p = wmax + (long)row * nw * kRC + j - kRC;
+    uint32_t m = 0u;
+#pragma unroll 8
+    for (int k = 0; k < nw; ++k) m = max(m, p[(long)k * kRC]);
+    zmax[row * kRC + j - kRC] = m < 0x7f800000u ? m : kOddColumn | 0x7f7f0000u;
   }
 }
 
@@ -403,28 +429,51 @@ constexpr int kAsgThreads = 256;
 constexpr int kAsgMaxTiles = 8;                // tiles per wave where the grid is full without
 constexpr uint32_t kTag = 0x3f00u;             // low half of a ranked distance: kTag | 63 - (4 cb + i)
 //
-// ACC (a whole Lloyd iteration): each token's zP also joins its cluster's fp64 sum, in LDS per
-// workgroup, and the workgroup's sums and counts go to part / pcnt for kmeans_mean_kernel; asg and
-// asg8 may be null.  The fp64 sums of fp32 values within a factor 2^14 of colmean's magnitude are
-// exact (every zP is a whole multiple of colmean's last place, or half of it, and 2^15 of them fit 53
-// bits), so that no order shows in the centroids.  Before, the ids of every iteration were sorted into
-// member lists and each cluster's rows gathered again: 0.14 + 0.44 ms per iteration at 32 sequences.
-constexpr int kAccStride = kRC + 1;            // doubles per cluster in LDS (spread over the banks)
+// ACC (a whole Lloyd iteration): each token's zP also joins its cluster's sum, in LDS per workgroup,
+// and the workgroup's sums and counts go to ll for kmeans_mean_kernel; asg and asg8 may be null.  No
+// order of the tokens shows in the centroids, nor how many tiles a wave takes (a segment of kSegTiles
+// tiles is summed exactly, and the segments are added in order):
+//   fp64     where every column of the row has |zP| <= 2^17 |colmean| =: 2^17 m.  Every zP is a multiple
+//            of half of m's last place (of m's 2^-25 at least), and 2048 of them stay below 2^28 m = 2^53
+//            times that, so that every partial sum is exact.
+//   wholes   else (a column whose mean is small against its values, or one with values that are not
+//            finite): a value counts in units of 2^-51 of a power of two above the row's largest |zP| in
+//            the column.  x + 1.5 * 2^52 holds the whole number in its low bits, and the bits are added
+//            as 64-bit integers (the constant's share comes off by the count).  A value keeps all of its
+//            24 bits down to 2^-27 of the largest.  Infinities and NaN are noted per cluster and column.
+// (fp64 atomics alone: a column of +-2^20 in pairs beside 2^-18 gave other centroids at every call.  Whole
+// numbers for every row: 9.17 ms for a build of 32 sequences of 32767 tokens, 8.79 so, 8.71 before.)
+// |zP| is bounded by |bf16(k W)| + |colmean| of the column (rounding keeps the order).  Before, the ids of
+// every iteration were sorted into member lists and each cluster's rows gathered again: 0.14 + 0.44 ms
+// per iteration at 32 sequences.
+constexpr int kAccStride = kRC + 1;            // sums per cluster in LDS (spread over the banks)
+constexpr int kSegTiles = kAsgThreads / 64 * kAsgMaxTiles;
+constexpr double kWhole = 6755399441055744.0;  // 1.5 * 2^52
+
+struct LloydArgs {                             // a whole iteration's inputs and partial results
+  const uint32_t* zmax;                        // bound words (rows, 16)
+  unsigned long long* part;                    // sums (rows, workgroups, C, 16), fp64 or whole numbers
+  int32_t* pcnt;                               // counts (rows, workgroups, C)
+  uint32_t* pbad;                              // (rows, workgroups, C): 2 bits a column, +inf and -inf (NaN: both)
+  int32_t* pexp;                               // (rows, 16): kFp64Sums, or the unit is 2^-pexp
+};
+constexpr int kFp64Sums = 0x7fffffff;
+
 template <int CB, bool ACC>
 __global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : CB <= 12 || !ACC ? 4 : 3) kmeans_assign_kernel(const uint16_t* zraw,
                                                                     const float* colmean, long zps, int T,
                                                                     const float* cent, int C,
                                                                     int32_t* asg, long as,
                                                                     uint8_t* asg8, long a8s,
-                                                                    int tiles_per_wave, double* part,
-                                                                    int32_t* pcnt) {
+                                                                    int tiles_per_wave, LloydArgs ll) {
   __shared__ __align__(16) uint16_t s_cb[CB * 16 * kRC];
   __shared__ __align__(16) float s_half[CB * 16];
-  __shared__ double s_acc[ACC ? CB * 16 * kAccStride : 1];
+  __shared__ unsigned long long s_acc[ACC ? CB * 16 * kAccStride : 1];   // (0 in either form)
   __shared__ int s_cnt[ACC ? CB * 16 : 1];
+  __shared__ uint32_t s_bad[ACC ? CB * 16 : 1];
   if (ACC) {
-    for (int i = threadIdx.x; i < CB * 16 * kAccStride; i += kAsgThreads) s_acc[i] = 0.0;
-    for (int i = threadIdx.x; i < CB * 16; i += kAsgThreads) s_cnt[i] = 0;
+    for (int i = threadIdx.x; i < CB * 16 * kAccStride; i += kAsgThreads) s_acc[i] = 0ull;
+    for (int i = threadIdx.x; i < CB * 16; i += kAsgThreads) { s_cnt[i] = 0; s_bad[i] = 0u; }
   }
   const int lane = threadIdx.x & 63, grp = lane >> 4;
   const int wave = threadIdx.x >> 6;
@@ -467,6 +516,24 @@ __global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : CB <= 12 || !ACC ? 
   float cm[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) cm[e] = colmean[row * kRC + 4 * grp + e];
+  int ex[4] = {0, 0, 0, 0};                    // |zP| < 2^(51 - ex)
+  bool wholes = false;                         // (uniform: every wave holds all columns)
+  if (ACC) {
+    bool far = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t w = ll.zmax[row * kRC + 4 * grp + e];
+      const float m = fabsf(cm[e]);
+      float b = __uint_as_float(w & ~kOddColumn) + (m < INFINITY ? m : 0.f);
+      if (!(b < INFINITY)) b = FLT_MAX;
+      far |= (w & kOddColumn) || !(b <= 131072.f * m && m < INFINITY);
+      ex[e] = 177 - (int)(__float_as_uint(b) >> 23);       // b < 2^(field - 126)
+    }
+    wholes = __any(far);
+    if (blockIdx.x == 0 && wave == 0 && (lane & 15) == 0)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ll.pexp[row * kRC + 4 * grp + e] = wholes ? ex[e] : kFp64Sums;
+  }
   const uint16_t* zr = zraw + (long)row * zps + 4 * grp;
   auto load = [&](uint2 (&z)[4], int tile) {
 #pragma unroll
@@ -528,10 +595,24 @@ __global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : CB <= 12 || !ACC ? 
       mine = grp == blk ? best : mine;
       if (ACC && tile * 64 + blk * 16 + (lane & 15) < T) {
         const int cid = 255 - (best & 0xff);          // of token lane % 16, in every lane group
+        if (!wholes) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          __hip_atomic_fetch_add(&s_acc[cid * kAccStride + 4 * grp + e], (double)zp[e], __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+          for (int e = 0; e < 4; ++e)
+            __hip_atomic_fetch_add(reinterpret_cast<double*>(&s_acc[cid * kAccStride + 4 * grp + e]), (double)zp[e],
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float v = zp[e];
+            if (!(fabsf(v) < INFINITY)) {
+              atomicOr(&s_bad[cid], (v > 0.f ? 1u : v < 0.f ? 2u : 3u) << (2 * (4 * grp + e)));
+              v = 0.f;
+            }
+            const double x = (double)__builtin_amdgcn_ldexpf(v, ex[e]) + kWhole;
+            __hip_atomic_fetch_add(&s_acc[cid * kAccStride + 4 * grp + e], (unsigned long long)__double_as_longlong(x),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+        }
         if (grp == 0) atomicAdd(&s_cnt[cid], 1);
       }
     }
@@ -547,46 +628,93 @@ __global__ void __launch_bounds__(kAsgThreads, CB <= 4 ? 6 : CB <= 12 || !ACC ? 
   if (ACC) {
     __syncthreads();
     const long g = ((long)row * gridDim.x + blockIdx.x) * C;
+    const unsigned long long base = wholes ? (unsigned long long)__double_as_longlong(kWhole) : 0ull;
     for (int i = threadIdx.x; i < C * kRC; i += kAsgThreads)
-      part[g * kRC + i] = s_acc[(i / kRC) * kAccStride + i % kRC];
-    for (int i = threadIdx.x; i < C; i += kAsgThreads) pcnt[g + i] = s_cnt[i];
+      ll.part[g * kRC + i] = s_acc[(i / kRC) * kAccStride + i % kRC] - s_cnt[i / kRC] * base;
+    for (int i = threadIdx.x; i < C; i += kAsgThreads) {
+      ll.pcnt[g + i] = s_cnt[i];
+      ll.pbad[g + i] = s_bad[i];
+    }
   }
 }
 
-// The centroids from the workgroups' sums (added in workgroup order): one thread per value, its
-// partials 8 at a time in flight; an empty cluster keeps its initial point.
-__global__ void __launch_bounds__(256) kmeans_mean_kernel(const double* part, const int32_t* pcnt, int nwg, int C,
+// The centroids from the workgroups' sums: one thread per value, its partials 8 at a time in flight.  A
+// segment's (of wgs workgroups) are added exactly, then the segments in order, in fp64; an empty
+// cluster keeps its initial point.
+__global__ void __launch_bounds__(256) kmeans_mean_kernel(LloydArgs ll, int nwg, int wgs, int C,
                                                           const uint16_t* zraw, const float* colmean, long zps,
                                                           const int32_t* init_idx, float* cent) {
   const int row = blockIdx.y;
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= C * kRC) return;
   const int c = i / kRC, j = i % kRC;
-  const double* p = part + (long)row * nwg * C * kRC + i;
-  const int32_t* q = pcnt + (long)row * nwg * C + c;
-  double acc = 0.0;
+  const unsigned long long* p = ll.part + (long)row * nwg * C * kRC + i;
+  const int32_t* q = ll.pcnt + (long)row * nwg * C + c;
+  const uint32_t* b = ll.pbad + (long)row * nwg * C + c;
+  const int ex = ll.pexp[row * kRC + j];
+  double acc = 0.0, sum = 0.0;
+  unsigned long long whole = 0ull;
   int cnt = 0;
-  for (int g0 = 0; g0 < nwg; g0 += 8) {
-    double x[8];
-    int y[8];
+  uint32_t bad = 0u;
+  for (int g0 = 0; g0 < nwg; g0 += 8) {        // (wgs divides 8)
+    unsigned long long px[8];
+    int pq[8];
+    uint32_t pb[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int g = min(g0 + u, nwg - 1);
-      x[u] = p[(long)g * C * kRC];
-      y[u] = q[(long)g * C];
+      px[u] = p[(long)g * C * kRC];
+      pq[u] = q[(long)g * C];
+      pb[u] = ex != kFp64Sums ? b[(long)g * C] : 0u;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (g0 + u < nwg) {
-        acc += x[u];
-        cnt += y[u];
+        sum += __longlong_as_double((long long)px[u]);
+        whole += px[u];                        // (two's complement, below 2^62: 2048 values)
+        cnt += pq[u];
+        bad |= pb[u];
+        if ((u + 1) % wgs == 0 || g0 + u == nwg - 1) {
+          acc += ex == kFp64Sums ? sum : __builtin_amdgcn_ldexp((double)(long long)whole, -ex);
+          sum = 0.0;
+          whole = 0ull;
+        }
       }
   }
+  bad = bad >> (2 * j) & 3u;
+  if (bad) acc = bad == 3u ? NAN : bad == 1u ? INFINITY : -INFINITY;
   cent[(long)row * C * kRC + i] =
       cnt > 0 ? (float)(acc / (double)cnt)
               : oa::bf16_to_f32(zraw[(long)row * zps + (long)init_idx[c] * kRC + j]) - colmean[row * kRC + j];
 }
 
+// The bound words of a projection that came without them: one workgroup per row reads it once, a thread
+// 8 columns of every 128th token.
+__global__ void __launch_bounds__(256) column_max_kernel(const uint16_t* zraw, long zps, int T, uint32_t* zmax) {
+  typedef uint32_t uint32x4a8 __attribute__((ext_vector_type(4), aligned(8)));
+  __shared__ uint32_t s_mx[kRC], s_odd[kRC];
+  const int row = blockIdx.x, half = threadIdx.x & 1;
+  if (threadIdx.x < kRC) s_mx[threadIdx.x] = s_odd[threadIdx.x] = 0u;
+  __syncthreads();
+  uint32_t mx[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u}, odd = 0u;
+#pragma unroll 4
+  for (int t = threadIdx.x >> 1; t < T; t += 128) {
+    const uint32x4a8 x = *reinterpret_cast<const uint32x4a8*>(zraw + (long)row * zps + (long)t * kRC + 8 * half);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t y = (k & 1 ? x[k >> 1] : x[k >> 1] << 16) & 0x7fff0000u;
+      if (y < 0x7f800000u) mx[k] = max(mx[k], y);
+      else odd |= 1u << k;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    atomicMax(&s_mx[8 * half + k], mx[k]);
+    if (odd >> k & 1u) s_odd[8 * half + k] = kOddColumn;
+  }
+  __syncthreads();
+  if (threadIdx.x < kRC) zmax[row * kRC + threadIdx.x] = s_mx[threadIdx.x] | s_odd[threadIdx.x];
+}
 
 // a wave copies 1 <= n <= (the LDS array's size) member positions into LDS, eight loads per lane
 // in flight at a time (one at a time, each copy waited on its load)
@@ -923,9 +1051,9 @@ extern "C" int oa_qgs_codes(const void* K, long k_stride_h, long k_stride_t, int
   return OA_LAUNCH_STATUS();
 }
 
-extern "C" int oa_qgc_project(const void* K, long k_stride_h, long k_stride_t, int rows, int G, int T,
+static int qgc_project(const void* K, long k_stride_h, long k_stride_t, int rows, int G, int T,
                               const void* W, float* zP, long zp_stride, float* colmean,
-                              double* tile_ws, uint16_t* zraw_out, void* stream) {
+                              double* tile_ws, uint16_t* zraw_out, uint32_t* wmax, uint32_t* zmax, void* stream) {
   if (rows <= 0 || G <= 0 || rows % G || T <= 0 || !K || !W || (!zP && !zraw_out) || !colmean ||
       !tile_ws || k_stride_t < kD || k_stride_t % 8 || k_stride_h % 8 || zp_stride < (long)T * kRC ||
       zp_stride % 4 || (reinterpret_cast<uintptr_t>(K) & 15) || (reinterpret_cast<uintptr_t>(zP) & 15) ||
@@ -937,12 +1065,13 @@ extern "C" int oa_qgc_project(const void* K, long k_stride_h, long k_stride_t, i
   if (G == 4)   // a KV row's four query rows per wave: each K block loaded once for all four
     hipLaunchKernelGGL(qgc_project_kernel<4>, dim3(nx, rows / 4), dim3(64), 0, s,
                        reinterpret_cast<const uint16_t*>(K), k_stride_h, k_stride_t, G, T,
-                       reinterpret_cast<const uint16_t*>(W), zP, zp_stride, zraw_out, tile_ws, ntiles);
+                       reinterpret_cast<const uint16_t*>(W), zP, zp_stride, zraw_out, tile_ws, ntiles, wmax);
   else
     hipLaunchKernelGGL(qgc_project_kernel<1>, dim3(nx, rows), dim3(64), 0, s,
                        reinterpret_cast<const uint16_t*>(K), k_stride_h, k_stride_t, G, T,
-                       reinterpret_cast<const uint16_t*>(W), zP, zp_stride, zraw_out, tile_ws, ntiles);
-  hipLaunchKernelGGL(qgc_colmean_kernel, dim3(rows), dim3(64), 0, s, T, tile_ws, ntiles, colmean);
+                       reinterpret_cast<const uint16_t*>(W), zP, zp_stride, zraw_out, tile_ws, ntiles, wmax);
+  hipLaunchKernelGGL(qgc_colmean_kernel, dim3(rows), dim3(64), 0, s, T, tile_ws, ntiles, colmean,
+                     wmax, nx, zmax);
   if (zP) {
     const int nb = std::min(16, (T * (kRC / 4) + 255) / 256);
     hipLaunchKernelGGL(qgc_center_kernel, dim3(nb, rows), dim3(256), 0, s, zP, zp_stride, T, colmean);
@@ -950,22 +1079,37 @@ extern "C" int oa_qgc_project(const void* K, long k_stride_h, long k_stride_t, i
   return OA_LAUNCH_STATUS();
 }
 
-// tiles per wave: up to eight spread the centroids' staging; fewer where the grid would not give
-// every SIMD eight waves
+extern "C" int oa_qgc_project(const void* K, long k_stride_h, long k_stride_t, int rows, int G, int T,
+                              const void* W, float* zP, long zp_stride, float* colmean, double* tile_ws,
+                              uint16_t* zraw_out, void* stream) {
+  return qgc_project(K, k_stride_h, k_stride_t, rows, G, T, W, zP, zp_stride, colmean, tile_ws, zraw_out, nullptr,
+                     nullptr, stream);
+}
+
+extern "C" int oa_qgc_project_max(const void* K, long k_stride_h, long k_stride_t, int rows, int G, int T,
+                                  const void* W, float* zP, long zp_stride, float* colmean, double* tile_ws,
+                                  uint16_t* zraw_out, uint32_t* max_ws, uint32_t* zmax, void* stream) {
+  if (!max_ws || !zmax) return OA_EINVAL;
+  return qgc_project(K, k_stride_h, k_stride_t, rows, G, T, W, zP, zp_stride, colmean, tile_ws, zraw_out, max_ws,
+                     zmax, stream);
+}
+
+// tiles per wave: up to eight spread the centroids' staging; fewer, a power of two so that workgroups
+// share a segment evenly, where the grid would not give every SIMD eight waves
 static int asg_tiles_per_wave(int rows, int T) {
-  const long ntiles = (T + 63) / 64;
-  return (int)std::min<long>(kAsgMaxTiles, std::max<long>(1, ntiles * rows / 8192));
+  const long want = (long)((T + 63) / 64) * rows / 8192;
+  return want >= kAsgMaxTiles ? kAsgMaxTiles : want >= 4 ? 4 : want >= 2 ? 2 : 1;
 }
 
 template <bool ACC>
 static void launch_assign(const uint16_t* zraw, const float* colmean, long z_stride, int rows, int T,
                           const float* cent, int C, int32_t* asg, long asg_stride, uint8_t* asg8,
-                          long asg8_stride, int tpw, double* part, int32_t* pcnt, hipStream_t stream) {
+                          long asg8_stride, int tpw, LloydArgs ll, hipStream_t stream) {
   const int ntiles = (T + 63) / 64, per = kAsgThreads / 64 * tpw;
   const dim3 grid((ntiles + per - 1) / per, rows), block(kAsgThreads);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, zraw, colmean, z_stride, T, cent, C, asg, asg_stride, asg8,
-                       asg8_stride, tpw, part, pcnt);
+                       asg8_stride, tpw, ll);
   };
   // the centroid blocks a wave holds: the least of these that covers C (padding ranks below)
   const int cb = (C + 15) / 16;
@@ -985,39 +1129,57 @@ extern "C" int oa_kmeans_assign(const uint16_t* zraw, const float* colmean, long
       (reinterpret_cast<uintptr_t>(zraw) & 7))
     return OA_EINVAL;
   const int tpw = asg_tiles_per_wave(rows, T);
-  launch_assign<false>(zraw, colmean, z_stride, rows, T, cent, C, asg, asg_stride, asg8, asg8_stride, tpw, nullptr,
-                       nullptr, (hipStream_t)stream);
+  launch_assign<false>(zraw, colmean, z_stride, rows, T, cent, C, asg, asg_stride, asg8, asg8_stride, tpw,
+                       LloydArgs{}, (hipStream_t)stream);
   return OA_LAUNCH_STATUS();
 }
 
-// a whole Lloyd iteration: part_ws holds a workgroup's sums and counts for each of the grid's
+// a whole Lloyd iteration: the workspace holds the sums, counts and flags of each of the grid's
+// workgroups, each row's units and bound words
 static int step_groups(int rows, int T) {
-  const int waves = kAsgThreads / 64, tpw = asg_tiles_per_wave(rows, T);
-  return ((T + 63) / 64 + waves * tpw - 1) / (waves * tpw);
+  const int per = kAsgThreads / 64 * asg_tiles_per_wave(rows, T);
+  return ((T + 63) / 64 + per - 1) / per;
 }
 
 extern "C" long oa_kmeans_step_ws(int rows, int T, int C) {
   if (rows <= 0 || T <= 0 || C <= 0 || C > kMaxC) return OA_EINVAL;
-  return (long)rows * step_groups(rows, T) * C * (kRC * 8 + 4);
+  return (long)rows * (step_groups(rows, T) * (long)C * (kRC * 8 + 8) + kRC * 8);
 }
 
-extern "C" int oa_kmeans_step(const uint16_t* zraw, const float* colmean, long z_stride, int rows, int T,
-                              float* cent, int C, const int32_t* init_idx, int32_t* asg, long asg_stride,
-                              uint8_t* asg8, long asg8_stride, void* ws, long ws_bytes, void* stream) {
+// zmax NULL: the bound words are formed here
+extern "C" int oa_kmeans_step_max(const uint16_t* zraw, const float* colmean, const uint32_t* zmax, long z_stride,
+                                  int rows, int T, float* cent, int C, const int32_t* init_idx, int32_t* asg,
+                                  long asg_stride, uint8_t* asg8, long asg8_stride, void* ws, long ws_bytes,
+                                  void* stream) {
   if (rows <= 0 || T <= 0 || C <= 0 || C > kMaxC || !zraw || !colmean || !cent || !init_idx || !ws ||
       z_stride < (long)T * kRC || z_stride % 4 || (!asg != !asg8) || (asg && (asg_stride < T || asg8_stride < T)) ||
       (reinterpret_cast<uintptr_t>(zraw) & 7) || (reinterpret_cast<uintptr_t>(ws) & 7) ||
       ws_bytes < oa_kmeans_step_ws(rows, T, C))
     return OA_EINVAL;
-  const int nwg = step_groups(rows, T);
-  double* part = static_cast<double*>(ws);
-  int32_t* pcnt = reinterpret_cast<int32_t*>(part + (long)rows * nwg * C * kRC);
+  const int nwg = step_groups(rows, T), tpw = asg_tiles_per_wave(rows, T);
   hipStream_t s = (hipStream_t)stream;
-  launch_assign<true>(zraw, colmean, z_stride, rows, T, cent, C, asg, asg_stride, asg8, asg8_stride,
-                      asg_tiles_per_wave(rows, T), part, pcnt, s);
-  hipLaunchKernelGGL(kmeans_mean_kernel, dim3((C * kRC + 255) / 256, rows), dim3(256), 0, s, part, pcnt, nwg, C,
-                     zraw, colmean, z_stride, init_idx, cent);
+  LloydArgs ll;
+  ll.part = static_cast<unsigned long long*>(ws);
+  ll.pcnt = reinterpret_cast<int32_t*>(ll.part + (long)rows * nwg * C * kRC);
+  ll.pbad = reinterpret_cast<uint32_t*>(ll.pcnt + (long)rows * nwg * C);
+  ll.pexp = reinterpret_cast<int32_t*>(ll.pbad + (long)rows * nwg * C);
+  ll.zmax = zmax;
+  if (!zmax) {
+    uint32_t* own = reinterpret_cast<uint32_t*>(ll.pexp + (long)rows * kRC);
+    hipLaunchKernelGGL(column_max_kernel, dim3(rows), dim3(256), 0, s, zraw, z_stride, T, own);
+    ll.zmax = own;
+  }
+  launch_assign<true>(zraw, colmean, z_stride, rows, T, cent, C, asg, asg_stride, asg8, asg8_stride, tpw, ll, s);
+  hipLaunchKernelGGL(kmeans_mean_kernel, dim3((C * kRC + 255) / 256, rows), dim3(256), 0, s, ll, nwg,
+                     kAsgMaxTiles / tpw, C, zraw, colmean, z_stride, init_idx, cent);
   return OA_LAUNCH_STATUS();
+}
+
+extern "C" int oa_kmeans_step(const uint16_t* zraw, const float* colmean, long z_stride, int rows, int T,
+                              float* cent, int C, const int32_t* init_idx, int32_t* asg, long asg_stride,
+                              uint8_t* asg8, long asg8_stride, void* ws, long ws_bytes, void* stream) {
+  return oa_kmeans_step_max(zraw, colmean, nullptr, z_stride, rows, T, cent, C, init_idx, asg, asg_stride, asg8,
+                            asg8_stride, ws, ws_bytes, stream);
 }
 
 // the sort stages a row's ids in LDS with 16-byte loads when the row fits and its rows are

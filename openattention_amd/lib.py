@@ -68,9 +68,11 @@ SIGNATURES = {
     "oa_dense_decode": [P, L, P, P, L, L, I, I, I, I, P, F, I, P, P, P, P, L, P],
     "oa_qgs_codes": [P, L, L, I, I, P, P, L, P, P, P, P],
     "oa_qgc_project": [P, L, L, I, I, I, P, P, L, P, P, P, P],
+    "oa_qgc_project_max": [P, L, L, I, I, I, P, P, L, P, P, P, P, P, P],
     "oa_kmeans_assign": [P, P, L, I, I, P, I, P, L, P, L, P],
     "oa_kmeans_step_ws": [I, I, I],
     "oa_kmeans_step": [P, P, L, I, I, P, I, P, P, L, P, L, P, L, P],
+    "oa_kmeans_step_max": [P, P, P, L, I, I, P, I, P, P, L, P, L, P, L, P],
     "oa_kmeans_update": [P, P, L, I, I, P, L, I, P, P, P, P, L, P, P, P],
     "oa_cluster_build": [P, P, L, L, I, I, I, P, L, I, P, P, P, P, P, L, P, P, P],
     "oa_cluster_sums": [P, P, L, L, I, I, I, I, P, P, P, P, P, L, P, P, P],

@@ -495,9 +495,8 @@ class OursHIP(Method):
                     held = n_first
                 if i0 == 0:      # the method's own result buffers hold the last row run, row 0, as after a step
                     self.last_sel = row(sel, 0)
-                    for f in ("score", "n_t", "quota", "exp_idx"):
-                        getattr(self, f).copy_(row(w[f], 0))
-                    self.out.copy_(row(o, 0))
+                    for to, t in [(getattr(self, f), w[f]) for f in ("score", "n_t", "quota", "exp_idx")] + [(self.out, o)]:
+                        to.view(B * HKV, G, -1).copy_(t[:Rg].view(B * HKV, nq, G, -1)[:, 0])
         finally:
             n_dev.fill_(n_keys)
         return out

@@ -733,10 +733,11 @@ def sym_eig_top(M, k: int, sweeps=None):
     return ev, vec
 
 
-def qgc_project(K, T: int, W, G: int, zraw, colmean, zP=None) -> None:
+def qgc_project(K, T: int, W, G: int, zraw, colmean, zP=None, zmax=None) -> None:
     """a12 projection: zraw (HQ, T, 16) int16/bf16 = bf16(k W) (what kmeans_assign and
-    kmeans_update read); colmean (HQ, 16); zP (HQ, T, 16) fp32 = bf16(k W) - colmean, or None."""
-    dev = _dev(K, W, zraw, colmean)
+    kmeans_update read); colmean (HQ, 16); zP (HQ, T, 16) fp32 = bf16(k W) - colmean, or None; zmax
+    (HQ, 16) int32 or None, the columns' bound words for kmeans_step."""
+    dev = _dev(K, W, zraw, colmean, zmax)
     HQ = W.shape[0]
     _need(W.dtype == torch.bfloat16 and W.is_contiguous() and W.shape[1:] == (HEAD_DIM, RANK_C),
           "W: (HQ, 128, 16) bf16 contiguous")
@@ -747,8 +748,14 @@ def qgc_project(K, T: int, W, G: int, zraw, colmean, zP=None) -> None:
         _need(zP.dtype == torch.float32 and zP.stride() == zraw.stride(), "zP: fp32, zraw's strides")
     ntiles = -(-T // 64)
     ws = torch.empty(HQ * ntiles * RANK_C, device=dev, dtype=torch.float64)
-    lib.call("oa_qgc_project", _ptr(K), K.stride(0), K.stride(1), HQ, G, T, _ptr(W), _ptr(zP),
-             zraw.stride(0), _ptr(colmean), _ptr(ws), _ptr(zraw), _stream(dev))
+    args = (_ptr(K), K.stride(0), K.stride(1), HQ, G, T, _ptr(W), _ptr(zP), zraw.stride(0), _ptr(colmean), _ptr(ws),
+            _ptr(zraw))
+    if zmax is None:
+        lib.call("oa_qgc_project", *args, _stream(dev))
+        return
+    _chk(zmax, "zmax", torch.int32, (HQ, RANK_C), contiguous=True)
+    max_ws = torch.empty(HQ * -(-T // 512) * RANK_C, device=dev, dtype=torch.int32)
+    lib.call("oa_qgc_project_max", *args, _ptr(max_ws), _ptr(zmax), _stream(dev))
 
 
 def _zraw(zraw, HQ: int, T: int) -> None:
@@ -770,11 +777,12 @@ def kmeans_assign(zraw, colmean, T: int, cent, asg, asg8) -> None:
              asg.stride(0), _ptr(asg8), asg8.stride(0), _stream(dev))
 
 
-def kmeans_step(zraw, colmean, T: int, init, cent, asg=None, asg8=None, ws=None) -> torch.Tensor:
+def kmeans_step(zraw, colmean, T: int, init, cent, asg=None, asg8=None, ws=None, zmax=None) -> torch.Tensor:
     """kmeans_assign then kmeans_update's centroids (cent in place) without member lists; asg and asg8
     both None (not written) or both given.  ws: a byte workspace of a former call with the same sizes,
-    or None; returns the workspace used."""
-    dev = _dev(zraw, colmean, cent, init, asg, asg8)
+    or None; returns the workspace used.  zmax: qgc_project's bound words for this zraw and colmean, or
+    None (zraw is then read once more for them)."""
+    dev = _dev(zraw, colmean, cent, init, asg, asg8, ws, zmax)
     HQ, C = cent.shape[0], cent.shape[1]
     _zraw(zraw, HQ, T)
     _need(colmean.is_contiguous() and colmean.shape == (HQ, RANK_C), "colmean: (HQ, 16) contiguous")
@@ -788,8 +796,10 @@ def kmeans_step(zraw, colmean, T: int, init, cent, asg=None, asg8=None, ws=None)
     _need(need > 0, "kmeans_step: rows, T and C must be positive, C at most 256")
     if ws is None or ws.numel() < need:
         ws = torch.empty(need, device=dev, dtype=torch.uint8)
-    lib.call("oa_kmeans_step", _ptr(zraw), _ptr(colmean), zraw.stride(0), HQ, T, _ptr(cent), C, _ptr(init),
-             _ptr(asg), 0 if asg is None else asg.stride(0), _ptr(asg8), 0 if asg8 is None else asg8.stride(0),
+    if zmax is not None:
+        _chk(zmax, "zmax", torch.int32, (HQ, RANK_C), contiguous=True)
+    lib.call("oa_kmeans_step_max", _ptr(zraw), _ptr(colmean), _ptr(zmax), zraw.stride(0), HQ, T, _ptr(cent), C,
+             _ptr(init), _ptr(asg), 0 if asg is None else asg.stride(0), _ptr(asg8), 0 if asg8 is None else asg8.stride(0),
              _ptr(ws), ws.numel(), _stream(dev))
     return ws
 

@@ -359,7 +359,8 @@ def _build_device(st, r0: int, K: torch.Tensor, V: torch.Tensor, T: int, layer: 
     # (fp32) as they read it
     zraw = torch.empty(HQ, T, RC, device=dev, dtype=torch.bfloat16)
     colmean = st.colmean[q0:q0 + HQ]
-    ops.qgc_project(K, T, st.W[q0:q0 + HQ], G, zraw, colmean)
+    zmax = torch.empty(HQ, RC, device=dev, dtype=torch.int32)
+    ops.qgc_project(K, T, st.W[q0:q0 + HQ], G, zraw, colmean, zmax=zmax)
     mark("project")
     init = _h2d(kmeans_init(T, C, layer).to(torch.int32), dev)
     cent = st.cent[q0:q0 + HQ]
@@ -370,7 +371,8 @@ def _build_device(st, r0: int, K: torch.Tensor, V: torch.Tensor, T: int, layer: 
     ws = None
     for it in range(ITERS):
         last = it == ITERS - 1
-        ws = ops.kmeans_step(zraw, colmean, T, init, cent, asg if last else None, asg8 if last else None, ws)
+        ws = ops.kmeans_step(zraw, colmean, T, init, cent, asg if last else None, asg8 if last else None, ws,
+                             zmax)
         mark("kmeans")
     del ws
     # a13: the CSR member lists of that assignment and the cluster statistics
