@@ -442,8 +442,8 @@ int oa_kmeans_update(const uint16_t* zraw, const float* colmean, long z_stride, 
 
 /*
  * Cluster statistics and CSR member lists: nb = member count, Sk = sum k, Sk2 = sum k*k,
- * Sv = sum v (fp64 sums in position order, one rounding); mem = members by cluster, in position
- * order (the stable argsort of the assignment), cstart / clen per cluster.  K, V: kv_rows rows
+ * Sv = sum v (fp64 sums, one rounding; the order of the terms follows from T, C and the members alone,
+ * so that a row gives the same bits in every batch); mem = members by cluster, in position order (the stable argsort of the assignment), cstart / clen per cluster.  K, V: kv_rows rows
  * of (T, 128) bf16; nb (rows, C); Sk, Sk2, Sv (rows, C, 128); mem (rows, mem_stride).
  * Replaces _k_cluster_sums and the CSR build of inference/ours_fastbuild.py:111-139, 293-301
  * (methods_eager.py:548-555).
@@ -455,8 +455,8 @@ int oa_cluster_build(const void* K, const void* V, long kv_stride_h, long kv_str
 
 /*
  * Cluster statistics over member lists already built (the ones oa_kmeans_update leaves for the
- * assignment it was given): nb = clen (as float), Sk = sum k, Sk2 = sum k*k, Sv = sum v (fp64
- * sums in list order, one rounding); the same outputs as oa_cluster_build for that assignment,
+ * assignment it was given): nb = clen (as float), Sk = sum k, Sk2 = sum k*k, Sv = sum v as
+ * oa_cluster_build forms them; the same outputs as oa_cluster_build for that assignment,
  * without sorting it again.  mem (rows, mem_stride), cstart / clen (rows, C) as oa_cluster_build
  * writes them.  Replaces _k_cluster_sums (inference/ours_fastbuild.py:111-139) where the CSR
  * lists of ours_fastbuild.py:293-301 are already at hand.

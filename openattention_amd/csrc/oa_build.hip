@@ -23,8 +23,8 @@
 //   update   per cluster the sum of the members, one rounding of sum / count to fp32: in fp64 in position
 //            order in oa_kmeans_update; in oa_kmeans_step exact over 2048 tokens (kmeans_assign_kernel
 //            says how), then in fp64 in order;
-//   sums     per cluster fp64 sums of k, k*k and v over the members in position order, one
-//            rounding to fp32.
+//   sums     per cluster fp64 sums of k, k*k and v over the members, a fixed order that the row's length
+//            and cluster count give (cluster_sums_kernel), one rounding to fp32.
 // The two matrix products of the QGC step (k W and zP . c) run on the bf16 matrix cores with
 // fp32 accumulation, as the reference's bf16 matmuls do; their fp32 partial rounding is the
 // hardware's, so the CPU restatement matches them up to an agreement rate (ties of the bf16
@@ -441,7 +441,7 @@ constexpr uint32_t kTag = 0x3f00u;             // low half of a ranked distance:
 //            the column.  x + 1.5 * 2^52 holds the whole number in its low bits, and the bits are added
 //            as 64-bit integers (the constant's share comes off by the count).  A value keeps all of its
 //            24 bits down to 2^-27 of the largest.  Infinities and NaN are noted per cluster and column.
-// (fp64 atomics alone: a column of +-2^20 in pairs beside 2^-18 gave other centroids at every call.  Whole
+// (fp64 atomics alone: a column of +-2^20 in pairs beside 2^-22 gave other centroids at every call.  Whole
 // numbers for every row: 9.17 ms for a build of 32 sequences of 32767 tokens, 8.79 so, 8.71 before.)
 // |zP| is bounded by |bf16(k W)| + |colmean| of the column (rounding keeps the order).  Before, the ids of
 // every iteration were sorted into member lists and each cluster's rows gathered again: 0.14 + 0.44 ms
@@ -914,8 +914,10 @@ __global__ void __launch_bounds__(kSortThreads) csr_sort_kernel(int T, const uin
 // The fp64 sums of k, k*k and v of one (cluster, query row) by W waves: a lane holds 8 dims (16-byte
 // loads) of the members its 16-lane group takes, every (4 W)-th of the list, 4 at a time in flight;
 // the groups' sums are joined by two lane swaps and (W > 1) through LDS.  A group adds its members in
-// position order; sums of bf16 values, and of their squares, are exact in fp64 unless they span more
-// than 2^30 in magnitude, so how the list is split does not show in the fp32 results.
+// position order.  Sums of up to 2^15 bf16 values are exact in fp64 where these span at most 2^30, of
+// their squares (16 bits, twice the span) where the values span at most 2^11; beyond, the order shows in
+// what rounding leaves, so that W follows from the row alone, not from the batch: the same row gives the
+// same bits in every call.
 // Bound by vector issue: 14 fp64 and conversion instructions per member and lane of 8 dims.  With a
 // lane on 2 dims (4-byte loads, a row address per member for every lane) 32 sequences of 32767 tokens
 // took 2215 us, and take 2086 us (by the counters 15 GB of the 17 GB gathered miss the L2s: waves of
@@ -1205,13 +1207,17 @@ extern "C" int oa_kmeans_update(const uint16_t* zraw, const float* colmean, long
   return OA_LAUNCH_STATUS();
 }
 
-// one wave per (cluster, row) where those fill the chip (16384 are four waves per SIMD), else four
-static void launch_sums(const void* K, const void* V, long ksh, long kst, int rows, int G, int C,
+// Waves per (cluster, row) by a row's mean members, whatever the batch: four from 256 up, where a
+// cluster of several times the mean holds a wave for long, else one (four waves' joins cost more than
+// they save).  On built indexes, one wave against four: 32, 8 and 1 sequences of 32767 tokens in 64
+// clusters 2123 / 1799, 611 / 477 and 146 / 81 us; in 192 clusters (170 members) 1702 / 2020, 461 / 518
+// and 87 / 72; 8 of 4096 in 256 clusters 96 / 247.
+static void launch_sums(const void* K, const void* V, long ksh, long kst, int rows, int G, int T, int C,
                         const int32_t* cstart, const int32_t* clen, float* Sk, float* Sk2, float* Sv,
                         const int32_t* mem, long ms, float* nb, hipStream_t s) {
   const uint16_t* k = reinterpret_cast<const uint16_t*>(K);
   const uint16_t* v = reinterpret_cast<const uint16_t*>(V);
-  if ((long)rows * C >= 16384)
+  if (T < 256L * C)
     hipLaunchKernelGGL(cluster_sums_kernel<1>, dim3(C * rows), dim3(64), 0, s, k, v, ksh, kst, G, C, cstart,
                        clen, Sk, Sk2, Sv, mem, ms, nb);
   else
@@ -1231,7 +1237,7 @@ extern "C" int oa_cluster_build(const void* K, const void* V, long kv_stride_h, 
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(csr_sort_kernel, dim3(rows), dim3(kSortThreads), 0, s, T, asg8, asg8_stride, C, nb,
                      cstart, clen, mem, mem_stride, sort_staged(T, asg8, asg8_stride));
-  launch_sums(K, V, kv_stride_h, kv_stride_t, rows, G, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride, nullptr, s);
+  launch_sums(K, V, kv_stride_h, kv_stride_t, rows, G, T, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride, nullptr, s);
   return OA_LAUNCH_STATUS();
 }
 
@@ -1244,7 +1250,7 @@ extern "C" int oa_cluster_sums(const void* K, const void* V, long kv_stride_h, l
       kv_stride_h % 2 || mem_stride < T || (reinterpret_cast<uintptr_t>(K) & 3) ||
       (reinterpret_cast<uintptr_t>(V) & 3))
     return OA_EINVAL;
-  launch_sums(K, V, kv_stride_h, kv_stride_t, rows, G, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride, nb,
+  launch_sums(K, V, kv_stride_h, kv_stride_t, rows, G, T, C, cstart, clen, Sk, Sk2, Sv, mem, mem_stride, nb,
               (hipStream_t)stream);
   return OA_LAUNCH_STATUS();
 }

@@ -67,18 +67,18 @@ def test_kmeans_step_of_several_tiles_per_wave(R, T, C):
 
 
 def _cancelling(T, C, big):
-    """(T, 16) tokens in pairs of one cluster: dimension 0 tells the clusters apart, dimension 5 holds
-    +-big in every pair, 6 whole multiples of 2^-26 about 2^-18, 7 one or the other."""
+    """(T, 16) tokens, t and t + 128 of every 256 in one cluster: dimension 0 tells the clusters apart,
+    dimension 5 holds big in the one and -big in the other, 6 whole multiples of 2^-30 about 2^-22, 7 one
+    or the other."""
     g = torch.Generator(device=DEV).manual_seed(T + C)
-    ids = torch.randint(0, C, (T // 2 + 1,), device=DEV, generator=g).repeat_interleave(2)[:T]
     t = torch.arange(T, device=DEV)
-    sign = torch.where(t % 2 == 0, 1.0, -1.0)
-    if T % 2:
-        sign[-1] = 0.0
+    ids = torch.randint(0, C, (T // 256 + 1, 1, 128), device=DEV, generator=g).expand(-1, 2, -1).reshape(-1)[:T]
+    sign = torch.where(t % 256 < 128, 1.0, -1.0)
+    sign[(t % 256 < 128) & (t + 128 >= T)] = 0.0
     z = torch.zeros(T, 16, device=DEV)
     z[:, 0] = 8.0 * (ids - C // 2)
     z[:, 5] = sign * big
-    z[:, 6] = (torch.randn(T, device=DEV, generator=g) * 256).round() * 2.0 ** -26
+    z[:, 6] = (torch.randn(T, device=DEV, generator=g) * 256).round() * 2.0 ** -30
     z[:, 7] = torch.where(t % 4 < 2, sign * big, z[:, 6])
     cent = torch.zeros(C, 16, device=DEV)
     cent[:, 0] = 8.0 * (torch.arange(C, device=DEV) - C // 2)
@@ -87,10 +87,10 @@ def _cancelling(T, C, big):
 
 @pytest.mark.parametrize("T,C", [(4096, 4), (20001, 16), (70000, 2)])
 def test_kmeans_step_sums_have_no_order(T, C):
-    """Columns whose mean is tiny against their values (+-2^20 in pairs beside 2^-18): the centroids of
+    """Columns whose mean is tiny against their values (+-2^20 in pairs beside 2^-22): the centroids of
     every call, of every row and of every batch (one to eight tiles per wave) are the same bits, and
     those of the exact mean, also with clusters of more than 2^15 members: the values are multiples of
-    2^-26 and the sums' unit is 2^-30, 2^-51 of 2^21."""
+    2^-30, the sums' unit (2^-51 of 2^21)."""
     print(f"[case] k-means sums without order T={T} C={C}", flush=True)
     z, cent, ids = _cancelling(T, C, 2.0 ** 20)
     init = torch.zeros(C, device=DEV, dtype=torch.int32)
@@ -191,3 +191,54 @@ def test_projection_bound_words(T, G):
     ops.kmeans_step(zraw, cm, T, init, a, zmax=zmax)
     ops.kmeans_step(zraw, cm, T, init, b)
     assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+def _cluster_build(K, V, T, asg8, C):
+    R = asg8.shape[0]
+    nb = torch.empty(R, C, device=DEV)
+    S = [torch.full((R, C, 128), 7.0, device=DEV) for _ in range(3)]
+    ops.cluster_build(K, V, T, 4, asg8, C, nb, *S, *_lists(R, T, C))
+    return nb, S
+
+
+@pytest.mark.parametrize("T,C", [(255, 1), (256, 1), (4095, 16), (4096, 16), (5001, 5), (700, 9)])
+def test_cluster_sums_do_not_depend_on_the_batch(T, C):
+    """Cluster statistics of a KV row in a batch of 1, of 3 and of as many as give 16384 (cluster, row)
+    pairs, with one and with four waves per cluster (256 mean members up): the same bits, over pairs of
+    values about +-2^32 beside values about 2^-12, whose fp64 sums show their order, uneven clusters, an
+    empty one, and rows off a 16-byte boundary; within n 2^-53 of the sum of magnitudes of the exact sums,
+    and their rounding to fp32."""
+    print(f"[case] cluster sums batches T={T} C={C}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + C)
+    t = torch.arange(T, device=DEV)
+    pair = torch.randn(2, 1, T // 2 + 1, 130, device=DEV, generator=g).repeat_interleave(2, 2)[:, :, :T]
+    big = pair * torch.where(t % 2 == 0, 2.0 ** 32, -(2.0 ** 32))[:, None]
+    one = torch.where((t % 4 < 2)[:, None], big, torch.randn(2, 1, T, 130, device=DEV, generator=g) * 2.0 ** -12)
+    one = one.to(torch.bfloat16)
+    ids = (C * torch.rand(4, T // 2 + 1, device=DEV, generator=g) ** 2).long().clamp(max=C - 1)
+    ids = ids.repeat_interleave(2, 1)[:, :T].clone()
+    if C > 3:
+        ids[ids == 3] = 4
+    base = None
+    for B in (1, 3, -(-16384 // (4 * C))):
+        if B * T > 1 << 21:
+            continue
+        kv = one.expand(2, B, T, 130).contiguous()
+        asg8 = torch.zeros(4 * B, -(-T // 64) * 64, device=DEV, dtype=torch.uint8)
+        asg8[:, :T] = ids.repeat(B, 1)
+        nb, S = _cluster_build(kv[0][..., 2:], kv[1][..., 2:], T, asg8, C)
+        if base is None:
+            base = nb, S
+        assert torch.equal(nb, base[0].repeat(B, 1))
+        for x, y in zip(S, base[1]):
+            assert torch.equal(x, y.repeat(B, 1, 1)), B
+    k, v = one[0, 0, :, 2:].double().cpu().numpy(), one[1, 0, :, 2:].double().cpu().numpy()
+    for r in (0, 3):
+        for c in range(C):
+            m = (ids[r] == c).cpu().numpy()
+            assert int(base[0][r, c]) == m.sum()
+            for got, x in zip(base[1], (k, k * k, v)):
+                for j in (0, 77):
+                    want = math.fsum(x[m, j])
+                    bound = m.sum() * 2.0 ** -53 * np.abs(x[m, j]).sum() + 2.0 ** -24 * abs(want)
+                    assert abs(float(got[r, c, j]) - want) <= bound, (r, c, j)

@@ -1467,7 +1467,7 @@ def test_kmeans_assign_edges_exact(C, T):
 def test_kmeans_step_equals_assign_then_update(R, T, C):
     """A Lloyd iteration in one call against the assignment and the member-list update: the same ids
     and the same centroid bits (the fp64 sums are exact, so their order does not show), with empty
-    clusters, ragged tiles, one and several workgroups per row and one tile or more per wave; without
+    clusters, ragged tiles, one and several workgroups per row, one tile per wave; without
     asg the ids are not written and the centroids are the same."""
     print(f"[case] k-means step R={R} T={T} C={C}", flush=True)
     g = torch.Generator(device=DEV).manual_seed(R * 7919 + T * 31 + C)
@@ -1495,8 +1495,8 @@ def test_kmeans_step_equals_assign_then_update(R, T, C):
 
 @pytest.mark.parametrize("HKV_,T,C", [(8, 3000, 64), (64, 300, 64), (65, 700, 70)])
 def test_cluster_sums_layouts_bit_exact(HKV_, T, C):
-    """Cluster statistics with four waves per (cluster, row) and with one (16384 pairs and more), over
-    uneven clusters, an empty one, and K, V rows that start 4 bytes off a 16-byte boundary."""
+    """Cluster statistics of short rows (one wave per (cluster, row)), few pairs and 16384, over uneven
+    clusters, an empty one, and K, V rows that start 4 bytes off a 16-byte boundary."""
     print(f"[case] cluster sums layouts HKV={HKV_} T={T} C={C}", flush=True)
     rng = np.random.default_rng(HKV_ + T)
     R = HKV_ * 4
