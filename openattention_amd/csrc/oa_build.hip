@@ -923,6 +923,8 @@ __global__ void __launch_bounds__(kSortThreads) csr_sort_kernel(int T, const uin
 // took 2215 us, and take 2086 us (by the counters 15 GB of the 17 GB gathered miss the L2s: waves of
 // clusters of different sizes drift apart in position); one such sequence (W = 4) 206 us, and takes 78
 // us.
+typedef uint32_t uint32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float floatx4a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int W>
 __global__ void __launch_bounds__(64 * W) cluster_sums_kernel(const uint16_t* K, const uint16_t* V, long ksh,
                                                               long kst, int G, int C, const int32_t* cstart,
@@ -966,20 +968,20 @@ __global__ void __launch_bounds__(64 * W) cluster_sums_kernel(const uint16_t* K,
   };
   if (cl > 0) next(grp);
   for (int m0 = grp; m0 < cl; m0 += U * kGroups) {
-    uint4 kw[U], vw[U];
+    uint32x4a4 kw[U], vw[U];                     // (K, V rows are 4-byte aligned)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const long off = (long)pos[u] * kst;
-      kw[u] = *reinterpret_cast<const uint4*>(kr + off);
-      vw[u] = *reinterpret_cast<const uint4*>(vr + off);
+      kw[u] = *reinterpret_cast<const uint32x4a4*>(kr + off);
+      vw[u] = *reinterpret_cast<const uint32x4a4*>(vr + off);
     }
     next(m0 + U * kGroups);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (m0 + u * kGroups < cl) {
         float k[8], v[8];
-        oa::unpack8(kw[u], k);
-        oa::unpack8(vw[u], v);
+        oa::unpack8(make_uint4(kw[u][0], kw[u][1], kw[u][2], kw[u][3]), k);
+        oa::unpack8(make_uint4(vw[u][0], vw[u][1], vw[u][2], vw[u][3]), v);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const double x = (double)k[e];
@@ -1019,11 +1021,11 @@ __global__ void __launch_bounds__(64 * W) cluster_sums_kernel(const uint16_t* K,
   // lane group 0 writes Sk, 1 Sk2, 2 Sv (every group holds all three)
   if (lane >= 48) return;
   float* out = (lane < 16 ? Sk : lane < 32 ? Sk2 : Sv) + ((long)row * C + c) * kD + d0;
-  float o[8];
+  floatx4a4 o[2];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = (float)(lane < 16 ? ks[e] : lane < 32 ? qs[e] : vs[e]);
-  *reinterpret_cast<float4*>(out) = make_float4(o[0], o[1], o[2], o[3]);
-  *reinterpret_cast<float4*>(out + 4) = make_float4(o[4], o[5], o[6], o[7]);
+  for (int e = 0; e < 8; ++e) o[e / 4][e % 4] = (float)(lane < 16 ? ks[e] : lane < 32 ? qs[e] : vs[e]);
+  reinterpret_cast<floatx4a4*>(out)[0] = o[0];
+  reinterpret_cast<floatx4a4*>(out)[1] = o[1];
 }
 
 }  // namespace

@@ -15,6 +15,10 @@ namespace {
 
 constexpr int kMaxQsh = 10;
 
+// (the statistics are aligned as floats, K and V as bf16)
+typedef float floatx2a4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t __attribute__((aligned(2))) uint32a2;
+
 struct StatsArgs {
   const uint16_t* K; const uint16_t* V; long kv_sb; long kv_ss;
   const int32_t* asg; long asg_stride;
@@ -37,9 +41,9 @@ __global__ void __launch_bounds__(256) rows_stats_kernel(StatsArgs a) {
   const uint16_t* vb = a.V + (long)kv * a.kv_sb + 2 * lane;
   const int32_t* ar = a.asg + (long)r * a.asg_stride;
   const long sb = ((long)r * a.C + c) * OA_D + 2 * lane;
-  float2 sk = *reinterpret_cast<const float2*>(a.Sk + sb);
-  float2 s2 = *reinterpret_cast<const float2*>(a.Sk2 + sb);
-  float2 sv = *reinterpret_cast<const float2*>(a.Sv + sb);
+  floatx2a4 sk = *reinterpret_cast<const floatx2a4*>(a.Sk + sb);
+  floatx2a4 s2 = *reinterpret_cast<const floatx2a4*>(a.Sk2 + sb);
+  floatx2a4 sv = *reinterpret_cast<const floatx2a4*>(a.Sv + sb);
   float nb = a.nb[(long)r * a.C + c];
   const int top = nq - 1 + a.later;                 // keys above the first row's
   // 64 cluster ids at a time, lane l holding that of key n0 + base + l
@@ -50,17 +54,17 @@ __global__ void __launch_bounds__(256) rows_stats_kernel(StatsArgs a) {
       if (i < nq) {
         const long v = (((((long)kv << a.qsh) + i) << 2) | (r & 3)) * a.C + c;
         const long o = v * OA_D + 2 * lane;
-        *reinterpret_cast<float2*>(a.rSk + o) = sk;
-        *reinterpret_cast<float2*>(a.rSk2 + o) = s2;
-        *reinterpret_cast<float2*>(a.rSv + o) = sv;
+        *reinterpret_cast<floatx2a4*>(a.rSk + o) = sk;
+        *reinterpret_cast<floatx2a4*>(a.rSk2 + o) = s2;
+        *reinterpret_cast<floatx2a4*>(a.rSv + o) = sv;
         if (lane == 0) a.rnb[v] = nb;
       }
       // the key before leaves on the way to row i - 1 (at j = 0 it is the next 64's last)
       if (i == 0) break;
       const int id = j > 0 ? __builtin_amdgcn_readlane(mine, j - 1) : ar[n0 + i - 1];
       if (id == c) {
-        const uint32_t kw = *reinterpret_cast<const uint32_t*>(kb + (long)(n0 + i - 1) * a.kv_ss);
-        const uint32_t vw = *reinterpret_cast<const uint32_t*>(vb + (long)(n0 + i - 1) * a.kv_ss);
+        const uint32_t kw = *reinterpret_cast<const uint32a2*>(kb + (long)(n0 + i - 1) * a.kv_ss);
+        const uint32_t vw = *reinterpret_cast<const uint32a2*>(vb + (long)(n0 + i - 1) * a.kv_ss);
         const float k0 = __uint_as_float(kw << 16), k1 = __uint_as_float(kw & 0xffff0000u);
         sk.x = sk.x - k0; sk.y = sk.y - k1;
         s2.x = s2.x - k0 * k0; s2.y = s2.y - k1 * k1;

@@ -425,6 +425,28 @@ def test_question_rows_leave_the_first_rows_results(B, Q):
         assert torch.equal(a, b)
 
 
+def test_question_rows_over_statistics_off_8_bytes():
+    """Index statistics that start 4 bytes off an 8-byte boundary: the same question rows."""
+    from openattention_amd.method import OursHIP
+    N, Q = 800, 9
+    K, V, _, qq, _ = synth.make_layer(17, 1, N, N, 64, DEV, n_question=Q)
+    static = synth.static_metric(1)
+    m = OursHIP(types.SimpleNamespace(rho=0.03), 1, N, DEV, n_layers=1, static=static)
+    st = m.st[0]
+    build_rows(st, K, V, qq, N, static["M"][0], static["inv_freq"], 1.0, 0)
+    got = []
+    for off in (False, True):
+        if off:
+            for f in ("nb", "Sk", "Sk2", "Sv"):
+                t = getattr(st, f)
+                setattr(st, f, torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape))
+            assert st.Sk.data_ptr() % 8 == 4
+        n_dev = torch.zeros(1, device=DEV, dtype=torch.int32)
+        out = torch.empty(1, HQ, Q, D, device=DEV, dtype=torch.bfloat16)
+        got.append(m.rows_step(st, K.view(-1, N, D), V.view(-1, N, D), qq, n_dev, N, out).clone())
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("B,N,Q,walk", [(1, 1200, 203, 1024), (1, 1200, 203, 64), (2, 900, 130, 96)])
 def test_question_rows_past_64_keys(B, N, Q, walk, monkeypatch):
     """More question rows than the 64 cluster ids that a wave takes back at a time, with every group's

@@ -242,3 +242,19 @@ def test_cluster_sums_do_not_depend_on_the_batch(T, C):
                     want = math.fsum(x[m, j])
                     bound = m.sum() * 2.0 ** -53 * np.abs(x[m, j]).sum() + 2.0 ** -24 * abs(want)
                     assert abs(float(got[r, c, j]) - want) <= bound, (r, c, j)
+
+
+@pytest.mark.parametrize("T,C", [(300, 8), (4097, 16)])
+def test_cluster_sums_into_rows_off_16_bytes(T, C):
+    """Statistics rows that start 4 bytes off a 16-byte boundary, with one and four waves per cluster: the
+    bits of aligned ones."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    K, V = (torch.randn(2, T, 128, device=DEV, generator=g).to(torch.bfloat16) for _ in range(2))
+    R = 8
+    asg8 = torch.zeros(R, -(-T // 64) * 64, device=DEV, dtype=torch.uint8)
+    asg8[:, :T] = torch.randint(0, C, (R, T), device=DEV, generator=g)
+    nb, S = _cluster_build(K, V, T, asg8, C)
+    off = [torch.full((R * C * 128 + 2,), 7.0, device=DEV) for _ in range(3)]
+    ops.cluster_build(K, V, T, 4, asg8, C, torch.empty_like(nb), *(t[1:-1].view(R, C, 128) for t in off), *_lists(R, T, C))
+    for t, want in zip(off, S):
+        assert torch.equal(t[1:-1].view(R, C, 128), want) and t[0] == 7.0 and t[-1] == 7.0
