@@ -104,6 +104,10 @@ def load() -> ct.CDLL:
     if have != ABI_VERSION:
         raise RuntimeError(f"kernel library {path} has ABI {have}, this binding expects {ABI_VERSION}: "
                            "rebuild it (__graft_entry__.build())")
+    missing = [name for name in SIGNATURES if not hasattr(lib, name)]
+    if missing:
+        raise RuntimeError(f"kernel library {path} lacks {', '.join(missing)}: it was built from older sources, "
+                           "rebuild it (__graft_entry__.build())")
     for name, argtypes in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.argtypes = argtypes

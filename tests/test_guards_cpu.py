@@ -1,4 +1,5 @@
 """What the decode path refuses on the host, before any kernel is launched."""
+import subprocess
 import types
 
 import pytest
@@ -182,3 +183,18 @@ def test_tracers_and_modes_are_noticed():
         torch.set_autocast_enabled("cuda", was)
         torch.set_autocast_dtype("cuda", dt)
     assert len(seen) == 8 and all(seen[2:])
+
+
+@pytest.mark.parametrize("abi,want", [(None, "lacks oa_"), (8, "has ABI 8")])
+def test_an_older_library_is_refused_with_a_rebuild_message(abi, want, tmp_path, monkeypatch):
+    """A kernel library of another ABI version, or of this one without the newer entry points, is refused
+    with the message that names it and says to rebuild."""
+    from openattention_amd import _build, lib
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text(f"int oa_abi_version(void) {{ return {lib.ABI_VERSION if abi is None else abi}; }}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setattr(_build, "lib_path", lambda: str(so))
+    monkeypatch.setattr(lib, "_LIB", None)
+    with pytest.raises(RuntimeError, match=want) as e:
+        lib.load()
+    assert "rebuild it" in str(e.value) and str(so) in str(e.value)
