@@ -453,8 +453,10 @@ def step(K, V, st, n_dev, q, w, sel, out, ns: int, nl: int, k_top: int, sm_scale
     _need(V.shape == K.shape and V.stride() == K.stride() and V.dtype == K.dtype, "V must match K")
     _need(R == GROUP * BH, "nb must have one row per query-head row")
     _chk(st.codes, "codes", torch.int8, (BH, None, RANK_Q), contiguous=True)
-    _chk(st.asg, "asg", torch.int32, (R, -Lk))
-    _chk(st.asg8, "asg8", torch.uint8, (R, -max(Lk, Lmax)))
+    # (the update writes ids, and question rows read them, at positions of K; a row without either reads
+    # those of its own keys, which an index shorter than the cache may hold)
+    _chk(st.asg, "asg", torch.int32, (R, -Lk if update or qshift or later else None))
+    _chk(st.asg8, "asg8", torch.uint8, (R, -(max(Lk, Lmax) if update else Lmax)))
     _chk(st.nb, "nb", torch.float32, (R, C), contiguous=True)
     _stats(R, C, (st.Sk, "Sk"), (st.Sk2, "Sk2"), (st.Sv, "Sv"))
     if update:
@@ -630,7 +632,7 @@ def prefill_attn_ok(q, k, v, sm_scale: float = 1.0) -> bool:
     the operation (autograd in either mode, a functional transform, what _watched names)."""
     if (sm_scale is None or not sm_scale >= 0 or _watched() or q.dim() != 4 or k.dim() != 4 or q.shape[0] != 1 or k.shape[0] != 1 or k.shape != v.shape
             or q.shape[3] != HEAD_DIM or k.shape[3] != HEAD_DIM or q.shape[1] != GROUP * k.shape[1]
-            or q.shape[2] != k.shape[2] or q.shape[2] < 1):
+            or q.shape[2] != k.shape[2] or not 1 <= q.shape[2] <= 1 << 24):
         return False
     for t in (q, k, v):
         if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != torch.bfloat16

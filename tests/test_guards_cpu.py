@@ -70,6 +70,32 @@ def test_step_refuses_tensors_on_another_device(rows):
                 call(stats={**stats, f: torch.empty(stats[f].shape, device="cpu")})
 
 
+def test_step_over_a_cache_longer_than_its_index():
+    """One row without an index update over K, V rows longer than the index's capacity passes the checks;
+    an update, or question rows, which reach the keys' positions, are refused."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    calls = []
+    with FakeTensorMode(), pytest.MonkeyPatch.context() as mp:
+        mp.setattr(ops, "_stream", lambda dev: 0)
+        mp.setattr(ops.lib, "call", lambda name, *a: calls.append(name))
+        m = OursHIP(types.SimpleNamespace(rho=0.01), 1, 256, "cuda", n_layers=1)
+        st = m.st[0]
+        K = torch.empty(8, 320, 128, device="cuda", dtype=torch.bfloat16)
+        q = torch.empty(32, 128, device="cuda", dtype=torch.bfloat16)
+        sel = torch.empty(32, 4, device="cuda", dtype=torch.int32)
+        n_dev = torch.empty(1, device="cuda", dtype=torch.int32)
+        stats = (st.nb, st.Sk, st.Sk2, st.Sv)
+
+        def call(**kw):
+            ops.step(K, K, st, n_dev, q, m, sel, m.out, 1, 1, 2, 0.1, m.E, RMAX, **kw)
+
+        call(update=False)
+        assert calls == ["oa_step"]
+        for kw in (dict(update=True), dict(update=False, later=1, stats=stats)):
+            with pytest.raises(ValueError, match="asg"):
+                call(**kw)
+
+
 def test_question_rows_are_grouped_where_a_group_holds_two():
     """Rows per launch of a multi-row call: the largest power of two that 1024 query-head rows and the
     call hold; a batch that leaves one row to a launch runs its rows one after the other in place."""
