@@ -919,10 +919,10 @@ __global__ void __launch_bounds__(kSortThreads) csr_sort_kernel(int T, const uin
 // what rounding leaves, so that W follows from the row alone, not from the batch: the same row gives the
 // same bits in every call.
 // Bound by vector issue: 14 fp64 and conversion instructions per member and lane of 8 dims.  With a
-// lane on 2 dims (4-byte loads, a row address per member for every lane) 32 sequences of 32767 tokens
-// took 2215 us, and take 2086 us (by the counters 15 GB of the 17 GB gathered miss the L2s: waves of
-// clusters of different sizes drift apart in position); one such sequence (W = 4) 206 us, and takes 78
-// us.
+// lane on 2 dims (4-byte loads, a row address per member for every lane) and one wave 32 sequences of
+// 32767 tokens in 64 clusters took 2215 us, with 8 dims 2086 (by the counters 15 GB of the 17 GB gathered
+// miss the L2s: waves of clusters of different sizes drift apart in position), with four waves 1782; one
+// such sequence 206 us, and with four waves 78.
 typedef uint32_t uint32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float floatx4a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int W>

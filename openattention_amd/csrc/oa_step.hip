@@ -27,8 +27,8 @@ struct StatsArgs {
   const int* n_dev; int C; int qsh; int later;
 };
 
-// One wave per (query-head row of the index, cluster): the cluster's statistics walk back from all
-// keys to the group's first row, lane l holding dims 2 l, 2 l + 1, and are written out at every row of
+// One wave per (query-head row of the index, cluster): the cluster's statistics walk back from those
+// given (of all keys, or of an earlier group's first row) to the group's first row, lane l holding dims 2 l, 2 l + 1, and are written out at every row of
 // the group.  Bound by the writes (1540 bytes per row and cluster).
 __global__ void __launch_bounds__(256) rows_stats_kernel(StatsArgs a) {
   const int r = blockIdx.y;

@@ -12,8 +12,8 @@ multibin.py:1894):
        oa_query_metric, the eigenpairs by oa_sym_eig_top (one-sided Jacobi).
   a11  codes: oa_qgs_codes (zc = k U, scale = max(max_t |zc| / 127, 1e-12), codes =
        clamp(rint(zc / scale), -127, 127); static_top_k.py:174-181).
-  a12  oa_qgc_project (zP = bf16(k W) - colmean on the bf16 matrix cores), then 4 Lloyd
-       iterations of oa_kmeans_step (bf16 distance bf16(bf16(zP . c) - bf16(|c|^2 / 2)), ties to
+  a12  oa_qgc_project_max (zP = bf16(k W) - colmean on the bf16 matrix cores), then 4 Lloyd
+       iterations of oa_kmeans_step_max (bf16 distance bf16(bf16(zP . c) - bf16(|c|^2 / 2)), ties to
        the lower cluster; then the member means, an empty cluster keeping its initial point)
        (methods_eager.py:526-547).
   a13  oa_cluster_build: n_b, sum k, sum k^2, sum v per cluster and the CSR member lists
