@@ -49,7 +49,7 @@ def _dev(*ts: torch.Tensor) -> torch.device:
 
 
 def _on(dev: torch.device, *ts: torch.Tensor) -> None:
-    """_dev's checks of further tensors against the device it returned (by index: a step checks 17 of
+    """_dev's checks of further tensors against the device it returned (by index: a step checks 30 of
     them, on the host path of every eager call)."""
     i = dev.index
     for t in ts:
@@ -439,8 +439,9 @@ def step(K, V, st, n_dev, q, w, sel, out, ns: int, nl: int, k_top: int, sm_scale
     fexp, H, TM, TMn, S, score, n_t, quota, qsk, exp_idx); the same outputs.  qshift > 0 or later > 0
     (update False): 2^qshift question rows per sequence, rows laid out ((kv << qshift) + i) * 4 + head
     in q, sel, out and w; stats = (nb, Sk, Sk2, Sv) receives their statistics."""
-    dev = _dev(K, V, n_dev, q, w.limbs, w.fexp, w.H, w.TM, w.S, w.score, w.n_t, w.quota, w.exp_idx, sel, out)
-    _on(dev, w.qsk, w.TMn, st.codes, st.asg, st.asg8, st.nb, st.Sk, st.Sk2, st.Sv, st.U, st.scale)
+    dev = _dev(K)
+    _on(dev, V, n_dev, q, w.limbs, w.fexp, w.H, w.TM, w.TMn, w.S, w.score, w.n_t, w.quota, w.qsk, w.exp_idx, sel, out,
+        st.codes, st.asg, st.asg8, st.nb, st.Sk, st.Sk2, st.Sv, st.U, st.scale)
     if update:
         _on(dev, st.W, st.colmean, st.cent, st.reclist, st.reccnt)
     if stats is not None:
